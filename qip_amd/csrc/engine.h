@@ -56,26 +56,23 @@ constexpr int kProductHighPerPass = 8;
 constexpr int kRingSlots = 8;
 constexpr size_t kRingSlotBytes = 64 * 64 * 16 + 4096;  // a 64x64 complex128 matrix + offsets
 
-// A diagonal gate on at most two targets, held back on the state (qipgpu_state::chain) so that a run
-// of them is applied by one kernel: the factor d[j] multiplies the amplitudes whose ctrl_mask bits are
-// all 1, j being the value of state bits tpos[0] (MSB) .. tpos[k-1].
-constexpr int kDiagChainMax = 16;
-struct ChainGate {
+// A small gate held back on the state (qipgpu_state::held) so that a run of them is applied in one pass
+// (runs.hip), where the bits of ctrl_mask are all 1: a 2x2 on state bit tpos[0], the exchange of bits
+// tpos[0] and tpos[1], or a diagonal on k <= 2 targets, its factor m[j] for j the value of state bits
+// tpos[0] (MSB) .. tpos[k-1].
+struct HeldGate {
+    enum Kind : uint8_t { kSingle, kSwap, kDiagonal };
     uint64_t ctrl_mask;
-    cx<double> d[4];
-    uint8_t k;
+    cx<double> m[4];
+    Kind kind;
+    uint8_t k;          // entries of tpos
     uint8_t tpos[2];
 };
-
-// A single-qubit gate (2x2 U on state bit tpos where the bits of ctrl_mask are 1), held back on the
-// state (qipgpu_state::run) so that a run of them whose bits share one 4096-amplitude tile is applied
-// in one pass, each gate in turn on the tile in LDS.
-constexpr int kTileRunMax = 32;
-struct RunGate {
-    uint64_t ctrl_mask;
-    cx<double> U[4];
-    uint8_t tpos;
-};
+// Gates held back at most: with this many, the next pass is applied. Enough for a pass to see the
+// two-qubit gates that follow a layer of single-qubit gates on 30 qubits.
+constexpr size_t kHeldMax = 64;
+// Diagonals of one sweep over the amplitudes that share the controls all of them have (k_diag_chain).
+constexpr int kDiagChainMax = 16;
 
 }  // namespace qipgpu
 
@@ -128,13 +125,8 @@ struct qipgpu_state {
     hipGraphNode_t rec_last = nullptr;
     // gates recorded for online fusion and not launched yet (complex64 states)
     qipgpu::Recorder *recorder = nullptr;
-    // gates held back (flush_held applies them before anything else touches the state): a run of
-    // diagonal gates or a run of single-qubit gates, never both at once
-    qipgpu::ChainGate chain[qipgpu::kDiagChainMax];
-    int32_t chain_len = 0;
-    qipgpu::RunGate run[qipgpu::kTileRunMax];
-    int32_t run_len = 0;
-    uint64_t run_bits = 0;     // target and control bits of the held single-qubit gates
+    // gates held back, in program order (flush_held applies them before anything else touches the state)
+    std::vector<qipgpu::HeldGate> held;
 };
 
 namespace qipgpu {
@@ -187,9 +179,15 @@ int device_cus();
 int check_qubits(const qipgpu_state *s, int32_t k, const int32_t *q, const char *what);
 // Reserve a staging ring slot, copy `bytes` from `src` to the device, return device pointer.
 int ring_upload(qipgpu_state *s, const void *src, size_t bytes, void **dev);
-// Apply the gates held back on the state, in order (engine.hip): every entry point that touches the
-// state does so first, through flush_recorded.
+// Hold a small gate back on the state; with kHeldMax held, the next pass of them is applied (runs.hip).
+int hold_gate(qipgpu_state *s, const HeldGate &g);
+// Apply the gates held back on the state (runs.hip): every entry point that touches the state does so
+// first, through flush_recorded.
 int flush_held(qipgpu_state *s);
+// One held gate by a sweep of its own; up to kDiagChainMax diagonals, in order, by one sweep over the
+// amplitudes that share the controls all of them have (engine.hip).
+int launch_held_gate(qipgpu_state *s, const HeldGate &g);
+int launch_diag_chain(qipgpu_state *s, const HeldGate *g, int count);
 // Apply the held-back gates, then launch every recorded gate (recorder.hip); the recorded gates are
 // left alone while the recorder itself is launching.
 int flush_recorded(qipgpu_state *s);

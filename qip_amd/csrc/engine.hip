@@ -481,9 +481,7 @@ int qipgpu_capture_end(qipgpu_state *s, qipgpu_graph **out) {
     if (!s->capturing) return set_error(QIPGPU_EINVAL, "the state is not capturing");
     // gates still held back belong to the recording: their node goes last
     if (!s->capture_refused && flush_held(s) != QIPGPU_OK) s->capture_refused = true;
-    s->chain_len = 0;
-    s->run_len = 0;
-    s->run_bits = 0;
+    s->held.clear();
     s->capturing = false;
     hipGraph_t g = s->rec_graph;
     s->rec_graph = nullptr;
@@ -564,11 +562,9 @@ int qipgpu_get_stream(qipgpu_state *s, void **stream) {
 int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_len,
                         const int32_t *group_idx, const double *feeds) {
     QIP_NOT_CAPTURING(s, "a state initialisation");
-    // every amplitude is rewritten, so recorded gates, held-back diagonals and the factor are moot
+    // every amplitude is rewritten, so recorded and held-back gates and the factor are moot
     s->fused_prev_count = 0;
-    s->chain_len = 0;
-    s->run_len = 0;
-    s->run_bits = 0;
+    s->held.clear();
     recorder_discard(s);
     if (n_groups < 0) return set_error(QIPGPU_EINVAL, "negative group count");
     uint64_t fed = 0;
@@ -934,7 +930,7 @@ static int launch_diag(qipgpu_state *s, const std::vector<int> &tbits, uint64_t 
     return launch_gate(s, &k_diag<R, K, ITEMS>, dim3(capped_grid(nb)), dim3(256), a);
 }
 
-// A run of held-back diagonal gates in one sweep over the amplitudes whose bits common_mask (the
+// A run of diagonal gates in one sweep over the amplitudes whose bits common_mask (the
 // controls every gate of the run has) are 1. Each amplitude meets the gates in order and is rounded
 // after each one, with k_diag's arithmetic, so the result is bit for bit that of launching the gates
 // one by one.
@@ -945,7 +941,7 @@ struct DiagChainArgs {
     uint64_t common_mask;
     PosList pl;          // common control positions
     int32_t ngates;
-    ChainGate g[kDiagChainMax];
+    HeldGate g[kDiagChainMax];
     BlockOrder order;
     uint32_t nblocks;
 };
@@ -971,7 +967,7 @@ __global__ __launch_bounds__(256) void k_diag_chain(const DiagChainArgs<R> a) {
                 if ((idx[it] & a.g[q].ctrl_mask) != a.g[q].ctrl_mask) continue;
                 uint32_t j = 0;
                 for (int b = 0; b < a.g[q].k; ++b) j = (j << 1) | (uint32_t)((idx[it] >> a.g[q].tpos[b]) & 1ull);
-                x = narrow<R>(cmul(widen(x), a.g[q].d[j]));
+                x = narrow<R>(cmul(widen(x), a.g[q].m[j]));
                 touched = true;
             }
             if (touched) a.amps[idx[it]] = x;
@@ -980,53 +976,42 @@ __global__ __launch_bounds__(256) void k_diag_chain(const DiagChainArgs<R> a) {
     }
 }
 
-// Amplitude-sized cost of one launch (about 4 us of HBM time) when choosing between one sweep for a
-// run of diagonal gates and a launch per gate.
-constexpr uint64_t kLaunchCostAmps = 1ull << 19;
-
 template <typename R>
-static int launch_chain_gate(qipgpu_state *s, const ChainGate &c) {
-    std::vector<int> tbits, cpos;
-    for (int b = 0; b < c.k; ++b) tbits.push_back(c.tpos[b]);
-    for (int p = 0; p < 64; ++p)
-        if (c.ctrl_mask >> p & 1) cpos.push_back(p);
-    std::vector<cd> d((size_t)1 << c.k);
-    for (size_t j = 0; j < d.size(); ++j) d[j] = cd(c.d[j].re, c.d[j].im);
-    switch (c.k) {
-        case 0: return launch_diag<R, 0>(s, tbits, c.ctrl_mask, cpos, d);
-        case 1: return launch_diag<R, 1>(s, tbits, c.ctrl_mask, cpos, d);
-        default: return launch_diag<R, 2>(s, tbits, c.ctrl_mask, cpos, d);
+static int launch_one(qipgpu_state *s, const HeldGate &g) {
+    std::vector<int> tbits(g.tpos, g.tpos + g.k), cpos;
+    for (int p = 0; p < s->n; ++p)
+        if (g.ctrl_mask >> p & 1) cpos.push_back(p);
+    std::vector<int> allpos(cpos);
+    allpos.insert(allpos.end(), tbits.begin(), tbits.end());
+    std::vector<cd> m(4);
+    for (int i = 0; i < 4; ++i) m[i] = cd(g.m[i].re, g.m[i].im);
+    if (g.kind == HeldGate::kSingle) return launch_dense_reg<R, 1>(s, tbits, g.ctrl_mask, allpos, m);
+    if (g.kind == HeldGate::kSwap) {
+        std::vector<cd> swap(16, cd(0.0, 0.0));
+        swap[0] = swap[6] = swap[9] = swap[15] = 1.0;
+        return launch_dense_reg<R, 2>(s, tbits, g.ctrl_mask, allpos, swap);
+    }
+    switch (g.k) {
+        case 0: return launch_diag<R, 0>(s, tbits, g.ctrl_mask, cpos, m);
+        case 1: return launch_diag<R, 1>(s, tbits, g.ctrl_mask, cpos, m);
+        default: return launch_diag<R, 2>(s, tbits, g.ctrl_mask, cpos, m);
     }
 }
 
 template <typename R>
-static int flush_chain_typed(qipgpu_state *s) {
-    const int m = s->chain_len;
-    s->chain_len = 0;
-    uint64_t common = ~0ull, separate = 0;
-    for (int q = 0; q < m; ++q) {
-        common &= s->chain[q].ctrl_mask;
-        separate += (s->len >> __builtin_popcountll(s->chain[q].ctrl_mask)) + kLaunchCostAmps;
-    }
-    const uint64_t swept = (s->len >> __builtin_popcountll(common)) + kLaunchCostAmps;
-    if (m == 1 || swept > separate) {   // one gate, or gates on small disjoint subspaces of a large state
-        for (int q = 0; q < m; ++q) {
-            const int rc = launch_chain_gate<R>(s, s->chain[q]);
-            if (rc) return rc;
-        }
-        return QIPGPU_OK;
-    }
+static int launch_chain(qipgpu_state *s, const HeldGate *g, int count) {
     DiagChainArgs<R> a;
     std::memset(&a, 0, sizeof(a));
     a.amps = (cx<R> *)s->amps;
-    a.common_mask = common;
+    a.common_mask = ~0ull;
+    for (int q = 0; q < count; ++q) a.common_mask &= g[q].ctrl_mask;
     std::vector<int> cpos;
     for (int p = 0; p < s->n; ++p)
-        if (common >> p & 1) cpos.push_back(p);
+        if (a.common_mask >> p & 1) cpos.push_back(p);
     a.count = s->len >> cpos.size();
     fill_poslist(a.pl, cpos);
-    a.ngates = m;
-    for (int q = 0; q < m; ++q) a.g[q] = s->chain[q];
+    a.ngates = count;
+    for (int q = 0; q < count; ++q) a.g[q] = g[q];
     constexpr int ITEMS = 4;
     const uint32_t nb = blocks_for(a.count, 256 * ITEMS);
     a.order = block_order(s->len * s->amp_bytes, s->amp_bytes, nb);
@@ -1034,274 +1019,26 @@ static int flush_chain_typed(qipgpu_state *s) {
     return launch_gate(s, &k_diag_chain<R, ITEMS>, dim3(capped_grid(nb)), dim3(256), a);
 }
 
-// A run of held-back single-qubit gates whose target and control bits all lie in one tile of 4096
-// amplitudes (tile bits P: those bits, state bits 0..3 and free bits, ascending; u bit i <-> state
-// bit P[i]). A workgroup loads a tile into LDS and applies the gates to it one after the other, each
-// to every pair of the tile with k_dense's arithmetic (FP64 from zero, rounded to the state's
-// precision), then stores the tile: the bits of a launch per gate, for one HBM pass.
-struct RunSlot {
-    cx<double> U[4];
-    uint32_t cmask;     // control bits, in tile (u) coordinates
-    uint32_t tb;        // target bit, in tile coordinates
-};
-
-template <typename R>
-struct TileRunArgs {
-    cx<R> *amps;
-    uint64_t ntiles;
-    int32_t ngates;
-    uint8_t pbits[12];
-    RunSlot g[kTileRunMax];
-};
-
-template <typename R>
-__device__ __forceinline__ uint64_t run_tile_base(uint64_t t, const TileRunArgs<R> &a) {
-#pragma unroll
-    for (int i = 0; i < 12; ++i) {
-        const uint32_t p = a.pbits[i];
-        const uint64_t lo = t & ((1ull << p) - 1ull);
-        t = ((t ^ lo) << 1) | lo;
-    }
-    return t;
-}
-
-// 512 threads per workgroup (two waves per SIMD from each workgroup, so one wave's LDS and FP64
-// latency overlaps another's). Thread t holds the tile's amplitudes u = t + 512 i, i = 0..7: u bits
-// 0..8 are t, bits 9..11 are i.
-constexpr uint32_t kRunThreads = 512;
-
-template <typename R>
-__device__ __forceinline__ uint64_t run_off_hi(int i, const TileRunArgs<R> &a) {
-    uint64_t o = 0;
-#pragma unroll
-    for (int b = 0; b < 3; ++b) o |= (uint64_t)((i >> b) & 1) << a.pbits[9 + b];
-    return o;
-}
-
-// One gate on one pair (x0: target bit 0, x1: target bit 1), as k_dense<R,1> computes it: each output
-// an FP64 sum from zero of U's row times the pair (cfma), rounded to the state's precision.
-template <typename R>
-__device__ __forceinline__ void run_gate(const RunSlot &g, cx<R> &x0, cx<R> &x1) {
-    cx<double> acc0, acc1;
-    acc0.re = acc0.im = acc1.re = acc1.im = 0.0;
-    cfma(acc0, g.U[0], widen(x0));
-    cfma(acc0, g.U[1], widen(x1));
-    cfma(acc1, g.U[2], widen(x0));
-    cfma(acc1, g.U[3], widen(x1));
-    x0 = narrow<R>(acc0);
-    x1 = narrow<R>(acc1);
-}
-
-// A thread's 8 amplitudes of a tile in registers, as separate real and imaginary parts (plain scalar
-// arrays stay in registers where arrays of the complex struct would go to scratch memory).
-template <typename R>
-struct RunRegs {
-    R re[8], im[8];
-};
-
-template <typename R>
-__device__ __forceinline__ void run_load(RunRegs<R> &v, uint64_t base, const TileRunArgs<R> &a) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const cx<R> x = a.amps[base + run_off_hi(i, a)];
-        v.re[i] = x.re;
-        v.im[i] = x.im;
-    }
-}
-
-template <typename R>
-__device__ __forceinline__ void run_tile(const RunRegs<R> &v, uint64_t base, cx<R> *t, const TileRunArgs<R> &a) {
-    const uint32_t tid = threadIdx.x;
-    __syncthreads();  // the previous tile has left LDS
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        cx<R> x;
-        x.re = v.re[i];
-        x.im = v.im[i];
-        t[tid + kRunThreads * i] = x;
-    }
-    __syncthreads();
-    int gi = 0;
-    // two gates per LDS round trip: each thread owns whole quads {u, u^b1, u^b2, u^b1^b2} (or pairs,
-    // when both gates act on one bit) and applies the first gate to them, then the second
-    for (; gi + 1 < a.ngates; gi += 2) {
-        const RunSlot &g1 = a.g[gi], &g2 = a.g[gi + 1];
-        const uint32_t b1 = 1u << g1.tb, b2 = 1u << g2.tb;
-        if (b1 == b2) {
-            const uint32_t lo = b1 - 1u;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t p = tid + kRunThreads * j;    // pair index 0..2047
-                const uint32_t u0 = ((p & ~lo) << 1) | (p & lo);
-                cx<R> x0 = t[u0], x1 = t[u0 | b1];
-                if ((u0 & g1.cmask) == g1.cmask) run_gate(g1, x0, x1);
-                if ((u0 & g2.cmask) == g2.cmask) run_gate(g2, x0, x1);
-                t[u0] = x0;
-                t[u0 | b1] = x1;
-            }
-        } else {
-            const uint32_t bl = b1 < b2 ? b1 : b2, bh = b1 < b2 ? b2 : b1;
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                uint32_t q = tid + kRunThreads * j;          // quad index 0..1023
-                q = ((q & ~(bl - 1u)) << 1) | (q & (bl - 1u));
-                const uint32_t u = ((q & ~(bh - 1u)) << 1) | (q & (bh - 1u));
-                cx<R> a00 = t[u], a10 = t[u | b1], a01 = t[u | b2], a11 = t[u | b1 | b2];
-                if ((u & g1.cmask) == g1.cmask) run_gate(g1, a00, a10);
-                if (((u | b2) & g1.cmask) == g1.cmask) run_gate(g1, a01, a11);
-                if ((u & g2.cmask) == g2.cmask) run_gate(g2, a00, a01);
-                if (((u | b1) & g2.cmask) == g2.cmask) run_gate(g2, a10, a11);
-                t[u] = a00;
-                t[u | b1] = a10;
-                t[u | b2] = a01;
-                t[u | b1 | b2] = a11;
-            }
-        }
-        __syncthreads();
-    }
-    if (gi < a.ngates) {
-        const RunSlot &g = a.g[gi];
-        const uint32_t b = 1u << g.tb, lo = b - 1u;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t p = tid + kRunThreads * j;
-            const uint32_t u0 = ((p & ~lo) << 1) | (p & lo);
-            if ((u0 & g.cmask) != g.cmask) continue;
-            cx<R> x0 = t[u0], x1 = t[u0 | b];
-            run_gate(g, x0, x1);
-            t[u0] = x0;
-            t[u0 | b] = x1;
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a.amps[base + run_off_hi(i, a)] = t[tid + kRunThreads * i];
-}
-
-// Contiguous tile ranges per workgroup, two (complex128) or four (complex64) workgroups per CU by LDS.
-template <typename R>
-__global__ __launch_bounds__(kRunThreads, 2) void k_tile_run(const TileRunArgs<R> a) {
-    __shared__ cx<R> t[4096];
-    const uint32_t tid = threadIdx.x;
-    uint64_t off_lo = 0;
-#pragma unroll
-    for (int b = 0; b < 9; ++b) off_lo |= (uint64_t)((tid >> b) & 1u) << a.pbits[b];
-    const uint64_t per = (a.ntiles + gridDim.x - 1) / gridDim.x;
-    uint64_t tile = (uint64_t)blockIdx.x * per;
-    const uint64_t end = min(tile + per, a.ntiles);
-    if (tile >= end) return;   // the same for every thread of the workgroup
-    const uint64_t last = end - 1;
-    // two register buffers alternate: the next tile's loads are in flight while one is processed
-    // (the last prefetch re-reads an in-range tile)
-    RunRegs<R> va, vb;
-    run_load(va, run_tile_base(tile, a) + off_lo, a);
-    for (;;) {
-        run_load(vb, run_tile_base(min(tile + 1, last), a) + off_lo, a);
-        run_tile(va, run_tile_base(tile, a) + off_lo, t, a);
-        if (++tile >= end) break;
-        run_load(va, run_tile_base(min(tile + 1, last), a) + off_lo, a);
-        run_tile(vb, run_tile_base(tile, a) + off_lo, t, a);
-        if (++tile >= end) break;
-    }
-}
-
-template <typename R>
-static int launch_run_gate(qipgpu_state *s, const RunGate &g) {
-    std::vector<int> tbits(1, g.tpos), allpos;
-    for (int p = 0; p < 64; ++p)
-        if (g.ctrl_mask >> p & 1) allpos.push_back(p);
-    allpos.push_back(g.tpos);
-    std::vector<cd> U(4);
-    for (int i = 0; i < 4; ++i) U[i] = cd(g.U[i].re, g.U[i].im);
-    return launch_dense_reg<R, 1>(s, tbits, g.ctrl_mask, allpos, U);
-}
-
-template <typename R>
-static int flush_run_typed(qipgpu_state *s) {
-    const int m = s->run_len;
-    const uint64_t bits = s->run_bits;
-    s->run_len = 0;
-    s->run_bits = 0;
-    uint64_t separate = 0;
-    for (int q = 0; q < m; ++q) separate += (s->len >> __builtin_popcountll(s->run[q].ctrl_mask)) + kLaunchCostAmps;
-    if (m == 1 || s->len + kLaunchCostAmps > separate) {   // one gate, or gates on small subspaces
-        for (int q = 0; q < m; ++q) {
-            const int rc = launch_run_gate<R>(s, s->run[q]);
-            if (rc) return rc;
-        }
-        return QIPGPU_OK;
-    }
-    // tile bits: the gates' bits, state bits 0..3, then free bits in the order 4, 5, 12..17, 6..11, 18..
-    uint64_t pmask = bits | 0xfull;
-    int order[64], no = 0;
-    for (int b = 4; b < 6; ++b) order[no++] = b;
-    for (int b = 12; b < 18; ++b) order[no++] = b;
-    for (int b = 6; b < 12; ++b) order[no++] = b;
-    for (int b = 18; b < 64; ++b) order[no++] = b;
-    for (int i = 0; i < no && __builtin_popcountll(pmask) < 12; ++i)
-        if (order[i] < s->n) pmask |= 1ull << order[i];
-    TileRunArgs<R> a;
-    std::memset(&a, 0, sizeof(a));
-    int ub[64];
-    for (int p = 0, i = 0; p < 64; ++p)
-        if (pmask >> p & 1) {
-            a.pbits[i] = (uint8_t)p;
-            ub[p] = i++;
-        }
-    a.amps = (cx<R> *)s->amps;
-    a.ntiles = s->len >> 12;
-    a.ngates = m;
-    for (int q = 0; q < m; ++q) {
-        const RunGate &g = s->run[q];
-        for (int i = 0; i < 4; ++i) a.g[q].U[i] = g.U[i];
-        a.g[q].tb = (uint32_t)ub[g.tpos];
-        uint32_t cm = 0;
-        for (int p = 0; p < 64; ++p)
-            if (g.ctrl_mask >> p & 1) cm |= 1u << ub[p];
-        a.g[q].cmask = cm;
-    }
-    const uint64_t per_cu = sizeof(R) == 8 ? 2 : 4;   // 64 KB / 32 KB of LDS per workgroup
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(a.ntiles, (uint64_t)device_cus() * per_cu);
-    return launch_gate(s, &k_tile_run<R>, dim3(grid), dim3(kRunThreads), a);
-}
-
-// Hold a single-qubit gate (target bit tpos, under ctrl_mask) back on the state: held diagonal gates
-// and a run it does not fit (more than 8 bits above bit 3, or full) are applied first.
-static int hold_single(qipgpu_state *s, int tpos, uint64_t ctrl_mask, const std::vector<cd> &U) {
-    const uint64_t gb = ctrl_mask | (1ull << tpos);
-    if (s->chain_len || s->run_len == kTileRunMax || __builtin_popcountll((s->run_bits | gb) & ~0xfull) > 8) {
-        const int rc = flush_held(s);
-        if (rc) return rc;
-    }
-    RunGate &g = s->run[s->run_len++];
+static void set_bits(HeldGate &g, HeldGate::Kind kind, const std::vector<int> &tbits, uint64_t ctrl_mask) {
     std::memset(&g, 0, sizeof(g));
+    g.kind = kind;
+    g.k = (uint8_t)tbits.size();
     g.ctrl_mask = ctrl_mask;
-    g.tpos = (uint8_t)tpos;
-    for (int i = 0; i < 4; ++i) {
-        g.U[i].re = U[i].real();
-        g.U[i].im = U[i].imag();
-    }
-    s->run_bits |= gb;
-    return QIPGPU_OK;
+    for (size_t b = 0; b < tbits.size(); ++b) g.tpos[b] = (uint8_t)tbits[b];
 }
 
-// Hold a diagonal gate (k <= 2 targets) back on the state; held single-qubit gates and a full run
-// are applied first.
-static int hold_diagonal(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<cd> &d) {
-    if (s->run_len || s->chain_len == kDiagChainMax) {
-        const int rc = flush_held(s);
-        if (rc) return rc;
+static void set_entries(HeldGate &g, const cd *m, size_t count) {
+    for (size_t i = 0; i < count; ++i) {
+        g.m[i].re = m[i].real();
+        g.m[i].im = m[i].imag();
     }
-    ChainGate &c = s->chain[s->chain_len++];
-    std::memset(&c, 0, sizeof(c));
-    c.ctrl_mask = ctrl_mask;
-    c.k = (uint8_t)tbits.size();
-    for (size_t b = 0; b < tbits.size(); ++b) c.tpos[b] = (uint8_t)tbits[b];
-    for (size_t j = 0; j < d.size(); ++j) {
-        c.d[j].re = d[j].real();
-        c.d[j].im = d[j].imag();
-    }
-    return QIPGPU_OK;
+}
+
+static bool is_swap(const std::vector<cd> &U) {
+    for (int r = 0; r < 4; ++r)
+        for (int c = 0; c < 4; ++c)
+            if (U[4 * r + c] != (c == (r >> 1 | (r & 1) << 1) ? 1.0 : 0.0)) return false;
+    return true;
 }
 
 template <typename R>
@@ -1328,13 +1065,15 @@ static int dispatch(qipgpu_state *s, const Analysed &an, const std::vector<int32
             identity = identity && d[j] == 1.0;
         }
         if (identity) return QIPGPU_OK;
-        if (k <= 2) return hold_diagonal(s, tbits, ctrl_mask, d);
+        if (k <= 2) {
+            HeldGate g;
+            set_bits(g, HeldGate::kDiagonal, tbits, ctrl_mask);
+            set_entries(g, d.data(), d.size());
+            return hold_gate(s, g);
+        }
         const int rc = flush_held(s);
         if (rc) return rc;
         switch (k) {
-            case 0: return launch_diag<R, 0>(s, tbits, ctrl_mask, cpos, d);
-            case 1: return launch_diag<R, 1>(s, tbits, ctrl_mask, cpos, d);
-            case 2: return launch_diag<R, 2>(s, tbits, ctrl_mask, cpos, d);
             case 3: return launch_diag<R, 3>(s, tbits, ctrl_mask, cpos, d);
             case 4: return launch_diag<R, 4>(s, tbits, ctrl_mask, cpos, d);
             case 5: return launch_diag<R, 5>(s, tbits, ctrl_mask, cpos, d);
@@ -1343,12 +1082,15 @@ static int dispatch(qipgpu_state *s, const Analysed &an, const std::vector<int32
         }
         return diag_large(s, tbits, ctrl_mask, cpos, d.data());
     }
-    if (k == 1 && s->n >= 12 && __builtin_popcountll((ctrl_mask | (1ull << tbits[0])) & ~0xfull) <= 8)
-        return hold_single(s, tbits[0], ctrl_mask, an.U);
+    if (k == 1 || (k == 2 && is_swap(an.U))) {
+        HeldGate g;
+        set_bits(g, k == 1 ? HeldGate::kSingle : HeldGate::kSwap, tbits, ctrl_mask);
+        if (k == 1) set_entries(g, an.U.data(), 4);
+        return hold_gate(s, g);
+    }
     const int rc = flush_held(s);
     if (rc) return rc;
     switch (k) {
-        case 1: return launch_dense_reg<R, 1>(s, tbits, ctrl_mask, allpos, an.U);
         case 2: return launch_dense_reg<R, 2>(s, tbits, ctrl_mask, allpos, an.U);
         case 3: return launch_dense_reg<R, 3>(s, tbits, ctrl_mask, allpos, an.U);
         default: break;
@@ -1366,14 +1108,12 @@ static int check_disjoint(const qipgpu_state *s, int32_t k, const int32_t *t, in
 
 namespace qipgpu {
 
-int flush_held(qipgpu_state *s) {
-    const bool c128 = s->dtype == QIPGPU_C128;
-    if (s->chain_len) {
-        const int rc = c128 ? flush_chain_typed<double>(s) : flush_chain_typed<float>(s);
-        if (rc) return rc;
-    }
-    if (s->run_len) return c128 ? flush_run_typed<double>(s) : flush_run_typed<float>(s);
-    return QIPGPU_OK;
+int launch_held_gate(qipgpu_state *s, const HeldGate &g) {
+    return s->dtype == QIPGPU_C128 ? launch_one<double>(s, g) : launch_one<float>(s, g);
+}
+
+int launch_diag_chain(qipgpu_state *s, const HeldGate *g, int count) {
+    return s->dtype == QIPGPU_C128 ? launch_chain<double>(s, g, count) : launch_chain<float>(s, g, count);
 }
 
 }  // namespace qipgpu
@@ -1387,8 +1127,8 @@ int qipgpu_apply_matrix(qipgpu_state *s, int32_t k, const int32_t *targets, cons
     int rc = check_disjoint(s, k, targets, n_ctrl, controls);
     if (rc) return rc;
     // linear in the state: a pending fused renormalisation (a scalar) stays pending; recorded gates
-    // go first (with the diagonal gates held back before them); held-back diagonal gates otherwise
-    // stay held, and dispatch applies them before anything that is not held
+    // go first (with the gates held back before them); held-back gates otherwise stay held, and
+    // dispatch applies them before anything that is not held
     rc = recorder_pending(s) ? flush_recorded(s) : QIPGPU_OK;
     if (rc) return rc;
     Analysed an = analyse(k, targets, mat);

@@ -1,0 +1,96 @@
+"""Held-back runs (marked gpu): single-qubit gates, swaps and diagonals under any controls wait on the
+state and go in passes over 4096-amplitude tiles, gates that round nothing (X, swaps, -1 factors)
+joining an earlier pass where that changes no value. Every run must equal, bit for bit, the same gates
+each launched alone (a synchronisation after every gate), and be within 1e-12 of the oracle."""
+import numpy
+import pytest
+
+from oracle.oracle_backend import OracleBackend
+from qip_amd import CMat, GpuBackend, SwapMat
+
+pytestmark = pytest.mark.gpu
+HM = numpy.array([[1.0, 1.0], [1.0, -1.0]]) / numpy.sqrt(2.0)
+XM = numpy.array([[0.0, 1.0], [1.0, 0.0]])
+ZM = numpy.diag([1.0, -1.0])
+
+
+def unitary(rng):
+    z = rng.standard_normal((2, 2)) + 1j * rng.standard_normal((2, 2))
+    q, r = numpy.linalg.qr(z)
+    return q * (numpy.diagonal(r) / numpy.abs(numpy.diagonal(r)))
+
+
+def gate(rng, n):
+    """A held gate on random qubits: Haar, H, X, phases, Z, a two-target diagonal or a swap, under up to
+    three controls."""
+    kind = int(rng.integers(0, 8))
+    width = 2 if kind in (5, 6) and n >= 2 else 1
+    controls = int(min(rng.integers(0, 4), n - width)) if rng.random() < 0.6 else 0
+    qs = tuple(int(q) for q in rng.permutation(n)[:controls + width])
+    if width == 2:
+        m = SwapMat(1) if kind == 5 else numpy.diag(numpy.exp(1j * rng.uniform(0, 6, 4)))
+    else:
+        m = [unitary(rng), HM, XM, ZM, numpy.diag([1.0, numpy.exp(1j * rng.uniform(0, 6))]),
+             numpy.diag(numpy.exp(1j * rng.uniform(0, 6, 2))), XM, unitary(rng)][kind]
+    for _ in range(controls):
+        m = CMat(m)
+    return {qs: m}
+
+
+def check(n, dtype, seq, rng, oracle):
+    psi = rng.standard_normal(2 ** n) + 1j * rng.standard_normal(2 ** n)
+    psi /= numpy.linalg.norm(psi)
+    held = GpuBackend.make_state(n, [list(range(n))], [psi], statetype=dtype)
+    alone = GpuBackend.make_state(n, [list(range(n))], [psi], statetype=dtype)
+    for d in seq:
+        held.kronselect_dot(d)
+        alone.kronselect_dot(d)
+        alone.synchronize()
+    got = held.get_state()
+    assert numpy.array_equal(got, alone.get_state())
+    if oracle:
+        ora = OracleBackend.make_state(n, [list(range(n))], [psi])
+        for d in seq:
+            ora.kronselect_dot(d)
+        assert numpy.max(numpy.abs(got - ora.get_state())) < 1e-12
+    held.close()
+    alone.close()
+
+
+@pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 8, 11, 12, 13, 17, 22])
+def test_mixed_runs_equal_separate_launches(n, dtype):
+    rng = numpy.random.default_rng(700 + n)
+    print("mixed runs n", n, numpy.dtype(dtype).name, flush=True)
+    check(n, dtype, [gate(rng, n) for _ in range(230)], rng, dtype == numpy.complex128 and n <= 13)
+
+
+@pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
+@pytest.mark.parametrize("low", [False, True])
+def test_layers_whose_two_qubit_gates_straddle_tiles(low, dtype):
+    """Haar layers with CNOTs, swaps and CZs between neighbours and across the register: the two-qubit
+    gates join passes whose tiles hold only the bits they change; targets on every tile position."""
+    n = 21
+    rng = numpy.random.default_rng(31 + low)
+    seq = []
+    for layer in range(5):
+        qs = list(range(n))[::-1 if low else 1]
+        seq += [{q: unitary(rng)} for q in qs]
+        seq += [{(q, q + 1): CMat(XM if layer % 2 else ZM)} for q in range(layer % 2, n - 1, 2)]
+        seq += [{(q, n - 1 - q): SwapMat(1)} for q in range(layer, n // 2, 2)]
+        seq += [{(n - 1 - q, q): CMat(numpy.diag([1.0, numpy.exp(0.3j * q)]))} for q in range(n // 2)]
+    print("layers n", n, numpy.dtype(dtype).name, "low" if low else "high", flush=True)
+    check(n, dtype, seq, rng, False)
+
+
+def test_runs_longer_than_a_launch_holds():
+    """More diagonals and coefficients than one launch's arguments hold, between gates that change bits."""
+    n = 14
+    rng = numpy.random.default_rng(5)
+    seq = []
+    for t in range(n):
+        seq.append({t: HM})
+        seq += [{(i, t): CMat(numpy.diag([1.0, numpy.exp(2j * numpy.pi / 2 ** (1 + i - t))]))} for i in range(t + 1, n)]
+    seq += [{(i, n - 1 - i): SwapMat(1)} for i in range(n // 2)]
+    seq += [{(0, 1): numpy.diag(numpy.exp(1j * rng.uniform(0, 6, 4)))} for _ in range(70)]
+    check(n, numpy.complex128, seq, rng, True)
