@@ -7,12 +7,10 @@
 // sum_j U[i][j] * in[base + off[j]]. That is the matrix product Y = U X with X[j][b] the amplitudes
 // of base b. FP64 arithmetic for both state precisions, rounded once on store.
 //
-//   k_dense_mfma<R, K>   K = 4..6, in place. A persistent workgroup takes tiles of B bases: it stages
-//                        X (D x B = 2048 amplitudes, 32 KB in FP64) in LDS as Re / Im planes, forms
-//                        Y = U X with three real products on FP64 MFMA (v_mfma_f64_16x16x4f64), each
-//                        wave holding its share of Re U and Im U in registers for the launch, and
-//                        writes Y back through the same planes. A tile holds every amplitude of its
-//                        bases before any is written, so in place is safe.
+//   k_dense_mfma<R, K>   K = 4..6, in place. Each wave forms Y = U X for 1024 amplitudes at a time with
+//                        three real products on FP64 MFMA (v_mfma_f64_16x16x4f64), U's fragments in
+//                        LDS. It holds every amplitude of its bases before any is written, so in place
+//                        is safe.
 //   k_dense_gemm<R>      K = 7..12, out of place: a 64 x 64 output tile per workgroup over 16-column
 //                        steps of j through LDS, into a compact [D][nbase] buffer; k_dense_scatter
 //                        writes it back to the bases' positions.
@@ -59,8 +57,6 @@ __device__ __forceinline__ uint64_t base_of(uint64_t g, const PosList &pl, uint6
     return insert_zeros(g, pl) | ctrl_mask;
 }
 
-constexpr int kTileThreads = 256;
-
 // ---- K = 4..6: tiles in place on FP64 MFMA -------------------------------------------------------
 //
 // Y = U X with U = A + i Bm and X = P + i Q takes three real D x D products (the 3M method, Higham,
@@ -71,194 +67,145 @@ constexpr int kTileThreads = 256;
 // terms of (|A| + |Bm|)(|P| + |Q|) instead of |A||Q| + |Bm||P|, at most a small constant factor more
 // in FP64 (the paper's bound).
 // v_mfma_f64_16x16x4f64 computes D[16 x 16] += A[16 x 4] B[4 x 16]; lane l holds A[l % 16][l / 16]
-// and B[l / 16][l % 16], and D[4 i + l / 16][l % 16] for its items i = 0..3, so the three products of
-// one output block land in the same lanes and are combined in registers.
+// and B[l / 16][l % 16], and D[4 i + l / 16][l % 16] for its items i = 0..3.
 //
-// Wave w owns output row block w % RB (RB = D / 16 blocks of 16 complex rows) and CW consecutive
-// 16-base column blocks starting at (w / RB) CW; its fragments of A and Bm (2 x D / 4 doubles per
-// lane) are gathered from U once per launch and stay in registers, and A + Bm is formed per k-step.
-// X goes through LDS as two FP64 planes (Re, Im) with one slot of padding per row (or per base, when
-// lanes run along the rows), and so does Y on its way out, so loads and stores stay coalesced. Per
-// tile: 3 D x D x B FMAs in 3 x (D / 4) x CW MFMAs per wave.
+// A wave works by itself on tiles of 1024 amplitudes: all D rows of 16 CB bases, 16 CB D = 1024. The rows
+// are numbered with their bits in state-bit order, so that item i of output row block rb (row 16 rb + 4 i
+// + l / 16) is the row the lane loaded for k-step 4 rb + i: amplitudes go from memory to the lanes
+// that multiply them and back from the same addresses, with no LDS in between. Sixteen lanes run along
+// the bases and the other four ways along the two lowest targets, so a load instruction reads runs of
+// 16 bases when the targets are high bits and of the four rows (64 B of complex128) when they are low.
+// U's fragments (64 KB at K = 6) are in LDS, where all waves read them; nothing else is, so the
+// tile loop has no barrier: while one wave of a SIMD loads or stores, the other's MFMAs run, and the
+// next tile's loads are in flight during this one's.
+// Bound: HBM, and at K = 6 on complex64 states the MFMAs (1.41 ms on 2^28 amplitudes at the 73 TFLOP/s
+// that a large FP64 product reaches). Per call on 2^28 amplitudes, targets low / high / scattered,
+// with the tile in LDS (four barriers a tile) before, and now; a copy takes 1.63 (complex128) and
+// 0.81 ms (complex64):
+//   complex128 K = 4 1.77 / 1.89 / 1.84 -> 1.90 / 1.66 / 1.72 ms; K = 5 1.95 / 1.77 / 1.96 -> 1.87 / 1.67 /
+//   1.78; K = 6 2.93 / 2.45 / 2.39 -> 1.75 / 1.79 / 1.76
+//   complex64 K = 4 1.40 / 1.05 / 1.05 -> 1.11 / 0.85 / 0.93; K = 5 1.95 / 1.51 / 1.51 -> 1.10 / 0.96 / 0.92;
+//   K = 6 2.93 / 2.38 / 2.38 -> 1.62 / 1.61 / 1.60
+// Workgroups take tiles a grid apart: 1.66 against 1.74 ms (K = 4, high targets) with contiguous ranges.
 template <int K>
 struct MfmaShape {
     static constexpr int D = 1 << K;
-    // 2048 amplitudes per tile: 34 KB of LDS and at most 168 VGPRs, so three workgroups share a CU
-    // (three waves per SIMD); with 4096 (67 KB) only two fit, which left the MFMA units idle while
-    // a workgroup loads or stores
-    static constexpr int TE = 2048;
-    static constexpr int WGS = 3;                // workgroups per CU
-    static constexpr int B = TE / D;             // bases per tile
-    static constexpr int LOADS = TE / kTileThreads;   // amplitudes per thread
+    static constexpr int KS = D / 4;             // 4-row k-steps
     static constexpr int RB = D / 16;            // 16-row output blocks
-    static constexpr int CB = B / 16;            // 16-column blocks
-    static constexpr int CW = CB * RB / 4;       // column blocks per wave (4 waves)
-    static constexpr int KS = D / 4;             // 4-column k-steps over the D complex columns
-    static constexpr int XS = B + 1;             // padded plane row, row-major planes (doubles)
-    static constexpr int XSJ = D + 1;            // padded plane column, base-major planes
-    static constexpr int PLANE = D * B + (D > B ? D : B);
+    static constexpr int CB = 64 / D;            // 16-base column blocks of a wave's tile
+    static constexpr int NR = K == 4 ? 1 : 2;    // output blocks formed at a time: NR rows of NC columns
+    static constexpr int NC = K == 4 ? 2 : 1;
+    static constexpr int BASES = 16 * CB;
     static_assert(K >= 4 && K <= 6, "MFMA tiles for 4 to 6 targets");
-    static_assert(CW * 4 == CB * RB, "column blocks split evenly over the waves");
 };
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef double f64x2 __attribute__((ext_vector_type(2)));
 
-template <typename R, int K, bool ROWS_FAST>
-__global__ __launch_bounds__(kTileThreads, MfmaShape<K>::WGS) void k_dense_mfma(cx<R> *amps, uint64_t nbase, uint64_t ctrl_mask,
-                                                                PosList pl, const uint64_t *__restrict__ off_g,
-                                                                const cx<double> *__restrict__ U_g, uint64_t ntiles) {
+constexpr int kTileThreads = 256;
+constexpr int kTileWaves = kTileThreads / 64;
+
+template <typename R, int K>
+struct DenseTileArgs {
+    cx<R> *amps;
+    uint64_t nbase;
+    uint64_t ntiles;                        // tiles of 16 CB bases
+    PosList pl;                             // target and control bits
+    uint64_t row_k[4];                      // offset of the two lowest targets' values, and the controls
+    uint64_t row_s[MfmaShape<K>::KS];       // offset of the other targets' values
+};
+
+template <typename R, int K>
+__global__ __launch_bounds__(kTileThreads, 2) void k_dense_mfma(const DenseTileArgs<R, K> a,
+                                                                const f64x2 *__restrict__ frag) {
     using M = MfmaShape<K>;
-    constexpr int D = M::D, B = M::B, XS = M::XS;
-    // Re and Im planes of the tile: row-major (row * XS + base) when lanes run along the bases,
-    // base-major (base * XSJ + row) when they run along the rows, so that consecutive lanes touch
-    // consecutive slots in the loads and stores and the MFMA operand reads spread over the banks
-    constexpr int XSJ = M::XSJ;
-    __shared__ double sX[2][M::PLANE];
-    auto idx = [](int j, int b) { return ROWS_FAST ? b * XSJ + j : j * XS + b; };
-    __shared__ uint64_t sOff[D];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, wave = tid >> 6;
-    for (int e = tid; e < D; e += kTileThreads) sOff[e] = off_g[e];
-
-    // this wave's fragments: lane -> output row rho = lane % 16 of its block, k = lane / 16 of each
-    // k-step; afr[0] = Re U, afr[1] = Im U (Re U + Im U is formed per k-step)
-    const int rho = lane & 15, kap = lane >> 4;
-    const int row0 = 16 * (wave % M::RB);        // first output row of the wave's block
-    const int col0 = 16 * M::CW * (wave / M::RB); // first base of the wave's column blocks
-    double afr[2][M::KS];
-#pragma unroll
-    for (int s = 0; s < M::KS; ++s) {
-        const cx<double> u = U_g[(row0 + rho) * D + 4 * s + kap];
-        afr[0][s] = u.re;
-        afr[1][s] = u.im;
-    }
+    constexpr int NF = M::KS * M::RB * 64;
+    __shared__ f64x2 sU[NF];                // [k-step][row block][lane]: Re and Im of U
+    for (int e = threadIdx.x; e < NF; e += kTileThreads) sU[e] = frag[e];
     __syncthreads();
-
-    // loads and stores: element i of this thread is (row j, base b); lanes run along the bases, or
-    // along the rows when ROWS_FAST
-    constexpr int BSTEP = kTileThreads / D;
-    constexpr int JSTEP = kTileThreads / B;
-    const int b_ld = ROWS_FAST ? tid / D : tid % B;
-    const int j_ld = ROWS_FAST ? tid % D : tid / B;
-    cx<R> pre[M::LOADS];
-    // position of base t B + v (v < B; a base past the end reads the last one, whose products are
-    // not stored)
-    auto base_at = [&](uint64_t t, int v) {
-        const uint64_t g = t * B + v;
-        return base_of(g < nbase ? g : nbase - 1, pl, ctrl_mask);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // this lane's part of its bases' positions; lanes past the last base work on an earlier one and
+    // store nothing (there is one tile then)
+    uint64_t at[M::CB];
+    bool stored[M::CB];
+#pragma unroll
+    for (int c = 0; c < M::CB; ++c) {
+        const uint64_t g = 16 * c + (lane & 15);
+        stored[c] = g < a.nbase;
+        const int kap = lane >> 4;
+        const uint64_t row = kap & 2 ? (kap & 1 ? a.row_k[3] : a.row_k[2]) : (kap & 1 ? a.row_k[1] : a.row_k[0]);
+        at[c] = insert_zeros(g & (a.nbase - 1), a.pl) + row;
+    }
+    const uint64_t step = (uint64_t)gridDim.x * kTileWaves, end = a.ntiles;
+    uint64_t t = (uint64_t)blockIdx.x * kTileWaves + wave;
+    if (t >= end) return;
+    auto tile_at = [&](uint64_t tile) { return a.amps + insert_zeros(tile * M::BASES, a.pl); };
+    auto load = [&](cx<R> (&x)[16], uint64_t tile) {
+        const cx<R> *p = tile_at(tile);
+        // a base's rows one after the other: low targets' rows share cache lines
+#pragma unroll
+        for (int c = 0; c < M::CB; ++c)
+#pragma unroll
+            for (int s = 0; s < M::KS; ++s) x[s * M::CB + c] = p[at[c] + a.row_s[s]];
     };
-    auto load_tile = [&](uint64_t t) {
-        if constexpr (ROWS_FAST) {
+    auto process = [&](const cx<R> (&x)[16], uint64_t tile) {
+        cx<R> *p = tile_at(tile);
 #pragma unroll
-            for (int i = 0; i < M::LOADS; ++i) pre[i] = amps[base_at(t, b_ld + BSTEP * i) + sOff[j_ld]];
-        } else {
-            const uint64_t base = base_at(t, b_ld);
+        for (int r0 = 0; r0 < M::RB; r0 += M::NR)
 #pragma unroll
-            for (int i = 0; i < M::LOADS; ++i) pre[i] = amps[base + sOff[j_ld + i * JSTEP]];
-        }
-    };
-    // plane slot of element i of this thread
-    auto slot = [&](int i) { return ROWS_FAST ? idx(j_ld, b_ld + BSTEP * i) : idx(j_ld + i * JSTEP, b_ld); };
-
-    // the tile's amplitudes (pre) into LDS as Re and Im planes
-    auto write_x = [&]() {
+            for (int c0 = 0; c0 < M::CB; c0 += M::NC) {
+                // U's fragments are read again for every tile: kept in registers over the loop they would spill
+                asm volatile("" ::: "memory");
+                f64x4 acc[3][M::NR][M::NC];
 #pragma unroll
-        for (int i = 0; i < M::LOADS; ++i) {
-            const cx<double> v = to_d(pre[i]);
-            sX[0][slot(i)] = v.re;
-            sX[1][slot(i)] = v.im;
-        }
-    };
-    f64x4 acc[3][M::CW];
-    // the three products of the tile in LDS: lanes read P and Q of row 4 s + kap, base col0 + 16 c + rho
-    auto products = [&]() {
+                for (int m = 0; m < 3; ++m)
 #pragma unroll
-        for (int m = 0; m < 3; ++m)
+                    for (int r = 0; r < M::NR; ++r)
 #pragma unroll
-            for (int c = 0; c < M::CW; ++c) acc[m][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+                        for (int c = 0; c < M::NC; ++c) acc[m][r][c] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-        for (int s = 0; s < M::KS; ++s) {
-            // the empty asm makes the copies opaque, so the sum below stays in the tile loop instead
-            // of being hoisted out of it as a third set of fragment registers
-            double a0 = afr[0][s], a1 = afr[1][s];
-            asm volatile("" : "+v"(a0), "+v"(a1));
-            const double a2 = a0 + a1;
-            const int at = idx(4 * s + kap, col0 + rho);
-            double p[M::CW], q[M::CW];
+                for (int s = 0; s < M::KS; ++s) {
+                    f64x2 u[M::NR];
 #pragma unroll
-            for (int c = 0; c < M::CW; ++c) {
-                p[c] = sX[0][at + idx(0, 16 * c)];
-                q[c] = sX[1][at + idx(0, 16 * c)];
-            }
+                    for (int r = 0; r < M::NR; ++r) u[r] = sU[(s * M::RB + r0 + r) * 64 + lane];
 #pragma unroll
-            for (int c = 0; c < M::CW; ++c) {
-                acc[0][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, p[c], acc[0][c], 0, 0, 0);
-                acc[1][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, q[c], acc[1][c], 0, 0, 0);
-                acc[2][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a2, p[c] + q[c], acc[2][c], 0, 0, 0);
-            }
-        }
-    };
-    // item i of a block is output row row0 + 4 i + kap, base col0 + 16 c + rho
-    auto write_y = [&]() {
+                    for (int c = 0; c < M::NC; ++c) {
+                        const cx<double> v = to_d(x[s * M::CB + c0 + c]);
+                        const double sum = v.re + v.im;
 #pragma unroll
-        for (int c = 0; c < M::CW; ++c)
+                        for (int r = 0; r < M::NR; ++r) {
+                            acc[0][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[r][0], v.re, acc[0][r][c], 0, 0, 0);
+                            acc[1][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[r][1], v.im, acc[1][r][c], 0, 0, 0);
+                            acc[2][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[r][0] + u[r][1], sum, acc[2][r][c], 0, 0, 0);
+                        }
+                    }
+                }
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int at = idx(row0 + 4 * i + kap, col0 + 16 * c + rho);
-                const double t1 = acc[0][c][i], t2 = acc[1][c][i];
-                sX[0][at] = t1 - t2;
-                sX[1][at] = acc[2][c][i] - t1 - t2;
+                for (int r = 0; r < M::NR; ++r)
+#pragma unroll
+                    for (int c = 0; c < M::NC; ++c)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const double t1 = acc[0][r][c][i], t2 = acc[1][r][c][i];
+                            cx<double> y;
+                            y.re = t1 - t2;
+                            y.im = acc[2][r][c][i] - t1 - t2;
+                            if (stored[c0 + c]) p[at[c0 + c] + a.row_s[4 * (r0 + r) + i]] = from_d<R>(y);
+                        }
             }
     };
-    // the tile's outputs from LDS to the state, with the load mapping
-    auto store_y = [&](uint64_t t) {
-#pragma unroll
-        for (int i = 0; i < M::LOADS; ++i) {
-            const int v = ROWS_FAST ? b_ld + BSTEP * i : b_ld;
-            if (t * B + v < nbase) {
-                cx<double> y;
-                y.re = sX[0][slot(i)];
-                y.im = sX[1][slot(i)];
-                const int j = ROWS_FAST ? j_ld : j_ld + i * JSTEP;
-                amps[base_at(t, v) + sOff[j]] = from_d<R>(y);
-            }
-        }
-    };
-
-    const uint64_t G = gridDim.x;
-    uint64_t t = blockIdx.x;
-    if (t >= ntiles) return;                   // the whole workgroup: no barrier is skipped by part of it
-    // the next tile's loads in registers while the products run, where they fit beside the
-    // fragments and accumulators at three workgroups per CU (all but K = 6 with lanes along the rows,
-    // whose extra address registers would spill); otherwise the other workgroups on the CU cover
-    // this one's loads
-    constexpr bool kPrefetch = K <= 5 || !ROWS_FAST;
-    if constexpr (kPrefetch) {
-        load_tile(t);
-        for (; t < ntiles; t += G) {
-            __syncthreads();                   // the previous tile's outputs have been read back
-            write_x();
-            __syncthreads();
-            if (t + G < ntiles) load_tile(t + G);   // in flight during the products
-            products();
-            __syncthreads();                   // every wave has read X
-            write_y();
-            __syncthreads();
-            store_y(t);
-        }
-    } else {
-        // no prefetch registers: the other workgroup on the CU covers this one's loads
-        for (; t < ntiles; t += G) {
-            __syncthreads();
-            load_tile(t);
-            write_x();
-            __syncthreads();
-            products();
-            __syncthreads();
-            write_y();
-            __syncthreads();
-            store_y(t);
-        }
+    // two register buffers alternate (the last prefetch re-reads an in-range tile and is not used)
+    cx<R> xa[16], xb[16];
+    load(xa, t);
+    for (;;) {
+        const uint64_t t1 = t + step, t2 = t1 + step;
+        load(xb, min(t1, end - 1));
+        process(xa, t);
+        if (t1 >= end) return;
+        load(xa, min(t2, end - 1));
+        process(xb, t1);
+        if (t2 >= end) return;
+        t = t2;
     }
 }
 
@@ -491,26 +438,40 @@ PosList poslist(std::vector<int> pos) {
 template <typename R, int K>
 int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<int> &allpos,
                 const std::complex<double> *U) {
-    constexpr int D = 1 << K;
-    const std::vector<uint64_t> off = offsets(tbits);
-    std::vector<char> host(sizeof(uint64_t) * D + sizeof(cx<double>) * D * D);
-    std::memcpy(host.data(), off.data(), sizeof(uint64_t) * D);
-    std::memcpy(host.data() + sizeof(uint64_t) * D, U, sizeof(cx<double>) * D * D);
+    using M = MfmaShape<K>;
+    constexpr int D = M::D;
+    // rows in state-bit order: bit b of a row is the b-th lowest target bit; its place in the caller's index
+    std::vector<int> sorted(tbits);
+    std::sort(sorted.begin(), sorted.end());
+    int caller[D];
+    for (int j = 0; j < D; ++j) {
+        caller[j] = 0;
+        for (int t = 0; t < K; ++t) {
+            const int b = (int)(std::find(sorted.begin(), sorted.end(), tbits[t]) - sorted.begin());
+            caller[j] |= (j >> b & 1) << (K - 1 - t);
+        }
+    }
+    DenseTileArgs<R, K> a;
+    std::memset(&a, 0, sizeof(a));
+    a.amps = (cx<R> *)s->amps;
+    a.nbase = s->len >> allpos.size();
+    a.ntiles = (a.nbase + M::BASES - 1) / M::BASES;
+    a.pl = poslist(allpos);
+    for (int j = 0; j < 4; ++j)
+        a.row_k[j] = ctrl_mask + ((uint64_t)(j & 1) << sorted[0]) + ((uint64_t)(j >> 1) << sorted[1]);
+    for (int j = 0; j < M::KS; ++j)
+        for (int b = 2; b < K; ++b) a.row_s[j] += (uint64_t)(j >> (b - 2) & 1) << sorted[b];
+    std::vector<std::complex<double>> frag((size_t)D * D);
+    for (int st = 0; st < M::KS; ++st)
+        for (int rb = 0; rb < M::RB; ++rb)
+            for (int l = 0; l < 64; ++l)
+                frag[(st * M::RB + rb) * 64 + l] = U[caller[16 * rb + l % 16] * D + caller[4 * st + l / 16]];
     void *d = nullptr;
-    int rc = ring_upload(s, host.data(), host.size(), &d);
+    int rc = ring_upload(s, frag.data(), frag.size() * sizeof(frag[0]), &d);
     if (rc) return rc;
-    const uint64_t nbase = s->len >> allpos.size();
-    const uint64_t ntiles = (nbase + MfmaShape<K>::B - 1) / MfmaShape<K>::B;
-    const bool rows_fast = std::find(tbits.begin(), tbits.end(), 0) != tbits.end();
-    const cx<double> *dU = (const cx<double> *)((char *)d + sizeof(uint64_t) * D);
-    // FP64 MFMA: the waves hold their operator fragments in registers; two workgroups per CU
-    const uint64_t grid = std::min<uint64_t>(ntiles, (uint64_t)device_cus() * MfmaShape<K>::WGS);
-    if (rows_fast)
-        hipLaunchKernelGGL((k_dense_mfma<R, K, true>), dim3((uint32_t)grid), dim3(kTileThreads), 0, s->stream,
-                           (cx<R> *)s->amps, nbase, ctrl_mask, poslist(allpos), (const uint64_t *)d, dU, ntiles);
-    else
-        hipLaunchKernelGGL((k_dense_mfma<R, K, false>), dim3((uint32_t)grid), dim3(kTileThreads), 0, s->stream,
-                           (cx<R> *)s->amps, nbase, ctrl_mask, poslist(allpos), (const uint64_t *)d, dU, ntiles);
+    const uint64_t grid = std::min<uint64_t>((a.ntiles + kTileWaves - 1) / kTileWaves, (uint64_t)device_cus() * 2);
+    hipLaunchKernelGGL((k_dense_mfma<R, K>), dim3((uint32_t)grid), dim3(kTileThreads), 0, s->stream, a,
+                       (const f64x2 *)d);
     QIP_LAUNCHED();
     return QIPGPU_OK;
 }
