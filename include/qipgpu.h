@@ -321,7 +321,7 @@ typedef struct qipgpu_batch qipgpu_batch;
 typedef struct {
     int32_t fusion_width;   /* 1..6: qubits per fused block of the large states (default 6) */
     int32_t lds_max_qubits; /* 11..13: states with n <= this run whole in LDS (default 13) */
-    int32_t chunk_tiles;    /* 1..64: 4096-amplitude tiles per workgroup in a block pass (default 8) */
+    int32_t chunk_tiles;    /* 1..64: most 4096-amplitude tiles per workgroup in a block pass (default 8) */
     int32_t use_graph;      /* 1: a run replays one captured hipGraph (default); 0: eager launches */
 } qipgpu_batch_tuning;
 

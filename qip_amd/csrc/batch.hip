@@ -9,10 +9,11 @@
 //     light-cone rule (plan.h). Block j of every tiled state belongs to wave j. Per wave:
 //       k_batch_build -- one workgroup per block: the 64x64 operator (block qubits padded to six
 //         with free state bits, tile6.h) composed from its gates in FP64 in LDS, split into BF16
-//         hi/lo MFMA fragments. Builds run on a second stream, one wave ahead, into two
-//         alternating fragment sets, so they overlap the previous wave's tile passes;
+//         hi/lo MFMA fragments. Builds run on a second stream, a group of waves at a time and one
+//         group ahead, into two alternating fragment sets, so they overlap the tile passes of the
+//         group before;
 //       k_batch_scales -- the renormalisation factor of each block from the FP64 norm partials of
-//         the same state's previous block;
+//         the same state's previous block, where those are too many for k_batch6 to sum itself;
 //       k_batch6 -- one workgroup per chunk of `chunk_tiles` tiles of one block (tile6.h),
 //         double-buffered loads within the chunk, FP64 norm partial per chunk.
 //   * k_batch_finish applies every tiled state's last renormalisation.
@@ -41,6 +42,16 @@ constexpr int kLdsMaxQubits = 13;        // 2 x 2^13 complex64 = 128 KB of LDS
 constexpr int kSmallThreads = 512;
 constexpr uint32_t kFinishSegment = 1u << 16;   // amplitudes per finishing workgroup
 constexpr size_t kStateAlign = 512;             // amplitudes (4 KB) between state slices
+// Operators are built a group of waves at a time, enough waves for two blocks per CU: a wave of a small
+// batch has fewer blocks than the GPU has CUs, and a build per wave then makes the waves wait for one
+// build after another (48 circuits of 10 to 20 qubits: 30 builds of 71 us, 2.1 of 2.5 ms).
+constexpr uint32_t kBuildBlocks = 512;
+// Chunks a wave is cut into at least, where it has that many tiles: two workgroups for each CU (the same
+// batch, 1400 tiles a wave: 1.19 ms a run with chunks of 8 tiles, 1.04 with 1 to 4).
+constexpr uint64_t kWaveChunks = 512;
+// Norm partials up to which a tile pass sums its blocks' factors itself (8 loads a lane); more of them
+// go through k_batch_scales, a launch per wave.
+constexpr uint32_t kMaxOwnPartials = 512;
 
 struct BGate {
     uint32_t mat;    // offset of the 2^k x 2^k complex128 matrix (ascending-bit order)
@@ -111,6 +122,29 @@ __device__ double group_sum_256(const double *__restrict__ partials, uint32_t p0
     return total;
 }
 
+// The next gates of a list in LDS: their headers, and the matrices of those on one or two qubits. A gate
+// read from memory when its turn comes costs two memory latencies in a row (its header, then its
+// matrix), more than its arithmetic; a chunk's are read side by side.
+constexpr uint32_t kGateChunk = 32;
+
+struct GateStage {
+    BGate gate[kGateChunk];
+    cx<double> mat[kGateChunk][16];
+};
+
+// Stage `count` (at most kGateChunk) gates; a barrier before, two after the loads.
+__device__ __forceinline__ void stage_gates(GateStage &st, const BGate *__restrict__ gates, uint32_t count,
+                                            const cx<double> *__restrict__ mats) {
+    __syncthreads();   // every wave is done with the gates staged before
+    for (uint32_t i = threadIdx.x; i < count; i += blockDim.x) st.gate[i] = gates[i];
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < count * 16; i += blockDim.x) {
+        const BGate g = st.gate[i >> 4];
+        if (g.k <= 2 && (i & 15u) < 1u << 2 * g.k) st.mat[i >> 4][i & 15u] = mats[g.mat + (i & 15u)];
+    }
+    __syncthreads();
+}
+
 __device__ __forceinline__ double renorm_factor(double norm) { return norm > 0.0 ? 1.0 / sqrt(norm) : 1.0; }
 
 // ---- reset ----------------------------------------------------------------------------------
@@ -143,6 +177,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_batch_small(cx<float> *arena,
                                                                const cx<double> *__restrict__ mats) {
     __shared__ cx<float> buf[2 << kLdsMaxQubits];
     __shared__ double red[kSmallThreads];
+    __shared__ GateStage stage;
     const BSmall st = smalls[blockIdx.x];
     const uint32_t len = 1u << st.n;
     const uint32_t tid = threadIdx.x;
@@ -151,8 +186,13 @@ __global__ __launch_bounds__(kSmallThreads) void k_batch_small(cx<float> *arena,
     for (uint32_t i = tid; i < len; i += kSmallThreads) cur[i] = amps[i];
     __syncthreads();
     for (uint32_t g = 0; g < st.ngates; ++g) {
-        const BGate gt = gates[st.gate0 + g];
-        const cx<double> *G = mats + gt.mat;
+        const uint32_t slot = g % kGateChunk;
+        if (slot == 0) stage_gates(stage, gates + st.gate0 + g, min(kGateChunk, st.ngates - g), mats);
+        BGate gt;
+        gt.k = __builtin_amdgcn_readfirstlane(stage.gate[slot].k);
+        gt.mask = __builtin_amdgcn_readfirstlane(stage.gate[slot].mask);
+        gt.mat = __builtin_amdgcn_readfirstlane(stage.gate[slot].mat);
+        const cx<double> *G = stage.mat[slot];
         if (gt.k == 1) {
             const uint32_t m = gt.mask, lowm = m - 1u;
             const cx<double> g00 = G[0], g01 = G[1], g10 = G[2], g11 = G[3];
@@ -176,6 +216,9 @@ __global__ __launch_bounds__(kSmallThreads) void k_batch_small(cx<float> *arena,
             }
         } else if (gt.k == 2) {
             const uint32_t mlo = gt.mask & (0u - gt.mask), mhi = gt.mask ^ mlo;
+            cx<double> gm[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) gm[t] = G[t];
             for (uint32_t p = tid; p < (len >> 2); p += kSmallThreads) {
                 uint32_t i = ((p & ~(mlo - 1u)) << 1) | (p & (mlo - 1u));
                 i = ((i & ~(mhi - 1u)) << 1) | (i & (mhi - 1u));
@@ -191,7 +234,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_batch_small(cx<float> *arena,
                 for (int r = 0; r < 4; ++r) {
                     cx<double> y = {0.0, 0.0};
 #pragma unroll
-                    for (int t = 0; t < 4; ++t) y = cmul_acc(y, G[4 * r + t], x[t]);
+                    for (int t = 0; t < 4; ++t) y = cmul_acc(y, gm[4 * r + t], x[t]);
                     cx<float> o;
                     o.re = (float)y.re;
                     o.im = (float)y.im;
@@ -200,6 +243,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_batch_small(cx<float> *arena,
             }
         } else {
             // k >= 3: each output from the 2^k inputs of its group, into the other buffer
+            G = mats + gt.mat;
             const uint32_t m = gt.mask, D = 1u << gt.k;
             for (uint32_t e = tid; e < len; e += kSmallThreads) {
                 const uint32_t s = gather_bits(e, m), base = e & ~m;
@@ -249,82 +293,97 @@ __global__ __launch_bounds__(kSmallThreads) void k_batch_small(cx<float> *arena,
 
 // ---- tiled states ---------------------------------------------------------------------------
 
+constexpr uint32_t kBuildRow = 65;
+
+// The operator of each block of a group of waves: one workgroup a block, the 64 x 64 product in LDS in FP64.
+// A gate mixes rows and leaves columns apart, so each wave keeps 16 columns to itself (lane: column
+// lane % 16, a quarter of the rows' groups by lane / 16) and updates them in place with no barrier
+// between gates. Bound by LDS traffic (each gate reads and writes the product). With a barrier and two
+// memory latencies a gate a run of the batch above took 2.35 ms, 1.19 ms so (group builds included).
 __global__ __launch_bounds__(256) void k_batch_build(const BBlock *__restrict__ blocks, uint32_t block0,
                                                      const BGate *__restrict__ gates,
                                                      const cx<double> *__restrict__ mats, bf16x8 *frags) {
-    __shared__ cx<double> m[2][4096];   // [row][column], row = tile row index (row bits)
+    // [row][column], row = tile row index (row bits), rows padded by one slot for the fragments' reads
+    __shared__ cx<double> m[64 * kBuildRow];
+    __shared__ GateStage stage;
     const BBlock bk = blocks[block0 + blockIdx.x];
     const uint32_t tid = threadIdx.x;
     for (uint32_t e = tid; e < 4096; e += 256) {
         cx<double> v;
         v.re = (e >> 6) == (e & 63) ? 1.0 : 0.0;
         v.im = 0.0;
-        m[0][e] = v;
+        m[(e >> 6) * kBuildRow + (e & 63)] = v;
     }
-    int cur = 0;
-    __syncthreads();
-    // Lane = column throughout, so rows, gate sub-indices and matrix entries are wave-uniform and
-    // come through the scalar cache. One- and two-qubit gates (the common case) update groups of
-    // rows in place with the matrix in registers; wider gates go out of place into the other
-    // buffer, one output row at a time.
-    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6), c = tid & 63;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6), part = (tid & 63u) >> 4;
+    const uint32_t c = wv * 16u + (tid & 15u);
     for (uint32_t g = 0; g < bk.ngates; ++g) {
-        const BGate gt = gates[bk.gate0 + g];
-        const cx<double> *G = mats + gt.mat;
-        const uint32_t msk = gt.mask;
-        if (gt.k == 1) {
+        const uint32_t slot = g % kGateChunk;
+        if (slot == 0) stage_gates(stage, gates + bk.gate0 + g, min(kGateChunk, bk.ngates - g), mats);
+        const uint32_t k = __builtin_amdgcn_readfirstlane(stage.gate[slot].k);
+        const uint32_t msk = __builtin_amdgcn_readfirstlane(stage.gate[slot].mask);
+        const cx<double> *G = stage.mat[slot];
+        if (k == 1) {
             const cx<double> g00 = G[0], g01 = G[1], g10 = G[2], g11 = G[3];
             const uint32_t lowm = msk - 1u;
 #pragma unroll
-            for (uint32_t q = 0; q < 8; ++q) {          // 32 row pairs, 8 per wave
-                const uint32_t j = wv + 4 * q;
+            for (uint32_t q = 0; q < 8; ++q) {          // 32 row pairs, 8 per lane
+                const uint32_t j = part + 4 * q;
                 const uint32_t r0 = ((j & ~lowm) << 1) | (j & lowm), r1 = r0 | msk;
-                const cx<double> x0 = m[cur][(r0 << 6) | c], x1 = m[cur][(r1 << 6) | c];
+                const cx<double> x0 = m[r0 * kBuildRow + c], x1 = m[r1 * kBuildRow + c];
                 cx<double> y0 = {0.0, 0.0}, y1 = {0.0, 0.0};
                 y0 = cmul_acc(cmul_acc(y0, g00, x0), g01, x1);
                 y1 = cmul_acc(cmul_acc(y1, g10, x0), g11, x1);
-                m[cur][(r0 << 6) | c] = y0;
-                m[cur][(r1 << 6) | c] = y1;
+                m[r0 * kBuildRow + c] = y0;
+                m[r1 * kBuildRow + c] = y1;
             }
-        } else if (gt.k == 2) {
+        } else if (k == 2) {
             cx<double> gm[16];
 #pragma unroll
             for (int t = 0; t < 16; ++t) gm[t] = G[t];
             const uint32_t mlo = msk & (0u - msk), mhi = msk ^ mlo;
 #pragma unroll
-            for (uint32_t q = 0; q < 4; ++q) {          // 16 row quads, 4 per wave
-                const uint32_t j = wv + 4 * q;
+            for (uint32_t q = 0; q < 4; ++q) {          // 16 row quads, 4 per lane
+                const uint32_t j = part + 4 * q;
                 uint32_t r = ((j & ~(mlo - 1u)) << 1) | (j & (mlo - 1u));
                 r = ((r & ~(mhi - 1u)) << 1) | (r & (mhi - 1u));
                 const uint32_t rows[4] = {r, r | mlo, r | mhi, r | mlo | mhi};
                 cx<double> x[4];
 #pragma unroll
-                for (int t = 0; t < 4; ++t) x[t] = m[cur][(rows[t] << 6) | c];
+                for (int t = 0; t < 4; ++t) x[t] = m[rows[t] * kBuildRow + c];
 #pragma unroll
                 for (int o = 0; o < 4; ++o) {
                     cx<double> y = {0.0, 0.0};
 #pragma unroll
                     for (int t = 0; t < 4; ++t) y = cmul_acc(y, gm[4 * o + t], x[t]);
-                    m[cur][(rows[o] << 6) | c] = y;
+                    m[rows[o] * kBuildRow + c] = y;
                 }
             }
         } else {
-            const uint32_t D = 1u << gt.k;
+            // a lane forms 16 rows of its column before any of the wave's lanes writes one
+            const uint32_t D = 1u << k;
+            const cx<double> *Gg = mats + __builtin_amdgcn_readfirstlane(stage.gate[slot].mat);
+            cx<double> y[16];
+#pragma unroll
             for (uint32_t i = 0; i < 16; ++i) {
-                const uint32_t r = wv + 4 * i;
+                const uint32_t r = part + 4 * i;
                 const uint32_t s = gather_bits(r, msk), rb = r & ~msk;
-                cx<double> y = {0.0, 0.0};
+                y[i].re = y[i].im = 0.0;
                 uint32_t d = 0;
                 for (uint32_t t = 0; t < D; ++t) {
-                    y = cmul_acc(y, G[s * D + t], m[cur][((rb | d) << 6) | c]);
+                    y[i] = cmul_acc(y[i], Gg[s * D + t], m[(rb | d) * kBuildRow + c]);
                     d = (d - msk) & msk;
                 }
-                m[cur ^ 1][(r << 6) | c] = y;
             }
-            cur ^= 1;
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (uint32_t i = 0; i < 16; ++i) m[(part + 4 * i) * kBuildRow + c] = y[i];
         }
-        __syncthreads();
+        // the next gate's rows are other lanes' of this wave: order its reads after these writes
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
+    __syncthreads();
     // split-BF16 A fragments, [wave][ks][hi/lo][lane] x 8
     bf16x8 *out = frags + (size_t)bk.frag * (kFragBytes / 16);
     for (uint32_t q = tid; q < 2048; q += 256) {
@@ -333,7 +392,7 @@ __global__ __launch_bounds__(256) void k_batch_build(const BBlock *__restrict__ 
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             const FragEntry fe = frag_entry(w, ks, lane, j);
-            const cx<double> u = m[cur][fe.rr * 64 + fe.cc];
+            const cx<double> u = m[fe.rr * kBuildRow + fe.cc];
             double val = fe.imag ? u.im : u.re;
             if (fe.negate) val = -val;
             const __bf16 h = (__bf16)(float)val;
@@ -364,6 +423,8 @@ __global__ __launch_bounds__(256, 2) void k_batch6(cx<float> *arena, const BBloc
                                                    const BChunk *__restrict__ chunks, uint32_t chunk0,
                                                    const bf16x8 *__restrict__ frags,
                                                    const double *__restrict__ scales, double *partials) {
+    // the renormalisation factor of the block: scales' where k_batch_scales has formed it (scales not
+    // null), else every wavefront sums the partials of the state's previous block itself, in one order
     __shared__ TileLds lds;
     __shared__ double red[4];
     const BChunk ch = chunks[chunk0 + blockIdx.x];
@@ -388,7 +449,9 @@ __global__ __launch_bounds__(256, 2) void k_batch6(cx<float> *arena, const BBloc
     ctx.ucol_out0 = u_of_col(lane & 31, a);
     ctx.ucol_out1 = u_of_col(32 + (lane & 31), a);
     ctx.urow_half = (lane >> 5) ? u_of_row(4, a) : 0u;
-    ctx.scale = scales[ch.block];
+    double pv[8];
+    const double *prev = partials + bk.prev_part;
+    if (!scales) partials_first(prev, bk.prev_count, lane, pv);
     const uint64_t off_t = u_offset<0, 9>(2u * (uint32_t)tid, a);
 
     // Same two-buffer pipeline as the single-state kernel, over this chunk's tiles; the last
@@ -398,6 +461,8 @@ __global__ __launch_bounds__(256, 2) void k_batch6(cx<float> *arena, const BBloc
     cx<float> va[16], vb[16];
     uint64_t tile = ch.tile0;
     load_tile(va, amps, tile_base(tile, a) + off_t, a);
+    if (scales) ctx.scale = scales[ch.block];
+    else ctx.scale = bk.prev_count ? renorm_factor(partials_sum(pv, prev, bk.prev_count, lane)) : 1.0;
     for (;;) {
         load_tile(vb, amps, tile_base(min(tile + 1, last), a) + off_t, a);
         process_tile(va, tile_base(tile, a) + off_t, amps, lds, ah, al, ctx, a, nacc);
@@ -520,7 +585,9 @@ struct Plan {
     std::vector<BChunk> chunks;
     std::vector<BFinish> finish;
     std::vector<uint32_t> wave_block0, wave_chunk0;   // size waves + 1
-    uint32_t max_wave_blocks = 0;
+    std::vector<uint32_t> group_wave0;                // first wave of each group of waves built together, size groups + 1
+    uint32_t max_wave_blocks = 0, max_group_blocks = 0;
+    uint32_t max_prev = 0;                            // most norm partials any block sums
     uint32_t nparts = 0;
     int64_t n_small = 0, n_tiled = 0;
     uint64_t algorithmic_bytes = 0;
@@ -582,10 +649,20 @@ int build_plan(const std::vector<int32_t> &ns, const std::vector<uint64_t> &offs
         for (int64_t g : per_state[i]) bgl[i][gate_block[g]].push_back(g);
     }
     std::vector<uint32_t> prev_part(count, 0), prev_count(count, 0);
+    uint32_t slot = 0;                                // fragment slot in the group
     for (size_t w = 0; w < waves; ++w) {
         p.wave_block0.push_back((uint32_t)p.blocks.size());
         p.wave_chunk0.push_back((uint32_t)p.chunks.size());
-        uint32_t slot = 0;
+        if (w == 0 || slot >= kBuildBlocks) {
+            p.group_wave0.push_back((uint32_t)w);
+            slot = 0;
+        }
+        const uint32_t wave_first = slot;
+        // shorter chunks where a wave has too few tiles for two workgroups on every CU
+        uint64_t wave_tiles = 0;
+        for (int32_t i : tiled)
+            if (w < bmask[i].size()) wave_tiles += 1ull << (ns[i] - kTileBits);
+        const uint64_t chunk = std::min<uint64_t>(t.chunk_tiles, std::max<uint64_t>(1, wave_tiles / kWaveChunks));
         for (int32_t i : tiled) {
             if (w >= bmask[i].size()) continue;
             const int n = ns[i];
@@ -606,6 +683,7 @@ int build_plan(const std::vector<int32_t> &ns, const std::vector<uint64_t> &offs
             bk.frag = slot++;
             bk.prev_part = prev_part[i];
             bk.prev_count = prev_count[i];
+            p.max_prev = std::max(p.max_prev, bk.prev_count);
             for (int64_t g : bgl[i][w]) {
                 BGate bg;
                 bg.mat = (uint32_t)mat_dev[g];
@@ -619,19 +697,21 @@ int build_plan(const std::vector<int32_t> &ns, const std::vector<uint64_t> &offs
             const uint64_t ntiles = bk.a.ntiles;
             prev_part[i] = p.nparts;
             prev_count[i] = 0;
-            for (uint64_t t0 = 0; t0 < ntiles; t0 += (uint64_t)t.chunk_tiles) {
+            for (uint64_t t0 = 0; t0 < ntiles; t0 += chunk) {
                 BChunk c;
                 c.block = bidx;
                 c.tile0 = (uint32_t)t0;
-                c.ntiles = (uint32_t)std::min<uint64_t>((uint64_t)t.chunk_tiles, ntiles - t0);
+                c.ntiles = (uint32_t)std::min<uint64_t>(chunk, ntiles - t0);
                 c.part = p.nparts++;
                 p.chunks.push_back(c);
                 ++prev_count[i];
             }
             p.algorithmic_bytes += 2 * 8 * (1ull << n);
         }
-        p.max_wave_blocks = std::max(p.max_wave_blocks, slot);
+        p.max_wave_blocks = std::max(p.max_wave_blocks, slot - wave_first);
+        p.max_group_blocks = std::max(p.max_group_blocks, slot);
     }
+    if (waves) p.group_wave0.push_back((uint32_t)waves);
     p.wave_block0.push_back((uint32_t)p.blocks.size());
     p.wave_chunk0.push_back((uint32_t)p.chunks.size());
     for (int32_t i : tiled) {
@@ -702,10 +782,10 @@ struct qipgpu_batch {
     cx<float> *arena = nullptr;
     uint64_t *d_offs = nullptr;
     hipStream_t stream = nullptr;   // waves, finish, resets, copies
-    hipStream_t side = nullptr;     // fragment builds, one wave ahead
+    hipStream_t side = nullptr;     // fragment builds, one group of waves ahead
     hipStream_t lds = nullptr;      // LDS states
     hipEvent_t fork = nullptr, join = nullptr;
-    std::vector<hipEvent_t> ev_built, ev_applied;   // per wave
+    std::vector<hipEvent_t> ev_built, ev_applied;   // per group of waves
     // loaded gates
     GateList gl;
     std::vector<uint64_t> mat_dev;      // per gate: offset in d_mats (complex units)
@@ -750,9 +830,9 @@ void free_plan(qipgpu_batch *b) {
 }
 
 // Enqueue one run of the plan. The run starts and ends on `stream`, which carries the tile passes,
-// the scale kernels and the finish. `side` builds wave w's fragments into set w % 2 once wave
-// w - 2's tile pass has released that set, one wave ahead of the tile passes; `lds` runs the LDS
-// states. Both join back into `stream` before the run ends.
+// the scale kernels and the finish. `side` builds the fragments of group g of waves into set g % 2 once
+// group g - 2's tile passes have released that set, one group ahead of the tile passes; `lds` runs the
+// LDS states. Both join back into `stream` before the run ends.
 int enqueue_run(qipgpu_batch *b) {
     const Plan &p = b->plan;
     const size_t waves = p.wave_block0.empty() ? 0 : p.wave_block0.size() - 1;
@@ -767,27 +847,32 @@ int enqueue_run(qipgpu_batch *b) {
         QIP_HIP(hipEventRecord(b->join, b->lds));
     }
     if (waves) QIP_HIP(hipStreamWaitEvent(b->side, b->fork, 0));
-    const size_t set = (size_t)p.max_wave_blocks * (kFragBytes / 16);
-    for (size_t w = 0; w < waves; ++w) {
-        const uint32_t nb = p.wave_block0[w + 1] - p.wave_block0[w];
-        const uint32_t nc = p.wave_chunk0[w + 1] - p.wave_chunk0[w];
-        bf16x8 *frags = b->d_frags + (w & 1) * set;
-        if (w >= 2) QIP_HIP(hipStreamWaitEvent(b->side, b->ev_applied[w - 2], 0));
-        hipLaunchKernelGGL(k_batch_build, dim3(nb), dim3(256), 0, b->side, (const BBlock *)b->d_blocks,
-                           p.wave_block0[w], (const BGate *)b->d_bgates, (const cx<double> *)b->d_mats, frags);
+    const size_t set = (size_t)p.max_group_blocks * (kFragBytes / 16);
+    const bool own = p.max_prev <= kMaxOwnPartials;
+    for (size_t g = 0; g + 1 < p.group_wave0.size(); ++g) {
+        const uint32_t w0 = p.group_wave0[g], w1 = p.group_wave0[g + 1];
+        bf16x8 *frags = b->d_frags + (g & 1) * set;
+        if (g >= 2) QIP_HIP(hipStreamWaitEvent(b->side, b->ev_applied[g - 2], 0));
+        hipLaunchKernelGGL(k_batch_build, dim3(p.wave_block0[w1] - p.wave_block0[w0]), dim3(256), 0, b->side,
+                           (const BBlock *)b->d_blocks, p.wave_block0[w0], (const BGate *)b->d_bgates,
+                           (const cx<double> *)b->d_mats, frags);
         QIP_LAUNCHED();
-        QIP_HIP(hipEventRecord(b->ev_built[w], b->side));
-        if (w > 0) {   // wave 0 blocks have no previous block: their factor stays 1
-            hipLaunchKernelGGL(k_batch_scales, dim3(nb), dim3(256), 0, b->stream, (const BBlock *)b->d_blocks,
-                               p.wave_block0[w], (const double *)b->d_partials, b->d_scales);
+        QIP_HIP(hipEventRecord(b->ev_built[g], b->side));
+        QIP_HIP(hipStreamWaitEvent(b->stream, b->ev_built[g], 0));
+        for (uint32_t w = w0; w < w1; ++w) {
+            const uint32_t nb = p.wave_block0[w + 1] - p.wave_block0[w];
+            const uint32_t nc = p.wave_chunk0[w + 1] - p.wave_chunk0[w];
+            if (!own && w > 0) {   // wave 0 blocks have no previous block: their factor stays 1
+                hipLaunchKernelGGL(k_batch_scales, dim3(nb), dim3(256), 0, b->stream, (const BBlock *)b->d_blocks,
+                                   p.wave_block0[w], (const double *)b->d_partials, b->d_scales);
+                QIP_LAUNCHED();
+            }
+            hipLaunchKernelGGL(k_batch6, dim3(nc), dim3(256), 0, b->stream, b->arena, (const BBlock *)b->d_blocks,
+                               (const BChunk *)b->d_chunks, p.wave_chunk0[w], (const bf16x8 *)frags,
+                               own ? (const double *)nullptr : (const double *)b->d_scales, b->d_partials);
             QIP_LAUNCHED();
         }
-        QIP_HIP(hipStreamWaitEvent(b->stream, b->ev_built[w], 0));
-        hipLaunchKernelGGL(k_batch6, dim3(nc), dim3(256), 0, b->stream, b->arena, (const BBlock *)b->d_blocks,
-                           (const BChunk *)b->d_chunks, p.wave_chunk0[w], (const bf16x8 *)frags,
-                           (const double *)b->d_scales, b->d_partials);
-        QIP_LAUNCHED();
-        QIP_HIP(hipEventRecord(b->ev_applied[w], b->stream));
+        QIP_HIP(hipEventRecord(b->ev_applied[g], b->stream));
     }
     if (!p.finish.empty()) {
         hipLaunchKernelGGL(k_batch_finish, dim3((uint32_t)p.finish.size()), dim3(256), 0, b->stream, b->arena,
@@ -824,19 +909,18 @@ int make_plan(qipgpu_batch *b, const Tuning &t) {
     if ((rc = upload(b->plan_mem, zeros, &b->d_partials))) return rc;
     std::vector<double> ones(std::max<size_t>(p.blocks.size(), 1), 1.0);
     if ((rc = upload(b->plan_mem, ones, &b->d_scales))) return rc;
-    const size_t waves = p.wave_block0.empty() ? 0 : p.wave_block0.size() - 1;
-    for (size_t w = 0; w < waves; ++w) {
+    for (size_t g = 0; g + 1 < p.group_wave0.size(); ++g) {
         hipEvent_t e1 = nullptr, e2 = nullptr;
         QIP_HIP(hipEventCreateWithFlags(&e1, hipEventDisableTiming));
         b->ev_built.push_back(e1);
         QIP_HIP(hipEventCreateWithFlags(&e2, hipEventDisableTiming));
         b->ev_applied.push_back(e2);
     }
-    if (p.max_wave_blocks) {   // two alternating fragment sets
+    if (p.max_group_blocks) {   // two alternating fragment sets
         void *f = nullptr;
-        if (hipMalloc(&f, 2 * kFragBytes * (size_t)p.max_wave_blocks) != hipSuccess) {
+        if (hipMalloc(&f, 2 * kFragBytes * (size_t)p.max_group_blocks) != hipSuccess) {
             (void)hipGetLastError();
-            return set_error(QIPGPU_ENOMEM, "batch plan: fragment buffer of %u blocks", p.max_wave_blocks);
+            return set_error(QIPGPU_ENOMEM, "batch plan: fragment buffer of %u blocks", p.max_group_blocks);
         }
         b->plan_mem.push_back(f);
         b->d_frags = (bf16x8 *)f;

@@ -19,30 +19,6 @@ namespace {
 
 constexpr int kFusedBlocksPerCU = 2;   // 69 KB of LDS and 212 VGPRs per workgroup
 
-// Sum `count` FP64 partials with one wavefront: lane l adds partials l, l + 64, ... in order, then a
-// butterfly over the lanes. Each butterfly step adds the same two values on both lanes of a pair, so
-// every lane, every wavefront and every workgroup that sums the same partials gets the same bits.
-// The first 512 partials are loaded up front (partials_first) so a caller can issue other loads
-// before the sum waits for these; partials_sum adds any beyond 512 and reduces.
-__device__ __forceinline__ void partials_first(const double *__restrict__ partial, uint32_t count, int lane,
-                                               double (&pv)[8]) {
-    // unconditional loads (index clamped into the array, which holds at least one partial), so
-    // none of them waits for another; partials_sum drops the clamped ones
-    const uint32_t last = count ? count - 1 : 0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) pv[j] = partial[min((uint32_t)lane + 64u * j, last)];
-}
-
-__device__ __forceinline__ double partials_sum(const double (&pv)[8], const double *__restrict__ partial,
-                                               uint32_t count, int lane) {
-    double acc = 0.0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc += (uint32_t)lane + 64u * j < count ? pv[j] : 0.0;
-    for (uint32_t i = (uint32_t)lane + 512u; i < count; i += 64) acc += partial[i];
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    return acc;
-}
-
 // One fused block. Every amplitude is scaled as it is loaded by 1/sqrt(norm of the previous block's
 // output): each workgroup sums the previous block's `prev_count` partials itself (the same sum in all
 // of them; prev_count = 0 means no pending factor), so a block is one launch with no cross-workgroup
