@@ -10,7 +10,7 @@
 //   k_dense_mfma<R, K>   K = 4..6, in place. Each wave forms Y = U X for 1024 amplitudes at a time with
 //                        three real products on FP64 MFMA (v_mfma_f64_16x16x4f64), U's fragments in
 //                        LDS. It holds every amplitude of its bases before any is written, so in place
-//                        is safe.
+//                        is safe. Small states take k_dense_split, a tile by four waves.
 //   k_dense_gemm<R>      K = 7..12, out of place: a 64 x 64 output tile per workgroup over 16-column
 //                        steps of j through LDS, into a compact [D][nbase] buffer; k_dense_scatter
 //                        writes it back to the bases' positions.
@@ -206,6 +206,54 @@ __global__ __launch_bounds__(kTileThreads, 2) void k_dense_mfma(const DenseTileA
         process(xb, t1);
         if (t2 >= end) return;
         t = t2;
+    }
+}
+
+// The same tile by the four waves of a workgroup, one 16 x 16 block of outputs each, for states with at most
+// kSplitTiles tiles: a wave that works a tile alone has a chain of up to 192 MFMAs (5 us), and fewer
+// tiles than the GPU has places for waves leave most of it idle. A wave's fragments come straight from
+// memory, all its loads at once; a barrier keeps the columns' loads ahead of the stores. 6 targets on
+// 2^17 amplitudes: 24.4 us a call with the kernel above, 20.2 so (most of both is staging U); at 2^20 they meet.
+constexpr uint64_t kSplitTiles = 512;
+
+template <typename R, int K>
+__global__ __launch_bounds__(kTileThreads) void k_dense_split(const DenseTileArgs<R, K> a,
+                                                              const f64x2 *__restrict__ frag) {
+    using M = MfmaShape<K>;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int rb = wave % M::RB, col = wave / M::RB;
+    const int kap = lane >> 4;
+    f64x2 u[M::KS];
+#pragma unroll
+    for (int s = 0; s < M::KS; ++s) u[s] = frag[(s * M::RB + rb) * 64 + lane];
+    const uint64_t g = (uint64_t)blockIdx.x * M::BASES + 16 * col + (lane & 15);
+    cx<R> *p = a.amps + insert_zeros(g & (a.nbase - 1), a.pl) +
+               (kap & 2 ? (kap & 1 ? a.row_k[3] : a.row_k[2]) : (kap & 1 ? a.row_k[1] : a.row_k[0]));
+    cx<R> x[M::KS];
+#pragma unroll
+    for (int s = 0; s < M::KS; ++s) x[s] = p[a.row_s[s]];
+    f64x4 acc[3];
+#pragma unroll
+    for (int m = 0; m < 3; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int s = 0; s < M::KS; ++s) {
+        const cx<double> v = to_d(x[s]);
+        acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s][0], v.re, acc[0], 0, 0, 0);
+        acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s][1], v.im, acc[1], 0, 0, 0);
+        acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s][0] + u[s][1], v.re + v.im, acc[2], 0, 0, 0);
+    }
+    __syncthreads();   // every wave of the tile holds its columns' amplitudes
+    if (g >= a.nbase) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        cx<double> y;
+        y.re = acc[0][i] - acc[1][i];
+        y.im = acc[2][i] - acc[0][i] - acc[1][i];
+        // row 16 rb + 4 i + kap: k-step 4 rb + i
+        uint64_t off = 0;
+#pragma unroll
+        for (int r = 0; r < M::RB; ++r) off = rb == r ? a.row_s[4 * r + i] : off;
+        p[off] = from_d<R>(y);
     }
 }
 
@@ -469,6 +517,12 @@ int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
     void *d = nullptr;
     int rc = ring_upload(s, frag.data(), frag.size() * sizeof(frag[0]), &d);
     if (rc) return rc;
+    if (a.ntiles <= kSplitTiles) {
+        hipLaunchKernelGGL((k_dense_split<R, K>), dim3((uint32_t)a.ntiles), dim3(kTileThreads), 0, s->stream, a,
+                           (const f64x2 *)d);
+        QIP_LAUNCHED();
+        return QIPGPU_OK;
+    }
     const uint64_t grid = std::min<uint64_t>((a.ntiles + kTileWaves - 1) / kTileWaves, (uint64_t)device_cus() * 2);
     hipLaunchKernelGGL((k_dense_mfma<R, K>), dim3((uint32_t)grid), dim3(kTileThreads), 0, s->stream, a,
                        (const f64x2 *)d);

@@ -1,5 +1,5 @@
 """Dense operators on 4 to 6 targets (marked gpu) at the edges of a wave's tile: fewer bases than one
-tile holds, exactly one, one more than a workgroup's waves take, and several ranges; targets low, high
+tile holds, exactly one, the largest number of tiles that workgroups share and more than that (20 qubits); targets low, high
 and scattered in an order of their own, with and without controls; against the oracle. Bars as for the
 rest of the operator domain: 1e-12 (complex128), 2e-6 of the largest amplitude (complex64)."""
 import numpy
@@ -18,7 +18,7 @@ def unitary(rng, d):
 
 @pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
 @pytest.mark.parametrize("k", [4, 5, 6])
-@pytest.mark.parametrize("extra", [0, 1, 3, 4, 6, 8, 11])
+@pytest.mark.parametrize("extra", [0, 1, 3, 4, 6, 8, 11, 15])
 def test_tiles_of_every_size_against_the_oracle(k, extra, dtype):
     n = k + extra
     rng = numpy.random.default_rng(100 * k + extra)
