@@ -353,7 +353,8 @@ def bench_grover24(args):
             res[name]["product_pass"] = product_pass_roofline(be, ns, amp)
         else:
             res[name]["note"] = ("the same H/X/MCZ iteration on Fused128Backend: each run of H and X layers "
-                                 "is one product of per-qubit 2x2s (3 product passes instead of 6)")
+                                 "is one product of per-qubit 2x2s, and the two share a pass with the MCZ (5 "
+                                 "product passes)")
         be.close()
     cfg = {"workload": "24-qubit iterative Grover: 23 search qubits + |-> ancilla, F(x==x*) oracle, {} iterations, "
                        "seeded measurement".format(t_iter), "n_qubits": ns + 1, "iterations": t_iter,
@@ -377,13 +378,15 @@ def product_pass_roofline(be, ns: int, amp: int):
     targets, mats = list(range(ns)), [H] * ns
     ev = HipEvents()
     be.flush() if hasattr(be, "flush") else None
-    GpuBackend.apply_product(be, targets, mats)        # launched directly, also on a recording backend
-    GpuBackend.apply_product(be, targets, mats)
+    for _ in range(2):
+        GpuBackend.apply_product(be, targets, mats)    # not recorded, also on a recording backend
+        be.flush()                                     # a product is held back for the next one
     be.synchronize()
     a, b = ev.create(), ev.create()
     ev.record(a, be.stream)
     for _ in range(10):
         GpuBackend.apply_product(be, targets, mats)
+        be.flush()
     ev.record(b, be.stream)
     passes = 10 * -(-(ns - 3) // 8)
     ms = ev.elapsed_ms(a, b) / passes
@@ -398,9 +401,10 @@ def grover_iteration_bytes(ns: int, amp: int, diffusion: str):
     """(algorithmic, touched) HBM bytes of one Grover iteration on ns search qubits + 1 ancilla.
     Algorithmic, per descriptor as the reference sweeps it: read + write of every amplitude a
     descriptor can change (2 S 2^n; the 22-controlled Z changes 2^2), plus the 4 B x 2^ns f table per
-    func_apply. Touched, what the kernels here move: each H or X layer on 23 qubits is three product
-    passes over the whole state (every pass keeps the four lowest state bits in its tile), func_apply
-    reads the table and swaps only the pairs where f(x) = 1 (one, for these oracles)."""
+    func_apply. Touched, what the kernels here move: an H layer on 23 qubits is three product passes over
+    the whole state (every pass keeps the four lowest state bits in its tile); X layers are multiplied into
+    the H layers beside them, and the two layers around the controlled Z share a pass, which applies it
+    too. func_apply reads the table and swaps only the pairs where f(x) = 1 (one, for these oracles)."""
     n = ns + 1
     sweep = 2 * amp * 2 ** n
     table = 4 * 2 ** ns
@@ -409,7 +413,7 @@ def grover_iteration_bytes(ns: int, amp: int, diffusion: str):
     mcz = 2 * amp * 2 ** (n - (ns - 1)) if diffusion == "mcz" else 0
     algorithmic = funcs * (sweep + table) + layers * sweep + mcz
     passes = -(-(ns - 3) // 8)                        # three low qubits ride in the first pass
-    touched = funcs * (table + 2 * 2 * amp) + layers * passes * sweep + mcz
+    touched = funcs * (table + 2 * 2 * amp) + (2 * passes - (1 if diffusion == "mcz" else 0)) * sweep
     return algorithmic, touched
 
 
@@ -817,6 +821,7 @@ def bench_product24(args):
                 ev.record(a, be.stream)
                 for _ in range(reps):
                     be.apply_product(targets, ms_)
+                    be.flush()                         # a product is held back for the next one
                 ev.record(b, be.stream)
                 ms = ev.elapsed_ms(a, b) / reps
                 gbs = 2 * amp * 2 ** n / ms / 1e6

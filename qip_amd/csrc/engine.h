@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <cstdarg>
 #include <cstdint>
 #include <complex>
@@ -68,6 +69,14 @@ struct HeldGate {
     uint8_t k;          // entries of tpos
     uint8_t tpos[2];
 };
+// Single-qubit operators on distinct state bits held back as one operator (product.hip): factor m[p] on
+// state bit p, for every bit of `bits`.
+struct HeldProduct {
+    uint64_t bits = 0;
+    std::vector<std::array<cx<double>, 4>> m;   // row-major 2x2 per state bit
+};
+// Diagonals that may stand between two held products (k_product_pair's arguments).
+constexpr size_t kBetweenMax = 4;
 // Gates held back at most: with this many, the next pass is applied. Enough for a pass to see the
 // two-qubit gates that follow a layer of single-qubit gates on 30 qubits.
 constexpr size_t kHeldMax = 64;
@@ -125,8 +134,12 @@ struct qipgpu_state {
     hipGraphNode_t rec_last = nullptr;
     // gates recorded for online fusion and not launched yet (complex64 states)
     qipgpu::Recorder *recorder = nullptr;
-    // gates held back, in program order (flush_held applies them before anything else touches the state)
+    // held back, in program order: a product, gates, a product (flush_held applies them before anything
+    // else touches the state). Gates held behind `before` are diagonals, at most kBetweenMax; `after` is
+    // held only behind both.
+    qipgpu::HeldProduct before;
     std::vector<qipgpu::HeldGate> held;
+    qipgpu::HeldProduct after;
 };
 
 namespace qipgpu {
@@ -181,15 +194,22 @@ int check_qubits(const qipgpu_state *s, int32_t k, const int32_t *q, const char 
 int ring_upload(qipgpu_state *s, const void *src, size_t bytes, void **dev);
 // Hold a small gate back on the state; with kHeldMax held, the next pass of them is applied (runs.hip).
 int hold_gate(qipgpu_state *s, const HeldGate &g);
-// Apply the gates held back on the state (runs.hip): every entry point that touches the state does so
-// first, through flush_recorded.
+// Apply what is held back on the state (runs.hip): every entry point that touches the state does so
+// first, through flush_recorded. drop_held forgets it (the state is overwritten).
 int flush_held(qipgpu_state *s);
+void drop_held(qipgpu_state *s);
+// The gates of s->held alone, in passes (runs.hip).
+int apply_held_gates(qipgpu_state *s);
+// s->before, s->held and s->after, where a product is held (product.hip).
+int apply_held_products(qipgpu_state *s);
 // One held gate by a sweep of its own; up to kDiagChainMax diagonals, in order, by one sweep over the
 // amplitudes that share the controls all of them have (engine.hip).
 int launch_held_gate(qipgpu_state *s, const HeldGate &g);
 int launch_diag_chain(qipgpu_state *s, const HeldGate *g, int count);
-// Apply the held-back gates, then launch every recorded gate (recorder.hip); the recorded gates are
-// left alone while the recorder itself is launching.
+// Launch every recorded gate (recorder.hip), after what is held back; they may themselves be held back.
+// Nothing while the recorder itself is launching.
+int launch_recorded(qipgpu_state *s);
+// launch_recorded, then apply what is held back.
 int flush_recorded(qipgpu_state *s);
 // While s is capturing: mark the capture refused and return QIPGPU_EUNSUP naming `what`.
 int refuse_in_capture(qipgpu_state *s, const char *what);

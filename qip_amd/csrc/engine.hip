@@ -481,7 +481,7 @@ int qipgpu_capture_end(qipgpu_state *s, qipgpu_graph **out) {
     if (!s->capturing) return set_error(QIPGPU_EINVAL, "the state is not capturing");
     // gates still held back belong to the recording: their node goes last
     if (!s->capture_refused && flush_held(s) != QIPGPU_OK) s->capture_refused = true;
-    s->held.clear();
+    drop_held(s);
     s->capturing = false;
     hipGraph_t g = s->rec_graph;
     s->rec_graph = nullptr;
@@ -564,7 +564,7 @@ int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_
     QIP_NOT_CAPTURING(s, "a state initialisation");
     // every amplitude is rewritten, so recorded and held-back gates and the factor are moot
     s->fused_prev_count = 0;
-    s->held.clear();
+    drop_held(s);
     recorder_discard(s);
     if (n_groups < 0) return set_error(QIPGPU_EINVAL, "negative group count");
     uint64_t fed = 0;
@@ -1127,9 +1127,8 @@ int qipgpu_apply_matrix(qipgpu_state *s, int32_t k, const int32_t *targets, cons
     int rc = check_disjoint(s, k, targets, n_ctrl, controls);
     if (rc) return rc;
     // linear in the state: a pending fused renormalisation (a scalar) stays pending; recorded gates
-    // go first (with the gates held back before them); held-back gates otherwise stay held, and
-    // dispatch applies them before anything that is not held
-    rc = recorder_pending(s) ? flush_recorded(s) : QIPGPU_OK;
+    // go first; what is held back stays held, and dispatch applies it before anything that is not held
+    rc = launch_recorded(s);
     if (rc) return rc;
     Analysed an = analyse(k, targets, mat);
     std::vector<int32_t> ctl(controls, controls + n_ctrl);
@@ -1142,7 +1141,7 @@ int qipgpu_apply_diagonal(qipgpu_state *s, int32_t k, const int32_t *targets, co
     int rc = check_disjoint(s, k, targets, n_ctrl, controls);
     if (rc) return rc;
     // as in qipgpu_apply_matrix
-    rc = recorder_pending(s) ? flush_recorded(s) : QIPGPU_OK;
+    rc = launch_recorded(s);
     if (rc) return rc;
     Analysed an;
     an.targets.assign(targets, targets + k);

@@ -27,7 +27,10 @@
 // per CU, which do not cover the barrier-separated phases (on a 24-qubit complex64 pass over all
 // three layouts, LDS is busy about an eighth of the time and the FP64 units about a third).
 #include <algorithm>
+#include <array>
+#include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <vector>
 
 #include "engine.h"
@@ -102,14 +105,15 @@ __device__ __forceinline__ cx<double> mac2(cx<double> m0, cx<double> x0, cx<doub
     return r;
 }
 
-// The factors on u bits B..B+3 applied to 16 registers whose index e is u bits B..B+3.
+// The factors g[B..B+3] of the u bits B..B+3 that are in fmask (real matrices: rmask) applied to 16
+// registers whose index e is those bits.
 template <int B>
-__device__ __forceinline__ void apply4(cx<double> (&x)[16], const ProductArgs &a) {
+__device__ __forceinline__ void apply4(cx<double> (&x)[16], uint32_t fmask, uint32_t rmask, const cx<double> (*g)[4]) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        if (!((a.fmask >> (B + j)) & 1u)) continue;
-        const cx<double> m00 = a.g[B + j][0], m01 = a.g[B + j][1], m10 = a.g[B + j][2], m11 = a.g[B + j][3];
-        if ((a.rmask >> (B + j)) & 1u) {   // real matrix: half the arithmetic
+        if (!((fmask >> (B + j)) & 1u)) continue;
+        const cx<double> m00 = g[B + j][0], m01 = g[B + j][1], m10 = g[B + j][2], m11 = g[B + j][3];
+        if ((rmask >> (B + j)) & 1u) {   // real matrix: half the arithmetic
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 if ((e >> j) & 1) continue;
@@ -131,6 +135,11 @@ __device__ __forceinline__ void apply4(cx<double> (&x)[16], const ProductArgs &a
             x[f] = mac2(m10, x0, m11, x1);
         }
     }
+}
+
+template <int B>
+__device__ __forceinline__ void apply4(cx<double> (&x)[16], const ProductArgs &a) {
+    apply4<B>(x, a.fmask, a.rmask, a.g);
 }
 
 template <typename R>
@@ -251,62 +260,139 @@ int launch_product(qipgpu_state *s, const ProductArgs &a) {
     return launch_gate(s, &k_product<R, kLds>, dim3(grid), dim3(256), (cx<R> *)s->amps, a);
 }
 
+// A product, diagonals and a second product on the same bits of one tile, in one pass: what a search's
+// diffusion holds between its passes over the other bits (H on every qubit, a phase, H on every qubit).
+// All factors sit on u bits 4..11: those on 8..11 are applied as loaded (A), those on 4..7 after a move
+// through LDS (B), the diagonals where the first product ends, and the way back. kLds = false: factors
+// on u bits 8..11 only.
+// Bound: HBM, as any product pass; it takes the place of two of them and of the diagonal's launch. 40
+// iterations of a search on 23 of 24 qubits with their start and reads, complex128: 96.3 ms with a pass
+// per 8 high bits of every layer (12 an iteration), 74.0 with 5; 80 iterations in complex64 84.2 -> 80.0.
+struct PairArgs {
+    ProductArgs p;                     // the first product (no X factor: xmask = 0)
+    uint32_t fmask2, rmask2;           // the second, on the same u bits
+    cx<double> g2[12][4];
+    uint32_t ndiag;
+    struct {
+        uint64_t ctrl, outer;          // state bits that have to be 1, and those of them outside the tile
+        cx<double> m[4];
+        uint32_t k;
+        uint32_t tpos[2];
+    } d[kBetweenMax];
+};
+static_assert(sizeof(PairArgs) <= 4000, "kernel arguments");
+
+// The diagonals, in FP64, on registers at tile base + off + u_offset<LO, LO + 4>(e << LO).
+template <int LO>
+__device__ __forceinline__ void diagonals(cx<double> (&x)[16], uint64_t tbase, uint64_t off, const PairArgs &a) {
+    for (uint32_t q = 0; q < a.ndiag; ++q) {
+        const uint64_t ctrl = a.d[q].ctrl, outer = a.d[q].outer;
+        if ((tbase & outer) != outer) continue;      // the same for the whole tile
+        const uint32_t k = a.d[q].k;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const uint64_t i = tbase + off + u_offset<LO, LO + 4>((uint32_t)e << LO, a.p);
+            if ((i & ctrl) != ctrl) continue;
+            uint32_t j = 0;
+            for (uint32_t b = 0; b < k; ++b) j = (j << 1) | (uint32_t)((i >> a.d[q].tpos[b]) & 1ull);
+            const cx<double> m = a.d[q].m[j], v = x[e];
+            x[e].re = m.re * v.re - m.im * v.im;
+            x[e].im = m.re * v.im + m.im * v.re;
+        }
+    }
+}
+
+template <typename R, bool kLds>
+__device__ __forceinline__ void pair_loop(cx<R> *amps, const PairArgs &a, TileStore *lds) {
+    const uint32_t tid = threadIdx.x;
+    const uint64_t off_a = u_offset<0, 8>(tid, a.p);
+    const uint64_t off_b = u_offset<0, 12>((tid & 15u) | (tid >> 4) << 8, a.p);
+    const uint64_t per = (a.p.ntiles + gridDim.x - 1) / gridDim.x;
+    uint64_t tile = (uint64_t)blockIdx.x * per;
+    const uint64_t end = min(tile + per, a.p.ntiles);
+    if (tile >= end) return;   // the same for every thread of the workgroup
+    const uint64_t last = end - 1;
+    cx<R> v[16];
+    load_raw(v, amps, tile_base(tile, a.p) + off_a, a.p);
+    for (;; ++tile) {
+        cx<double> x[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            x[i].re = (double)v[i].re;
+            x[i].im = (double)v[i].im;
+        }
+        const uint64_t tbase = tile_base(tile, a.p);
+        load_raw(v, amps, tile_base(min(tile + 1, last), a.p) + off_a, a.p);
+        apply4<8>(x, a.p);
+        if constexpr (kLds) {
+            // slots as in product_tile; a thread's A slots are read by itself alone at the end of a tile,
+            // so the next tile's writes there need no barrier
+            const auto ta = lds->at((int)(tid + (tid >> 4)));
+            const auto tb = lds->at((int)((tid & 15u) + 272u * (tid >> 4)));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) ta.put(272 * i, x[i]);
+            __syncthreads();
+#pragma unroll
+            for (int e = 0; e < 16; ++e) x[e] = tb.get(17 * e);
+            apply4<4>(x, a.p);
+            diagonals<4>(x, tbase, off_b, a);
+            apply4<4>(x, a.fmask2, a.rmask2, a.g2);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) tb.put(17 * e, x[e]);   // the slots this thread read
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) x[i] = ta.get(272 * i);
+        } else {
+            diagonals<8>(x, tbase, off_a, a);
+        }
+        apply4<8>(x, a.fmask2, a.rmask2, a.g2);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) amps[tbase + off_a + u_offset<8, 12>(256u * (uint32_t)i, a.p)] = narrow<R>(x[i]);
+        if (tile == last) return;
+    }
+}
+
+template <typename R, bool kLds>
+__global__ __launch_bounds__(256, 2) void k_product_pair(cx<R> *amps, PairArgs a) {
+    if constexpr (kLds) {
+        __shared__ TileStore t;
+        pair_loop<R, true>(amps, a, &t);
+    } else {
+        pair_loop<R, false>(amps, a, nullptr);
+    }
+}
+
+template <typename R>
+int launch_pair(qipgpu_state *s, const PairArgs &a) {
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(a.p.ntiles, (uint64_t)device_cus() * 2);
+    if (a.p.fmask & 0xf0u) return launch_gate(s, &k_product_pair<R, true>, dim3(grid), dim3(256), (cx<R> *)s->amps, a);
+    return launch_gate(s, &k_product_pair<R, false>, dim3(grid), dim3(256), (cx<R> *)s->amps, a);
+}
+
 constexpr int kLowBits = kProductLowBits;           // state bits every pass keeps in its tile
 constexpr int kHighPerPass = kProductHighPerPass;   // = kTileBits - kLowBits
 static_assert(kLowBits + kHighPerPass == kTileBits, "a pass tile holds 12 state bits");
 
-// One pass: the k single-qubit gates (k <= 12, all targets of at most kHighPerPass above the low
-// bits) in one sweep.
-int product_pass(qipgpu_state *s, int32_t k, const int32_t *targets, const double *mats) {
-    const int n = s->n;
-    uint64_t tmask = 0;
-    std::vector<int> tbits(k);
-    for (int j = 0; j < k; ++j) {
-        tbits[j] = n - 1 - targets[j];
-        tmask |= 1ull << tbits[j];
-    }
-    auto is_x = [&](int j) {
-        const double *m = mats + 8 * j;
-        return m[0] == 0.0 && m[1] == 0.0 && m[2] == 1.0 && m[3] == 0.0 && m[4] == 1.0 && m[5] == 0.0 &&
-               m[6] == 0.0 && m[7] == 0.0;
-    };
-    // u bits 0..3 are state bits 0..3, which every pass keeps. The targets above them go on u bits
-    // 4..11 by kind: a factor that needs arithmetic takes the register bits 8..11 of layout A first
-    // (applied without a transpose), then 6, 7, 4, 5; an X takes the lane bits 4, 5 first, then
-    // 8..11, and 6, 7 last (flipped at the store everywhere; on 6, 7 at the cost of a barrier). The
-    // free u bits take the lowest free state bits.
-    int ubit[kTileBits];
-    std::fill(ubit, ubit + kTileBits, -1);
-    for (int b = 0; b < kLowBits; ++b) ubit[b] = b;
-    std::vector<int> place(k, -1);
-    for (int j = 0; j < k; ++j)
-        if (tbits[j] < kLowBits) place[j] = tbits[j];
-    auto take = [&](int j, std::initializer_list<int> order) {
-        for (int u : order)
-            if (ubit[u] < 0) {
-                ubit[u] = tbits[j];
-                place[j] = u;
-                return;
-            }
-    };
-    for (int j = 0; j < k; ++j)
-        if (place[j] < 0 && !is_x(j)) take(j, {8, 9, 10, 11});
-    for (int j = 0; j < k; ++j)
-        if (place[j] < 0 && is_x(j)) take(j, {4, 5, 8, 9, 10, 11});
-    for (int j = 0; j < k; ++j)
-        if (place[j] < 0) take(j, {6, 7, 4, 5});
-    // at most kHighPerPass = 8 targets above the low bits share the 8 u bits 4..11: after the
-    // rounds above every one has a place (arithmetic overflow finds 8..11 full and 4..7 free enough,
-    // X overflow finds only 6, 7 free)
-    for (int j = 0; j < k; ++j)
-        if (place[j] < 0) return set_error(QIPGPU_EINVAL, "product pass: target %d has no tile bit", targets[j]);
+typedef std::array<cx<double>, 4> Factor;           // row-major 2x2
+
+bool is_x(const Factor &m) {
+    return m[0].re == 0.0 && m[0].im == 0.0 && m[1].re == 1.0 && m[1].im == 0.0 && m[2].re == 1.0 && m[2].im == 0.0 &&
+           m[3].re == 0.0 && m[3].im == 0.0;
+}
+
+bool is_real(const Factor &m) { return m[0].im == 0.0 && m[1].im == 0.0 && m[2].im == 0.0 && m[3].im == 0.0; }
+
+// The tile of a pass on `n` state bits: ubit[u] = the state bit placed on tile bit u, or -1 where the lowest
+// state bits of none take their place.
+void set_tile(ProductArgs &a, int n, int (&ubit)[kTileBits]) {
+    uint64_t placed = 0;
+    for (int u = 0; u < kTileBits; ++u)
+        if (ubit[u] >= 0) placed |= 1ull << ubit[u];
     for (int b = kLowBits, u = kLowBits; u < kTileBits; ++u) {
         if (ubit[u] >= 0) continue;
-        while (tmask >> b & 1) ++b;
+        while (placed >> b & 1) ++b;
         ubit[u] = b++;
     }
-    ProductArgs a;
-    std::memset(&a, 0, sizeof(a));
     a.ntiles = 1ull << (n - kTileBits);
     std::vector<int> sorted(ubit, ubit + kTileBits);
     std::sort(sorted.begin(), sorted.end());
@@ -314,21 +400,55 @@ int product_pass(qipgpu_state *s, int32_t k, const int32_t *targets, const doubl
         a.pbits[i] = (uint8_t)ubit[i];
         a.zbits[i] = (uint8_t)sorted[i];
     }
+}
+
+// One pass: the factors on the listed state bits (at most kHighPerPass of them above the low bits).
+int product_pass(qipgpu_state *s, const std::vector<int> &tbits, const HeldProduct &h) {
+    // u bits 0..3 are state bits 0..3, which every pass keeps. The targets above them go on u bits
+    // 4..11 by kind: a factor that needs arithmetic takes the register bits 8..11 of layout A first
+    // (applied without a transpose), then 6, 7, 4, 5; an X takes the lane bits 4, 5 first, then
+    // 8..11, and 6, 7 last (flipped at the store everywhere; on 6, 7 at the cost of a barrier). The
+    // free u bits take the lowest free state bits.
+    const size_t k = tbits.size();
+    int ubit[kTileBits];
+    std::fill(ubit, ubit + kTileBits, -1);
+    for (int b = 0; b < kLowBits; ++b) ubit[b] = b;
+    std::vector<int> place(k, -1);
+    for (size_t j = 0; j < k; ++j)
+        if (tbits[j] < kLowBits) place[j] = tbits[j];
+    auto take = [&](size_t j, std::initializer_list<int> order) {
+        for (int u : order)
+            if (ubit[u] < 0) {
+                ubit[u] = tbits[j];
+                place[j] = u;
+                return;
+            }
+    };
+    for (size_t j = 0; j < k; ++j)
+        if (place[j] < 0 && !is_x(h.m[tbits[j]])) take(j, {8, 9, 10, 11});
+    for (size_t j = 0; j < k; ++j)
+        if (place[j] < 0 && is_x(h.m[tbits[j]])) take(j, {4, 5, 8, 9, 10, 11});
+    for (size_t j = 0; j < k; ++j)
+        if (place[j] < 0) take(j, {6, 7, 4, 5});
+    // at most kHighPerPass = 8 targets above the low bits share the 8 u bits 4..11: after the
+    // rounds above every one has a place (arithmetic overflow finds 8..11 full and 4..7 free enough,
+    // X overflow finds only 6, 7 free)
+    for (size_t j = 0; j < k; ++j)
+        if (place[j] < 0) return set_error(QIPGPU_EINVAL, "product pass: state bit %d has no tile bit", tbits[j]);
+    ProductArgs a;
+    std::memset(&a, 0, sizeof(a));
+    set_tile(a, s->n, ubit);
     // each factor's kind by its matrix (the comment at ProductArgs)
-    for (int j = 0; j < k; ++j) {
+    for (size_t j = 0; j < k; ++j) {
         const int ub = place[j];
-        const double *m = mats + 8 * j;
-        const bool real = m[1] == 0.0 && m[3] == 0.0 && m[5] == 0.0 && m[7] == 0.0;
-        if (is_x(j)) {
+        const Factor &m = h.m[tbits[j]];
+        if (is_x(m)) {
             a.xmask |= 1u << ub;
             continue;
         }
         a.fmask |= 1u << ub;
-        if (real) a.rmask |= 1u << ub;
-        for (int e = 0; e < 4; ++e) {
-            a.g[ub][e].re = m[2 * e];
-            a.g[ub][e].im = m[2 * e + 1];
-        }
+        if (is_real(m)) a.rmask |= 1u << ub;
+        std::copy(m.begin(), m.end(), a.g[ub]);
     }
     const bool lds = (a.fmask & 0xffu) != 0;   // a factor below u bit 8 needs a transpose
     a.xsync = !lds && (a.xmask & 0xc0u) != 0;
@@ -336,7 +456,132 @@ int product_pass(qipgpu_state *s, int32_t k, const int32_t *targets, const doubl
     return lds ? launch_product<float, true>(s, a) : launch_product<float, false>(s, a);
 }
 
+std::vector<int> bits_of(uint64_t mask) {
+    std::vector<int> out;
+    for (int p = 0; p < 64; ++p)
+        if (mask >> p & 1) out.push_back(p);
+    return out;
+}
+
+// The passes of the factors on the state bits `bits`: they commute, so the first pass takes every factor on the
+// low bits and up to kHighPerPass others, each further pass up to kHighPerPass more (highest bits
+// first, the order in which a register's qubits come).
+int product_passes(qipgpu_state *s, const HeldProduct &h, uint64_t bits) {
+    const uint64_t low = (1ull << kLowBits) - 1;
+    std::vector<int> pick = bits_of(bits & low), high = bits_of(bits & ~low);
+    std::reverse(high.begin(), high.end());
+    for (size_t next = 0; !pick.empty() || next < high.size(); pick.clear()) {
+        for (int c = 0; c < kHighPerPass && next < high.size(); ++c) pick.push_back(high[next++]);
+        const int rc = product_pass(s, pick, h);
+        if (rc) return rc;
+    }
+    return QIPGPU_OK;
+}
+
+// The state bits whose factors of both products go into one pass with the diagonals between, or 0. With
+// the same high bits under both, the last pass of the first and the first of the second are one:
+// hb high bits then take 2 ceil(hb / kHighPerPass) - 1 passes. A factor that is exactly X has its store
+// for itself (product_pass) and stays out of this.
+uint64_t shared_bits(const HeldProduct &b, const HeldProduct &a) {
+    const uint64_t low = (1ull << kLowBits) - 1;
+    if (b.bits != a.bits || !(b.bits & ~low)) return 0;
+    const std::vector<int> high = bits_of(b.bits & ~low);
+    const size_t rest = high.size() % kHighPerPass, count = rest ? rest : (size_t)kHighPerPass;
+    if (count == high.size() && (b.bits & low)) return 0;    // the low bits' pass takes them along
+    uint64_t out = 0;
+    size_t got = 0;
+    for (int p : high) {
+        if (got == count) break;
+        if (is_x(b.m[p]) || is_x(a.m[p])) continue;
+        out |= 1ull << p;
+        ++got;
+    }
+    return got == count ? out : 0;
+}
+
+int pair_pass(qipgpu_state *s, const HeldProduct &b, const std::vector<HeldGate> &between, const HeldProduct &after,
+              uint64_t bits) {
+    static const int order[kHighPerPass] = {8, 9, 10, 11, 6, 7, 4, 5};
+    int ubit[kTileBits];
+    std::fill(ubit, ubit + kTileBits, -1);
+    for (int p = 0; p < kLowBits; ++p) ubit[p] = p;
+    PairArgs a;
+    std::memset(&a, 0, sizeof(a));
+    int next = 0;
+    for (int p : bits_of(bits)) {
+        const int u = order[next++];
+        ubit[u] = p;
+        a.p.fmask |= 1u << u;
+        if (is_real(b.m[p])) a.p.rmask |= 1u << u;
+        if (is_real(after.m[p])) a.rmask2 |= 1u << u;
+        std::copy(b.m[p].begin(), b.m[p].end(), a.p.g[u]);
+        std::copy(after.m[p].begin(), after.m[p].end(), a.g2[u]);
+    }
+    a.fmask2 = a.p.fmask;
+    set_tile(a.p, s->n, ubit);
+    uint64_t tile = 0;
+    for (int p : ubit) tile |= 1ull << p;
+    for (const HeldGate &g : between) {
+        auto &d = a.d[a.ndiag++];
+        d.ctrl = g.ctrl_mask;
+        d.outer = g.ctrl_mask & ~tile;
+        d.k = g.k;
+        for (int i = 0; i < g.k; ++i) d.tpos[i] = g.tpos[i];
+        std::copy(g.m, g.m + 4, d.m);
+    }
+    return s->dtype == QIPGPU_C128 ? launch_pair<double>(s, a) : launch_pair<float>(s, a);
+}
+
+bool finite(const HeldProduct &h) {
+    for (int p : bits_of(h.bits))
+        for (const cx<double> &e : h.m[p])
+            if (!std::isfinite(e.re) || !std::isfinite(e.im)) return false;
+    return true;
+}
+
+// h := f on state bit p after what h has there, in FP64 (exact where either is a permutation). Two X cancel.
+void compose(HeldProduct &h, int p, const Factor &f) {
+    if (!(h.bits >> p & 1)) {
+        h.bits |= 1ull << p;
+        h.m[p] = f;
+        return;
+    }
+    const Factor g = h.m[p];
+    if (is_x(f) && is_x(g)) {
+        h.bits &= ~(1ull << p);
+        return;
+    }
+    for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j) {
+            const cx<double> a = f[2 * i], b = f[2 * i + 1], c = g[j], d = g[2 + j];
+            h.m[p][2 * i + j].re = a.re * c.re - a.im * c.im + b.re * d.re - b.im * d.im;
+            h.m[p][2 * i + j].im = a.re * c.im + a.im * c.re + b.re * d.im + b.im * d.re;
+        }
+}
+
 }  // namespace
+
+namespace qipgpu {
+
+int apply_held_products(qipgpu_state *s) {
+    HeldProduct before, after;
+    std::vector<HeldGate> between;
+    std::swap(before, s->before);
+    std::swap(after, s->after);
+    std::swap(between, s->held);
+    const uint64_t both = shared_bits(before, after);
+    int rc = product_passes(s, before, before.bits & ~both);
+    if (rc) return rc;
+    if (both) {
+        rc = pair_pass(s, before, between, after, both);
+    } else {
+        s->held = between;
+        rc = apply_held_gates(s);
+    }
+    return rc ? rc : product_passes(s, after, after.bits & ~both);
+}
+
+}  // namespace qipgpu
 
 extern "C" int qipgpu_apply_product(qipgpu_state *s, int32_t k, const int32_t *targets, const double *mats) {
     if (k < 1 || k > QIPGPU_MAX_PRODUCT) return set_error(QIPGPU_EINVAL, "product of %d single-qubit gates (1..%d)", k,
@@ -346,26 +591,30 @@ extern "C" int qipgpu_apply_product(qipgpu_state *s, int32_t k, const int32_t *t
     if (rc) return rc;
     // linear in the state: a pending fused renormalisation (a scalar) stays pending; recorded gates
     // go first
-    rc = flush_recorded(s);
+    rc = launch_recorded(s);
     if (rc) return rc;
-    // the factors commute: the first pass takes every factor on the low bits and up to
-    // kHighPerPass others, each further pass up to kHighPerPass more
-    std::vector<int> low, high;
-    for (int j = 0; j < k; ++j) (s->n - 1 - targets[j] < kLowBits ? low : high).push_back(j);
-    size_t next = 0;
-    bool first = true;
-    while (first || next < high.size()) {
-        std::vector<int> pick(first ? low : std::vector<int>());
-        for (int c = 0; c < kHighPerPass && next < high.size(); ++c) pick.push_back(high[next++]);
-        first = false;
-        if (pick.empty()) continue;
-        std::vector<int32_t> t;
-        std::vector<double> m;
-        for (int j : pick) {
-            t.push_back(targets[j]);
-            m.insert(m.end(), mats + 8 * j, mats + 8 * j + 8);
+    // The product is held back: one that follows it at once is multiplied into it (its factors, 2x2 in
+    // FP64), one that follows after diagonals may share a pass with it (shared_bits). On 23 of 24
+    // qubits an H layer, an X layer, a controlled Z, an X layer and an H layer are 5 passes, 12 when
+    // each layer had its own. An infinity or a NaN in a factor would spread through such products, so
+    // factors that hold one meet the state by themselves.
+    HeldProduct f;
+    f.m.resize(s->n);
+    for (int j = 0; j < k; ++j) {
+        const int p = s->n - 1 - targets[j];
+        f.bits |= 1ull << p;
+        for (int e = 0; e < 4; ++e) {
+            f.m[p][e].re = mats[8 * j + 2 * e];
+            f.m[p][e].im = mats[8 * j + 2 * e + 1];
         }
-        if ((rc = product_pass(s, (int32_t)t.size(), t.data(), m.data()))) return rc;
     }
+    const bool plain = finite(f);
+    if (s->after.bits ? !plain || !finite(s->after) : !s->held.empty() && (!s->before.bits || !plain)) {
+        if ((rc = flush_held(s))) return rc;
+    }
+    if (s->before.bits && s->held.empty() && (!plain || !finite(s->before)) && (rc = flush_held(s))) return rc;
+    HeldProduct &h = s->before.bits && !s->held.empty() ? s->after : s->before;
+    if (!h.bits) h.m.assign(s->n, Factor());
+    for (int p : bits_of(f.bits)) compose(h, p, f.m[p]);
     return QIPGPU_OK;
 }

@@ -383,17 +383,18 @@ void simulate_recorder(int32_t n, int32_t width, bool streaming, bool use_launch
 
 }  // namespace
 
-int flush_recorded(qipgpu_state *s) {
-    int rc = flush_held(s);   // held-back gates came first
-    if (rc) return rc;
+int launch_recorded(qipgpu_state *s) {
     Recorder *r = s->recorder;
     if (!r || r->in_flush || r->k.empty()) return QIPGPU_OK;
     std::vector<PlannedBlock> blocks;
     plan_recorded(*r, false, blocks);
     r->since_plan = 0;
-    rc = launch_planned(s, blocks, (int64_t)blocks.size());
-    if (rc) return rc;
-    return flush_held(s);     // a complex128 block that is diagonal is held like any such gate
+    return launch_planned(s, blocks, (int64_t)blocks.size());
+}
+
+int flush_recorded(qipgpu_state *s) {
+    const int rc = launch_recorded(s);
+    return rc ? rc : flush_held(s);
 }
 
 void recorder_discard(qipgpu_state *s) {
@@ -429,9 +430,7 @@ int qipgpu_fused_set_recording(qipgpu_state *s, int32_t width, int32_t streaming
 int qipgpu_fused_record(qipgpu_state *s, int32_t n_gates, const int32_t *gate_k, const int32_t *gate_qubits,
                         const double *mats) {
     QIP_NOT_CAPTURING(s, "gate recording for fusion");
-    int rc = flush_held(s);   // gates held back come before what is recorded now
-    if (rc) return rc;
-    rc = ensure_recorder(s);
+    int rc = ensure_recorder(s);   // what is held back comes before what is recorded now
     if (rc) return rc;
     if (n_gates < 0) return set_error(QIPGPU_EINVAL, "negative gate count");
     if (n_gates > 0 && (!gate_k || !gate_qubits || !mats)) return set_error(QIPGPU_EINVAL, "null argument");

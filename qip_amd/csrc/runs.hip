@@ -713,16 +713,29 @@ int apply_next(qipgpu_state *s) {
 namespace qipgpu {
 
 int hold_gate(qipgpu_state *s, const HeldGate &g) {
+    // behind a held product only diagonals wait, for a second product that may share a pass with both
+    if (s->before.bits &&
+        (s->after.bits || g.kind != HeldGate::kDiagonal || s->held.size() == kBetweenMax)) {
+        const int rc = apply_held_products(s);
+        if (rc) return rc;
+    }
     s->held.push_back(g);
     return s->held.size() < kHeldMax ? QIPGPU_OK : apply_next(s);
 }
 
-int flush_held(qipgpu_state *s) {
+int apply_held_gates(qipgpu_state *s) {
     while (!s->held.empty()) {
         const int rc = apply_next(s);
         if (rc) return rc;
     }
     return QIPGPU_OK;
+}
+
+int flush_held(qipgpu_state *s) { return s->before.bits ? apply_held_products(s) : apply_held_gates(s); }
+
+void drop_held(qipgpu_state *s) {
+    s->before.bits = s->after.bits = 0;
+    s->held.clear();
 }
 
 }  // namespace qipgpu
