@@ -62,6 +62,11 @@ int qipgpu_info(const qipgpu_state *s, int32_t *n, int32_t *dtype);
  * complex128 entries of each feed. */
 int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_len,
                         const int32_t *group_idx, const double *feeds);
+/* The same with each feed by its own address, feeds[g]; real[g] != 0 (real may be null: none) marks one
+ * that is 2^len_g real numbers. The feeds are read before the call returns; the state is written in
+ * the order of its queue. */
+int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_len, const int32_t *group_idx,
+                      const double *const *feeds, const int32_t *real);
 
 /* Copies of amplitude windows [start, end) in the state's own dtype:
  *   get:  get_state / get_relative_range   (qip/backend.py:106-107,168-169)

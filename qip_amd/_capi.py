@@ -34,6 +34,7 @@ SIGNATURES = {
     "qipgpu_destroy": (ctypes.c_int, [_P]),
     "qipgpu_info": (ctypes.c_int, [_P, _PI32, _PI32]),
     "qipgpu_init_product": (ctypes.c_int, [_P, _I32, _P, _P, _P]),
+    "qipgpu_init_feeds": (ctypes.c_int, [_P, _I32, _P, _P, _PP, _P]),
     "qipgpu_get_range": (ctypes.c_int, [_P, _I64, _I64, _P]),
     "qipgpu_set_range": (ctypes.c_int, [_P, _I64, _I64, _P]),
     "qipgpu_add_range": (ctypes.c_int, [_P, _I64, _I64, _P]),

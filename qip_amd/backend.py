@@ -338,10 +338,13 @@ class GpuBackend(StateType):
         if len(feed_list) == 0:
             _capi.check(self._lib.qipgpu_init_product(self._h, 0, None, None, None), "init")
             return
-        groups = [list(g) for g in index_groups]
+        groups = [list(g) for g in index_groups][:len(feed_list)]
         feeds = []
         for g, f in zip(groups, feed_list):
-            v = numpy.asarray(f).astype(numpy.complex128).ravel()
+            # real feeds cross the link as real numbers (half the bytes) and are widened on the device
+            v = numpy.asarray(f)
+            real = v.dtype.kind in "fiub"
+            v = numpy.ascontiguousarray(v, dtype=numpy.float64 if real else numpy.complex128).ravel()
             if v.shape[0] < 2 ** len(g):
                 raise IndexError("feed of length {} for {} qubits".format(v.shape[0], len(g)))
             feeds.append(v[: 2 ** len(g)])
@@ -351,9 +354,10 @@ class GpuBackend(StateType):
             return
         glen = _capi.i32([len(g) for g in groups])
         gidx = _capi.i32([q for g in groups for q in g])
-        flat = numpy.ascontiguousarray(numpy.concatenate(feeds)).view(numpy.float64)
-        _capi.check(self._lib.qipgpu_init_product(self._h, len(groups), _capi.ptr(glen), _capi.ptr(gidx),
-                                                  _capi.ptr(flat)), "init")
+        at = (ctypes.c_void_p * len(feeds))(*[v.ctypes.data for v in feeds])
+        kinds = _capi.i32([v.dtype == numpy.float64 for v in feeds])
+        _capi.check(self._lib.qipgpu_init_feeds(self._h, len(groups), _capi.ptr(glen), _capi.ptr(gidx), at,
+                                                _capi.ptr(kinds)), "init")
 
     def reinit(self, index_groups: Sequence[Sequence[int]] = (), feed_list: Sequence[InitialState] = ()) -> None:
         """Rewrite the state in place as make_state would build it (no reallocation)."""

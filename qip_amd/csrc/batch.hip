@@ -1218,10 +1218,7 @@ int qipgpu_batch_get_state(qipgpu_batch *b, int32_t i, void *out) {
     if (i < 0 || i >= b->count) return set_error(QIPGPU_EINVAL, "state %d outside 0..%d", i, b->count - 1);
     int rc = sync_streams(b);
     if (rc) return rc;
-    QIP_HIP(hipMemcpyAsync(out, b->arena + b->offs[i], sizeof(cx<float>) << b->ns[i], hipMemcpyDeviceToHost,
-                           b->stream));
-    QIP_HIP(hipStreamSynchronize(b->stream));
-    return QIPGPU_OK;
+    return copy_to_host(b->stream, out, b->arena + b->offs[i], sizeof(cx<float>) << b->ns[i]);
 }
 
 int qipgpu_batch_set_state(qipgpu_batch *b, int32_t i, const void *in) {
@@ -1229,9 +1226,9 @@ int qipgpu_batch_set_state(qipgpu_batch *b, int32_t i, const void *in) {
     if (i < 0 || i >= b->count) return set_error(QIPGPU_EINVAL, "state %d outside 0..%d", i, b->count - 1);
     int rc = sync_streams(b);
     if (rc) return rc;
-    QIP_HIP(hipMemcpyAsync(b->arena + b->offs[i], in, sizeof(cx<float>) << b->ns[i], hipMemcpyHostToDevice,
-                           b->stream));
-    QIP_HIP(hipStreamSynchronize(b->stream));
+    rc = copy_to_device(b->stream, b->arena + b->offs[i], in, sizeof(cx<float>) << b->ns[i]);
+    if (rc) return rc;
+    QIP_HIP(hipStreamSynchronize(b->stream));   // the batch's other queues may run next
     return QIPGPU_OK;
 }
 

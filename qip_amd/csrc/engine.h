@@ -186,6 +186,11 @@ struct TempBuffer {
 
 // Make sure s->scratch holds at least `bytes`.
 int ensure_scratch(qipgpu_state *s, size_t bytes);
+// Copies between the caller's memory and the current device's through pinned staging memory (transfer.hip),
+// in `st`'s order: to the host, complete on return; to the device, enqueued, the host memory free on
+// return.
+int copy_to_host(hipStream_t st, void *host, const void *dev, size_t bytes);
+int copy_to_device(hipStream_t st, void *dev, const void *host, size_t bytes);
 // Compute units of the current device, queried once per device (persistent grids are sized by it).
 int device_cus();
 // Validate a list of qubit indices against n (range, distinctness); returns QIPGPU_OK or EINVAL.

@@ -294,6 +294,24 @@ __global__ __launch_bounds__(256) void k_init_chunked(cx<R> *amps, InitArgs a, i
     }
 }
 
+// |0...0>: 16 B words of zeros, the first of them `first`.
+__global__ __launch_bounds__(256) void k_init_basis(uint4 *amps, uint64_t words, uint4 first) {
+    const uint64_t stride = (uint64_t)gridDim.x * 256;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < words; i += stride)
+        amps[i] = i ? make_uint4(0, 0, 0, 0) : first;
+}
+
+// A feed given as real numbers.
+__global__ __launch_bounds__(256) void k_widen_feed(const double *__restrict__ in, cx<double> *__restrict__ out, uint64_t count) {
+    const uint64_t stride = (uint64_t)gridDim.x * 256;
+    for (uint64_t i = (uint64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += stride) {
+        cx<double> v;
+        v.re = in[i];
+        v.im = 0.0;
+        out[i] = v;
+    }
+}
+
 template <typename R>
 __global__ __launch_bounds__(256) void k_init_product(cx<R> *amps, InitArgs a) {
 #pragma clang fp contract(off)
@@ -358,36 +376,47 @@ namespace {
 // Amplitude buffers and queues of destroyed small states, kept for the next state of the same size on
 // the same device: creating a state then costs no allocation, and a state made again after another
 // was destroyed gets the same buffer, so gate graphs captured on the first replay on the second. At
-// most kPoolEntries buffers of up to kPoolMaxBytes each are held (2 GiB), until the process ends.
+// most kPoolEntries buffers of up to kPoolMaxBytes each are held (2 GiB), until the process ends. The
+// state's scratch goes along while it is small: a run that reads probabilities allocates nothing then.
 struct PoolEntry {
     int device;
     size_t bytes;
     void *amps;
     hipStream_t stream;
+    void *scratch;          // up to kPoolScratch bytes
+    size_t scratch_cap;
 };
+constexpr size_t kPoolScratch = size_t(16) << 20;
 constexpr size_t kPoolMaxBytes = size_t(256) << 20;
 constexpr size_t kPoolEntries = 8;
 std::mutex g_pool_mu;
 std::vector<PoolEntry> g_pool;
 
 // the most recently given buffer of the size first
-bool pool_take(int device, size_t bytes, void **amps, hipStream_t *stream) {
+bool pool_take(qipgpu_state *s) {
+    const size_t bytes = s->len * s->amp_bytes;
     std::lock_guard<std::mutex> lock(g_pool_mu);
     for (size_t i = g_pool.size(); i-- > 0;)
-        if (g_pool[i].device == device && g_pool[i].bytes == bytes) {
-            *amps = g_pool[i].amps;
-            *stream = g_pool[i].stream;
+        if (g_pool[i].device == s->device && g_pool[i].bytes == bytes) {
+            s->amps = g_pool[i].amps;
+            s->stream = g_pool[i].stream;
+            s->scratch = g_pool[i].scratch;
+            s->scratch_cap = g_pool[i].scratch_cap;
             g_pool.erase(g_pool.begin() + (long)i);
             return true;
         }
     return false;
 }
 
-bool pool_give(int device, size_t bytes, void *amps, hipStream_t stream) {
+bool pool_give(qipgpu_state *s) {
+    const size_t bytes = s->len * s->amp_bytes;
     if (bytes > kPoolMaxBytes) return false;
     std::lock_guard<std::mutex> lock(g_pool_mu);
     if (g_pool.size() >= kPoolEntries) return false;
-    g_pool.push_back(PoolEntry{device, bytes, amps, stream});
+    const bool small = s->scratch_cap <= kPoolScratch;
+    g_pool.push_back(PoolEntry{s->device, bytes, s->amps, s->stream, small ? s->scratch : nullptr,
+                               small ? s->scratch_cap : 0});
+    if (small) s->scratch = nullptr;
     return true;
 }
 
@@ -408,7 +437,7 @@ int qipgpu_create(int32_t n, int32_t dtype, qipgpu_state **out) {
         delete s;
         return set_error(QIPGPU_EHIP, "hipGetDevice failed");
     }
-    if (pool_take(s->device, s->len * s->amp_bytes, &s->amps, &s->stream)) {
+    if (pool_take(s)) {
         *out = s;
         return QIPGPU_OK;
     }
@@ -431,7 +460,7 @@ int qipgpu_destroy(qipgpu_state *s) {
     if (!s) return QIPGPU_OK;
     if (s->rec_graph) (void)hipGraphDestroy(s->rec_graph);   // an unfinished recording is dropped
     (void)hipStreamSynchronize(s->stream);
-    const bool pooled = s->amps && pool_give(s->device, s->len * s->amp_bytes, s->amps, s->stream);
+    const bool pooled = s->amps && pool_give(s);
     if (s->amps && !pooled) (void)hipFree(s->amps);
     if (s->scratch) (void)hipFree(s->scratch);
     if (s->d_ring) (void)hipFree(s->d_ring);
@@ -562,6 +591,19 @@ int qipgpu_get_stream(qipgpu_state *s, void **stream) {
 int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_len,
                         const int32_t *group_idx, const double *feeds) {
     QIP_NOT_CAPTURING(s, "a state initialisation");
+    if (n_groups < 0) return set_error(QIPGPU_EINVAL, "negative group count");
+    std::vector<const double *> each(n_groups);
+    for (int g = 0; g < n_groups; ++g) {
+        if (group_len[g] < 1 || group_len[g] > s->n) return set_error(QIPGPU_EINVAL, "bad feed group length %d", group_len[g]);
+        each[g] = feeds;
+        feeds += 2ull << group_len[g];
+    }
+    return qipgpu_init_feeds(s, n_groups, group_len, group_idx, each.data(), nullptr);
+}
+
+int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_len, const int32_t *group_idx,
+                      const double *const *feeds, const int32_t *real) {
+    QIP_NOT_CAPTURING(s, "a state initialisation");
     // every amplitude is rewritten, so recorded and held-back gates and the factor are moot
     s->fused_prev_count = 0;
     drop_held(s);
@@ -583,15 +625,15 @@ int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_
     }
     if (n_groups == 0) {
         // |0...0> (qip/backend.py:90-91)
-        QIP_HIP(hipMemsetAsync(s->amps, 0, s->len * s->amp_bytes, s->stream));
-        if (s->dtype == QIPGPU_C128) {
-            const double one[2] = {1.0, 0.0};
-            QIP_HIP(hipMemcpyAsync(s->amps, one, sizeof(one), hipMemcpyHostToDevice, s->stream));
-        } else {
-            const float one[2] = {1.0f, 0.0f};
-            QIP_HIP(hipMemcpyAsync(s->amps, one, sizeof(one), hipMemcpyHostToDevice, s->stream));
-        }
-        QIP_HIP(hipStreamSynchronize(s->stream));
+        const uint64_t words = s->len * s->amp_bytes / sizeof(uint4);
+        const uint32_t nb = capped_grid(blocks_for(words, 256));
+        const double d = 1.0;
+        const float f = 1.0f;
+        uint4 first = make_uint4(0, 0, 0, 0);
+        if (s->dtype == QIPGPU_C128) std::memcpy(&first, &d, sizeof(d));
+        else std::memcpy(&first, &f, sizeof(f));
+        hipLaunchKernelGGL(k_init_basis, dim3(nb), dim3(256), 0, s->stream, (uint4 *)s->amps, words, first);
+        QIP_LAUNCHED();
         return QIPGPU_OK;
     }
     // device copies of the descriptor: [glen | gpos | pad | goff | feeds]
@@ -600,16 +642,31 @@ int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_
     const size_t b_glen = sizeof(int32_t) * n_groups, b_gpos = sizeof(int32_t) * total_idx;
     const size_t o_goff = ((b_glen + b_gpos + 15) / 16) * 16;
     const size_t o_feed = o_goff + ((sizeof(int64_t) * n_groups + 15) / 16) * 16;
-    const size_t bytes = o_feed + sizeof(double) * 2 * total_feed;
-    int rc = ensure_scratch(s, bytes);
+    // a real feed crosses the link as it is, behind the feeds, and is widened on the device
+    const size_t o_real = o_feed + sizeof(double) * 2 * total_feed;
+    size_t real_bytes = 0;
+    for (int g = 0; g < n_groups; ++g)
+        if (real && real[g]) real_bytes = std::max(real_bytes, sizeof(double) << group_len[g]);
+    int rc = ensure_scratch(s, o_real + real_bytes);
     if (rc) return rc;
     char *d = static_cast<char *>(s->scratch);
-    std::vector<char> h(bytes);
+    std::vector<char> h(o_feed);
     std::memcpy(h.data(), group_len, b_glen);
     std::memcpy(h.data() + b_glen, gpos.data(), b_gpos);
     std::memcpy(h.data() + o_goff, goff.data(), sizeof(int64_t) * n_groups);
-    std::memcpy(h.data() + o_feed, feeds, sizeof(double) * 2 * total_feed);
-    QIP_HIP(hipMemcpyAsync(d, h.data(), bytes, hipMemcpyHostToDevice, s->stream));
+    if ((rc = copy_to_device(s->stream, d, h.data(), o_feed))) return rc;
+    for (int g = 0; g < n_groups; ++g) {
+        const uint64_t count = 1ull << group_len[g];
+        cx<double> *to = reinterpret_cast<cx<double> *>(d + o_feed) + goff[g];
+        const bool widen = real && real[g];
+        rc = copy_to_device(s->stream, widen ? (void *)(d + o_real) : (void *)to, feeds[g],
+                            (widen ? sizeof(double) : sizeof(cx<double>)) * count);
+        if (rc) return rc;
+        if (!widen) continue;
+        hipLaunchKernelGGL(k_widen_feed, dim3(std::min<uint32_t>(blocks_for(count, 256), 1u << 16)), dim3(256), 0, s->stream,
+                           (const double *)(d + o_real), to, count);
+        QIP_LAUNCHED();
+    }
     InitArgs a;
     a.len = s->len;
     a.unfed_mask = (s->len - 1) & ~fed;
@@ -646,7 +703,6 @@ int qipgpu_init_product(qipgpu_state *s, int32_t n_groups, const int32_t *group_
             hipLaunchKernelGGL(k_init_product<float>, dim3(nb), dim3(256), 0, s->stream, (cx<float> *)s->amps, a);
     }
     QIP_LAUNCHED();
-    QIP_HIP(hipStreamSynchronize(s->stream));  // host descriptor buffer goes out of scope
     return QIPGPU_OK;
 }
 
@@ -665,10 +721,8 @@ int qipgpu_get_range(qipgpu_state *s, int64_t start, int64_t end, void *host) {
     rc = settle(s);
     if (rc) return rc;
     // on the state's own queue, not the legacy one, which would wait for every blocking queue
-    QIP_HIP(hipMemcpyAsync(host, static_cast<char *>(s->amps) + start * s->amp_bytes, (end - start) * s->amp_bytes,
-                           hipMemcpyDeviceToHost, s->stream));
-    QIP_HIP(hipStreamSynchronize(s->stream));
-    return QIPGPU_OK;
+    return copy_to_host(s->stream, host, static_cast<char *>(s->amps) + start * s->amp_bytes,
+                        (end - start) * s->amp_bytes);
 }
 
 int qipgpu_set_range(qipgpu_state *s, int64_t start, int64_t end, const void *host) {
@@ -678,10 +732,8 @@ int qipgpu_set_range(qipgpu_state *s, int64_t start, int64_t end, const void *ho
     if (end == start) return QIPGPU_OK;
     rc = settle(s);
     if (rc) return rc;
-    QIP_HIP(hipMemcpyAsync(static_cast<char *>(s->amps) + start * s->amp_bytes, host, (end - start) * s->amp_bytes,
-                           hipMemcpyHostToDevice, s->stream));
-    QIP_HIP(hipStreamSynchronize(s->stream));   // the host data is read before return
-    return QIPGPU_OK;
+    return copy_to_device(s->stream, static_cast<char *>(s->amps) + start * s->amp_bytes, host,
+                          (end - start) * s->amp_bytes);
 }
 
 int qipgpu_add_range(qipgpu_state *s, int64_t start, int64_t end, const void *host) {
@@ -694,7 +746,8 @@ int qipgpu_add_range(qipgpu_state *s, int64_t start, int64_t end, const void *ho
     if (rc) return rc;
     rc = ensure_scratch(s, count * s->amp_bytes);
     if (rc) return rc;
-    QIP_HIP(hipMemcpyAsync(s->scratch, host, count * s->amp_bytes, hipMemcpyHostToDevice, s->stream));
+    rc = copy_to_device(s->stream, s->scratch, host, count * s->amp_bytes);
+    if (rc) return rc;
     const uint32_t nb = std::min<uint32_t>(blocks_for(count, 256), 1u << 20);
     if (s->dtype == QIPGPU_C128)
         hipLaunchKernelGGL(k_add_range<double>, dim3(nb), dim3(256), 0, s->stream,
@@ -703,7 +756,6 @@ int qipgpu_add_range(qipgpu_state *s, int64_t start, int64_t end, const void *ho
         hipLaunchKernelGGL(k_add_range<float>, dim3(nb), dim3(256), 0, s->stream, (cx<float> *)s->amps + start,
                            (const cx<float> *)s->scratch, count);
     QIP_LAUNCHED();
-    QIP_HIP(hipStreamSynchronize(s->stream));
     return QIPGPU_OK;
 }
 
@@ -1878,9 +1930,7 @@ static int marginals_host(qipgpu_state *s, int32_t k, const int32_t *indices, Or
                           uint64_t m_count, double *out) {
     int rc = marginals_dev(s, k, indices, order, m_lo, m_count, 0);
     if (rc) return rc;
-    QIP_HIP(hipMemcpyAsync(out, s->scratch, sizeof(double) * m_count, hipMemcpyDeviceToHost, s->stream));
-    QIP_HIP(hipStreamSynchronize(s->stream));
-    return QIPGPU_OK;
+    return copy_to_host(s->stream, out, s->scratch, sizeof(double) * m_count);
 }
 
 }  // namespace
@@ -2049,9 +2099,7 @@ int qipgpu_total_prob(qipgpu_state *s, double *out) {
     if (rc) return rc;
     rc = norm_to_device(s, static_cast<double *>(s->scratch));
     if (rc) return rc;
-    QIP_HIP(hipMemcpyAsync(out, s->scratch, sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    QIP_HIP(hipStreamSynchronize(s->stream));
-    return QIPGPU_OK;
+    return copy_to_host(s->stream, out, s->scratch, sizeof(double));
 }
 
 int qipgpu_probabilities(qipgpu_state *s, int32_t k, const int32_t *indices, double *out) {
@@ -2119,9 +2167,8 @@ int qipgpu_top_probabilities(qipgpu_state *s, int32_t k, const int32_t *indices,
         len = blocks * T;
     }
     std::vector<uint64_t> idx(T);
-    QIP_HIP(hipMemcpyAsync(ps, vin, sizeof(double) * T, hipMemcpyDeviceToHost, s->stream));
-    QIP_HIP(hipMemcpyAsync(idx.data(), iin, sizeof(uint64_t) * T, hipMemcpyDeviceToHost, s->stream));
-    QIP_HIP(hipStreamSynchronize(s->stream));
+    if ((rc = copy_to_host(s->stream, ps, vin, sizeof(double) * T))) return rc;
+    if ((rc = copy_to_host(s->stream, idx.data(), iin, sizeof(uint64_t) * T))) return rc;
     for (uint32_t i = 0; i < T; ++i) ms[i] = (int64_t)idx[i];
     return QIPGPU_OK;
 }
