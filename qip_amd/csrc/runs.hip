@@ -1,8 +1,9 @@
 // runs.hip -- small gates held back on a state and applied in runs, one pass over the state per run.
 //
 // Held gates are single-qubit operators (any 2x2 under any controls), two-qubit swaps and diagonals on
-// at most two targets. A pass cuts the state into tiles of 4096 amplitudes: 12 tile bits, state bits
-// 0..3 among them (runs of 256 B for complex128), so up to 8 others. Only a bit that a gate changes
+// at most two targets. A pass cuts the state into tiles: of 4096 amplitudes on large states (12 tile bits,
+// state bits 0..3 among them for runs of 256 B of complex128, so up to 8 others), of 1024 on small ones
+// (10 tile bits with bits 0 and 1 among them, again 8 others). Only a bit that a gate changes
 // has to be a tile bit: a diagonal multiplies an amplitude by a factor that its index decides, and a
 // control only decides whether an amplitude takes part, so their bits may lie anywhere. A tile is read
 // once, every gate of the run is applied to it in order, and it is written once.
@@ -24,9 +25,20 @@ using namespace qipgpu;
 
 namespace {
 
-constexpr int kTileBits = 12;
-constexpr int kLowBits = 4;                        // state bits 0..3, in every tile
-constexpr int kHighBits = kTileBits - kLowBits;
+constexpr int kMaxTileBits = 12;
+
+// How a kernel cuts the state: its tiles, the lowest state bits that are in every one, and the register
+// bits of a thread's amplitudes. In layout l the registers hold tile bits
+// [tile_bits - reg_bits (l + 1), tile_bits - reg_bits l).
+struct Shape {
+    int tile_bits, low_bits, reg_bits;
+    int high_bits() const { return tile_bits - low_bits; }
+    int layouts() const { return tile_bits / reg_bits; }
+    int first_reg(int layout) const { return tile_bits - reg_bits * (layout + 1); }
+    int layout_of(int u) const { return layouts() - 1 - u / reg_bits; }
+};
+constexpr Shape kWide = {12, 4, 4};      // k_tile_run
+constexpr Shape kThin = {10, 2, 2};      // k_tile_thin
 
 // What one operation of a pass does to the amplitudes whose index matches its masks.
 enum OpKind : uint32_t {
@@ -45,12 +57,13 @@ struct __attribute__((aligned(32))) RunOp {
     uint32_t tmask, tval;   // tile position bits of the thread that have to read tval
     uint32_t live;          // the registers (amplitudes, or pairs by their lower one) that take part
     uint32_t action;        // bit 4 kind + the target's register bit
-    uint32_t layout;        // layout the operation is applied in (0 A, 1 B, 2 C)
+    uint32_t layout;        // layout the operation is applied in
     uint32_t coef;          // first coefficient
 };
 
-// One launch's operations fit 4 KB of kernel arguments. The kernel reads one operation and eight
+// One launch's operations fit 4 KB of kernel arguments. The kernels read up to two operations and eight
 // coefficients past the last.
+constexpr uint32_t kAnyLayout = ~0u;    // (host) an operation without a target fits every layout
 constexpr int kOpsMax = 72;
 constexpr int kCoefsMax = 200;
 
@@ -59,18 +72,18 @@ struct TileRunArgs {
     cx<R> *amps;
     uint32_t ntiles;
     uint32_t nops;
-    uint32_t dead;           // tile position bits that the state does not have (n < 12)
-    uint8_t pbits[12];       // u bit i <-> state bit pbits[i]
-    uint8_t zbits[12];       // the same state bits, ascending (tile bases)
-    RunOp op[kOpsMax + 1];
+    uint32_t dead;           // tile position bits that the state does not have
+    uint8_t pbits[kMaxTileBits];   // u bit i <-> state bit pbits[i]
+    uint8_t zbits[kMaxTileBits];   // the same state bits, ascending (tile bases)
+    RunOp op[kOpsMax + 2];
     double coef[kCoefsMax + 8];
 };
 static_assert(sizeof(TileRunArgs<double>) <= 4096, "kernel arguments");
 
-template <typename R>
+template <int T, typename R>
 __device__ __forceinline__ uint64_t tile_base(uint64_t t, const TileRunArgs<R> &a) {
 #pragma unroll
-    for (int i = 0; i < kTileBits; ++i) {
+    for (int i = 0; i < T; ++i) {
         const uint32_t p = a.zbits[i];
         const uint64_t lo = t & ((1ull << p) - 1ull);
         t = ((t ^ lo) << 1) | lo;
@@ -292,22 +305,26 @@ __device__ __forceinline__ void lds_put(cx<R> *t, const Regs<R> &x, uint32_t lay
     else put16<1>(t + 17u * tid, x);
 }
 
+// The (empty) instructions at the ends of the branches differ, or the compiler sinks the loads into the place
+// where they meet, in halves and with a second set of registers (250 VGPRs for 164).
 template <typename R>
 __device__ __forceinline__ void lds_get(const cx<R> *t, Regs<R> &x, uint32_t layout, uint32_t tid) {
-    if (layout == 0) get16<272>(t + tid + (tid >> 4), x);
-    else if (layout == 1) get16<17>(t + (tid & 15u) + 272u * (tid >> 4), x);
-    else get16<1>(t + 17u * tid, x);
+    if (layout == 0) {
+        get16<272>(t + tid + (tid >> 4), x);
+        asm volatile("; layout A");
+    } else if (layout == 1) {
+        get16<17>(t + (tid & 15u) + 272u * (tid >> 4), x);
+        asm volatile("; layout B");
+    } else {
+        get16<1>(t + 17u * tid, x);
+        asm volatile("; layout C");
+    }
 }
 
-template <typename R, bool SMALL>
-__device__ __forceinline__ void tile_load(Regs<R> &x, uint64_t base, uint32_t tid, const TileRunArgs<R> &a) {
+template <typename R>
+__device__ __forceinline__ void tile_load(Regs<R> &x, uint64_t base, const TileRunArgs<R> &a) {
     each16([&](auto E) {
         constexpr int e = E;
-        if constexpr (SMALL) {
-            x.re[e] = 0;
-            x.im[e] = 0;
-            if ((tid + 256u * e) & a.dead) return;
-        }
         const cx<R> v = a.amps[base + u_offset<8, 12>(256u * e, a)];
         x.re[e] = v.re;
         x.im[e] = v.im;
@@ -332,9 +349,7 @@ __device__ __forceinline__ Coefs coefs_at(const TileRunArgs<R> &a, uint32_t at) 
 // targets above bit 3 on u bits 8..11 and the other four on 4..7, so the usual run of gates on 8 high
 // bits takes one move (A, then B, stored from B) where a pass that keeps the tile in LDS takes a read
 // and a write for every gate or two. The next tile's loads are in flight while one is worked on.
-// SMALL: the one tile of a state of fewer than 12 qubits (positions it does not have are neither read
-// nor written).
-template <typename R, bool SMALL>
+template <typename R>
 __global__ __launch_bounds__(256, sizeof(R) == 8 ? 2 : 4) void k_tile_run(const TileRunArgs<R> a) {
     __shared__ cx<R> t[4096 + 256];
     const uint32_t tid = threadIdx.x;
@@ -345,11 +360,11 @@ __global__ __launch_bounds__(256, sizeof(R) == 8 ? 2 : 4) void k_tile_run(const 
     const uint32_t end = min(tile + per, a.ntiles);
     if (tile >= end) return;   // the same for every thread of the workgroup
     Regs<R> nx;
-    tile_load<R, SMALL>(nx, tile_base(tile, a) + off_a, tid, a);
+    tile_load<R>(nx, tile_base<12>(tile, a) + off_a, a);
     for (bool first = true;; first = false) {
         Regs<R> x = nx;
-        const uint64_t base = tile_base(tile, a);
-        if (!SMALL) tile_load<R, SMALL>(nx, tile_base(min(tile + 1, end - 1), a) + off_a, tid, a);
+        const uint64_t base = tile_base<12>(tile, a);
+        tile_load<R>(nx, tile_base<12>(min(tile + 1, end - 1), a) + off_a, a);
         // a tile's first move writes slots that others may still read from the tile before
         bool fresh = !first;
         uint32_t layout = 0, ut = tid;
@@ -385,7 +400,6 @@ __global__ __launch_bounds__(256, sizeof(R) == 8 ? 2 : 4) void k_tile_run(const 
         if (layout == 0) {
             each16([&](auto E) {
                 constexpr int e = E;
-                if (SMALL && ((tid + 256u * e) & a.dead)) return;
                 cx<R> v;
                 v.re = x.re[e];
                 v.im = x.im[e];
@@ -394,7 +408,6 @@ __global__ __launch_bounds__(256, sizeof(R) == 8 ? 2 : 4) void k_tile_run(const 
         } else {
             each16([&](auto E) {
                 constexpr int e = E;
-                if (SMALL && (((tid & 15u) | (tid >> 4) << 8 | 16u * e) & a.dead)) return;
                 cx<R> v;
                 v.re = x.re[e];
                 v.im = x.im[e];
@@ -403,6 +416,141 @@ __global__ __launch_bounds__(256, sizeof(R) == 8 ? 2 : 4) void k_tile_run(const 
         }
         if (++tile >= end) return;
     }
+}
+
+// One operation on four amplitudes, register bit J its target; the registers of `live` and the lanes of `on`
+// keep the result.
+template <typename R, int KIND, int J>
+__device__ __forceinline__ void thin_pairs(R (&re)[4], R (&im)[4], const Coefs &c, uint32_t live, bool on) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        constexpr int f = 1 << J;
+        const int e = J == 0 ? 2 * i : i;
+        const bool keep = on && (live >> e & 1u);
+        double ar = re[e], ai = im[e], br = re[e + f], bi = im[e + f];
+        if constexpr (KIND == kFlip) {
+            const double tr = ar, ti = ai;
+            ar = br;
+            ai = bi;
+            br = tr;
+            bi = ti;
+        } else if constexpr (KIND == kReal) {
+            pair_real(ar, ai, br, bi, c);
+        } else {
+            pair_general(ar, ai, br, bi, c);
+        }
+        re[e] = keep ? (R)ar : re[e];
+        im[e] = keep ? (R)ai : im[e];
+        re[e + f] = keep ? (R)br : re[e + f];
+        im[e + f] = keep ? (R)bi : im[e + f];
+    }
+}
+
+// The same passes on small states, whose few tiles leave a kernel waiting on itself: k_tile_run's 16 amplitudes
+// a thread take an operation's pairs one after the other on 16 CUs of a 16-qubit state, through 42 KB
+// of code that each pass fetches anew. Here a tile has 1024 amplitudes, four to a thread, and an operation is
+// the same few instructions for each. Two tile bits vary across a thread's registers, so a tile moves
+// through LDS for every other target; a thread writes the slots it read, and a state that lives in the
+// caches may be stored from any layout.
+template <typename R>
+__global__ __launch_bounds__(256) void k_tile_thin(const TileRunArgs<R> a) {
+    constexpr int T = kThin.tile_bits;
+    __shared__ cx<R> t[(1 << T) + (1 << (T - 4))];
+    const uint32_t tid = threadIdx.x, tile = blockIdx.x;
+    const uint64_t base = tile_base<T>(tile, a);
+    // the first tile position of this thread's registers with their bits from `lo` on
+    auto first = [&](uint32_t lo) { return (tid & ((1u << lo) - 1u)) | (tid >> lo) << (lo + 2); };
+    uint32_t layout = 0, lo = T - 2, u = first(lo);
+    R re[4], im[4];
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+        re[e] = 0;
+        im[e] = 0;
+        if ((u | e << lo) & a.dead) continue;
+        const cx<R> v = a.amps[base + u_offset<0, T>(u | e << lo, a)];
+        re[e] = v.re;
+        im[e] = v.im;
+    }
+    // an operation's coefficients are read while the one before it is applied, its other words while the one
+    // before that is
+    RunOp op = a.op[0], nop = a.op[1];
+    Coefs c = coefs_at(a, op.coef);
+    for (uint32_t q = 0; q < a.nops; ++q) {
+        const Coefs nc = coefs_at(a, nop.coef);
+        const RunOp nnop = a.op[q + 2];
+        if (op.layout != layout) {
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e) {
+                const uint32_t p = u | e << lo;
+                cx<R> v;
+                v.re = re[e];
+                v.im = im[e];
+                t[p + (p >> 4)] = v;
+            }
+            __syncthreads();
+            layout = op.layout;
+            lo = T - 2 - 2 * layout;
+            u = first(lo);
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e) {
+                const uint32_t p = u | e << lo;
+                const cx<R> v = t[p + (p >> 4)];
+                re[e] = v.re;
+                im[e] = v.im;
+            }
+        }
+        if (((tile ^ op.oval) & op.omask) == 0) {
+            const bool on = ((u ^ op.tval) & op.tmask) == 0;
+            const uint32_t act = op.action;
+            // nested, so that an operation jumps over few others
+            if (act & 1u << 4 * kPhase) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const bool keep = on && (op.live >> e & 1u);
+                    double vr = re[e], vi = im[e];
+                    factor(vr, vi, c);
+                    re[e] = keep ? (R)vr : re[e];
+                    im[e] = keep ? (R)vi : im[e];
+                }
+            } else if (act & 1u << 4 * kNegate) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t sign = on && (op.live >> e & 1u) ? 0x80000000u : 0u;
+                    turn(re[e], sign);
+                    turn(im[e], sign);
+                }
+            } else if (act & (1u << 4 * kGeneral | 1u << 4 * kReal | 1u << 4 * kFlip)) {
+                if (act & 1u << 4 * kGeneral) thin_pairs<R, kGeneral, 0>(re, im, c, op.live, on);
+                else if (act & 1u << 4 * kReal) thin_pairs<R, kReal, 0>(re, im, c, op.live, on);
+                else thin_pairs<R, kFlip, 0>(re, im, c, op.live, on);
+            } else {
+                if (act & 2u << 4 * kGeneral) thin_pairs<R, kGeneral, 1>(re, im, c, op.live, on);
+                else if (act & 2u << 4 * kReal) thin_pairs<R, kReal, 1>(re, im, c, op.live, on);
+                else thin_pairs<R, kFlip, 1>(re, im, c, op.live, on);
+            }
+        }
+        op = nop;
+        nop = nnop;
+        c = nc;
+    }
+#pragma unroll
+    for (uint32_t e = 0; e < 4; ++e) {
+        if ((u | e << lo) & a.dead) continue;
+        cx<R> v;
+        v.re = re[e];
+        v.im = im[e];
+        a.amps[base + u_offset<0, T>(u | e << lo, a)] = v;
+    }
+}
+
+// States of up to 19 qubits take the thin kernel. Graphs of a Fourier transform / of 8 layers of a random
+// circuit in complex128, us a launch, wide -> thin: 13 qubits 86 / 153 -> 54 / 96, 16 124 / 190 -> 74 / 122,
+// 18 146 / 232 -> 97 / 176, 19 170 / 280 -> 136 / 263; 20 196 / 316 -> 215 / 342 (its 1024 tiles fill the
+// GPU, and a pass's instructions for four amplitudes count again).
+constexpr int kThinQubits = 19;
+
+Shape shape_of(const qipgpu_state *s) {
+    return s->n > kThinQubits ? kWide : kThin;
 }
 
 // ---- host side -------------------------------------------------------------------------------------
@@ -474,17 +622,17 @@ void op_counts(const HeldGate &g, int *ops, int *coefs) {
 // The held gates that the next pass takes, in order: the first, and every later one whose changed bits
 // fit the tile beside those taken and that may go before the gates left behind. On a layered circuit
 // the CNOTs and CZs of a layer so join the passes of its single-qubit gates.
-void plan_pass(const std::vector<HeldGate> &held, std::vector<char> &taken) {
+void plan_pass(const Shape &sh, const std::vector<HeldGate> &held, std::vector<char> &taken) {
     taken.assign(held.size(), 0);
     uint64_t high = 0;
     int ops = 0, coefs = 0;
     Passed left;
     for (size_t i = 0; i < held.size(); ++i) {
         const HeldGate &g = held[i];
-        const uint64_t h = (high | changed_bits(g)) & ~((1ull << kLowBits) - 1ull);
+        const uint64_t h = (high | changed_bits(g)) & ~((1ull << sh.low_bits) - 1ull);
         int no, nc;
         op_counts(g, &no, &nc);
-        if (!left.lets(g) || __builtin_popcountll(h) > kHighBits || ops + no > kOpsMax || coefs + nc > kCoefsMax) {
+        if (!left.lets(g) || __builtin_popcountll(h) > sh.high_bits() || ops + no > kOpsMax || coefs + nc > kCoefsMax) {
             left.add(g);
             continue;
         }
@@ -498,40 +646,43 @@ void plan_pass(const std::vector<HeldGate> &held, std::vector<char> &taken) {
 template <typename R>
 int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
     const int n = s->n;
+    const Shape shape = shape_of(s);
     TileRunArgs<R> a;
     std::memset(&a, 0, sizeof(a));
     a.amps = (cx<R> *)s->amps;
-    a.ntiles = n > kTileBits ? 1u << (n - kTileBits) : 1u;
-    // tile position of each state bit: bits 0..3 on u 0..3, changed bits by first use on 8..11, then
-    // 4..7, the lowest other bits on what is left (position bits a small state has no bit for are dead)
-    int upos[64], state_bit[kTileBits];
+    a.ntiles = n > shape.tile_bits ? 1u << (n - shape.tile_bits) : 1u;
+    // tile position of each state bit: the low bits on the lowest, changed bits by first use on the registers
+    // of layout 0, then of 1 and so on, the lowest other bits on what is left (position bits a small
+    // state has no bit for are dead)
+    int upos[64], state_bit[kMaxTileBits];
     std::fill(upos, upos + 64, -1);
-    std::fill(state_bit, state_bit + kTileBits, -1);
+    std::fill(state_bit, state_bit + kMaxTileBits, -1);
     auto place = [&](int p, int u) {
         upos[p] = u;
         state_bit[u] = p;
     };
-    for (int p = 0; p < kLowBits && p < n; ++p) place(p, p);
-    static const int order[kHighBits] = {8, 9, 10, 11, 4, 5, 6, 7};
-    int next = 0;
+    for (int p = 0; p < shape.low_bits && p < n; ++p) place(p, p);
+    int order[kMaxTileBits], next = 0;
+    for (int l = 0; l < shape.layouts(); ++l)
+        for (int j = 0; j < shape.reg_bits; ++j) order[l * shape.reg_bits + j] = shape.first_reg(l) + j;
     for (const HeldGate &g : gates)
         for (int i = 0; i < g.k && g.kind != HeldGate::kDiagonal; ++i)
             if (upos[g.tpos[i]] < 0) place(g.tpos[i], order[next++]);
-    // free positions: lanes first (u 4..7 from the lowest free bits keep longer runs together), then 8..11
-    // free bits in the order 4, 5, 12..17, 6..11, 18..: the memory pattern measured fastest for tiles
+    // free positions: the lowest first (longer runs together), from the free bits in the order 0..5, 12..17,
+    // 6..11, 18..: the memory pattern measured fastest for tiles
     std::vector<int> fill;
-    for (int p = 4; p < 6; ++p) fill.push_back(p);
+    for (int p = 0; p < 6; ++p) fill.push_back(p);
     for (int p = 12; p < 18; ++p) fill.push_back(p);
     for (int p = 6; p < 12; ++p) fill.push_back(p);
     for (int p = 18; p < 64; ++p) fill.push_back(p);
     size_t f = 0;
-    for (int u = kLowBits; u < kTileBits; ++u) {
+    for (int u = 0; u < shape.tile_bits; ++u) {
         if (state_bit[u] >= 0) continue;
         while (f < fill.size() && (fill[f] >= n || upos[fill[f]] >= 0)) ++f;
         if (f < fill.size()) place(fill[f], u);
     }
     std::vector<int> sorted;
-    for (int u = 0; u < kTileBits; ++u) {
+    for (int u = 0; u < shape.tile_bits; ++u) {
         if (state_bit[u] < 0) {
             a.dead |= 1u << u;
             continue;
@@ -569,8 +720,8 @@ int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
         }
     };
     auto target = [&](RunOp &op, int p) {
-        op.layout = (uint32_t)(2 - upos[p] / 4);
-        op.action <<= upos[p] % 4;
+        op.layout = (uint32_t)shape.layout_of(upos[p]);
+        op.action <<= upos[p] % shape.reg_bits;
     };
     auto push = [&](const RunOp &op, const HeldGate &g) { parts.push_back(Part{op, g, false}); };
     for (const HeldGate &g : gates) {
@@ -619,7 +770,7 @@ int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
                 std::memset(&op, 0, sizeof(op));
                 const OpKind kind = g.m[j].re == -1.0 && g.m[j].im == 0.0 ? kNegate : kPhase;
                 op.action = 1u << 4 * kind;
-                op.layout = 3;      // any
+                op.layout = kAnyLayout;
                 op.coef = (uint32_t)ncoef;
                 if (kind == kPhase) {
                     a.coef[ncoef++] = g.m[j].re;
@@ -636,15 +787,16 @@ int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
         int goal = -1;
         for (Part &p : parts) {
             if (p.done) continue;
-            if ((p.op.layout == layout || p.op.layout == 3) && left.lets(p.gate)) {
+            if ((p.op.layout == layout || p.op.layout == kAnyLayout) && left.lets(p.gate)) {
                 RunOp &op = a.op[a.nops++] = p.op;
-                const uint32_t sh = 8u - 4u * layout, rm = op.tmask >> sh & 15u, rv = op.tval >> sh & 15u;
+                const uint32_t regs = 1u << shape.reg_bits, sh = (uint32_t)shape.first_reg((int)layout);
+                const uint32_t rm = op.tmask >> sh & (regs - 1u), rv = op.tval >> sh & (regs - 1u);
                 op.layout = layout;
-                op.tmask &= ~(15u << sh);
-                op.tval &= ~(15u << sh);
-                for (uint32_t e = 0; e < 16; ++e)
+                op.tmask &= ~((regs - 1u) << sh);
+                op.tval &= ~((regs - 1u) << sh);
+                for (uint32_t e = 0; e < regs; ++e)
                     if ((e & rm) == rv) op.live |= 1u << e;
-                if (op.tmask) {     // some lanes of a wave
+                if (op.tmask && shape.reg_bits == kWide.reg_bits) {     // some lanes of a wave
                     if (op.action & 0xfu << 4 * kGeneral) op.action <<= 4 * (kSomeGeneral - kGeneral);
                     else if (op.action & 0xfu << 4 * kFlip) op.action <<= 4 * (kSomeFlip - kFlip);
                     else if (op.action & 1u << 4 * kPhase) op.action <<= 4 * (kSomePhase - kPhase);
@@ -659,9 +811,11 @@ int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
         if (done < parts.size()) layout = (uint32_t)goal;
     }
     if (!a.nops) return QIPGPU_OK;
-    const uint32_t grid = std::min<uint32_t>(a.ntiles, (uint32_t)device_cus() * (sizeof(R) == 8 ? 2 : 4));
-    if (a.dead) return launch_gate(s, &k_tile_run<R, true>, dim3(grid), dim3(256), a);
-    return launch_gate(s, &k_tile_run<R, false>, dim3(grid), dim3(256), a);
+    if (shape.reg_bits == kWide.reg_bits) {
+        const uint32_t grid = std::min<uint32_t>(a.ntiles, (uint32_t)device_cus() * (sizeof(R) == 8 ? 2 : 4));
+        return launch_gate(s, &k_tile_run<R>, dim3(grid), dim3(256), a);
+    }
+    return launch_gate(s, &k_tile_thin<R>, dim3(a.ntiles), dim3(256), a);
 }
 
 // Amplitude-sized cost of one launch (about 4 us of HBM time) when choosing between one pass for a run
@@ -673,7 +827,7 @@ constexpr uint64_t kLaunchCostAmps = 1ull << 19;
 // where that moves fewer amplitudes.
 int apply_next(qipgpu_state *s) {
     std::vector<char> taken;
-    plan_pass(s->held, taken);
+    plan_pass(shape_of(s), s->held, taken);
     std::vector<HeldGate> gates;
     size_t w = 0;
     for (size_t i = 0; i < s->held.size(); ++i) {

@@ -94,3 +94,19 @@ def test_runs_longer_than_a_launch_holds():
     seq += [{(i, n - 1 - i): SwapMat(1)} for i in range(n // 2)]
     seq += [{(0, 1): numpy.diag(numpy.exp(1j * rng.uniform(0, 6, 4)))} for _ in range(70)]
     check(n, numpy.complex128, seq, rng, True)
+
+
+@pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
+@pytest.mark.parametrize("n", [4, 9, 10, 14, 19, 20])
+def test_every_target_and_control_of_small_states(n, dtype):
+    """Every operation kind on every target, with the control just above and just below it, on states of
+    one tile of 1024, of several, and on either side of the size at which tiles become 4096."""
+    rng = numpy.random.default_rng(90 + n)
+    seq = []
+    for t in range(n):
+        above, below = (t + 1) % n, (t - 1) % n
+        seq += [{t: unitary(rng)}, {t: HM}, {(above, t): CMat(XM)}, {(below, t): CMat(unitary(rng))}, {t: XM},
+                {(above, t): CMat(numpy.diag([1.0, numpy.exp(0.7j)]))}, {(t, below): CMat(ZM)},
+                {(t, (t + n // 2) % n): SwapMat(1)}, {(below, t): numpy.diag(numpy.exp(1j * rng.uniform(0, 6, 4)))}]
+    print("targets n", n, numpy.dtype(dtype).name, flush=True)
+    check(n, dtype, seq, rng, dtype == numpy.complex128 and n <= 10)
