@@ -1672,10 +1672,17 @@ __global__ __launch_bounds__(256) void k_marg_final(const double *__restrict__ p
 // Marginals of every outcome in one pass over the state (n >= 12). The state is read in chunks of
 // 4096 amplitudes, the state bits 0..11; the other bits are the k_hi measured bits above 11 and the
 // free (unmeasured) bits above 11. Block b takes outcome bits m_hi = b / nparts and the part
-// b % nparts of the free-bit combinations, sums |amp|^2 per chunk position over its chunks (thread t
-// keeps positions t + 256 j in registers, so every load is contiguous across the block), then folds
-// the 4096 position sums into the 2^k_lo outcomes of the measured bits among 0..11, in a fixed order.
-// k_marg_pass_final adds the parts of each outcome in order and writes it at its output index.
+// b % nparts of the free-bit combinations and sums |amp|^2 per chunk position over its chunks: thread t
+// keeps positions t + 256 j in registers, so every load is contiguous across the block. The free
+// bits among 0..11 are then summed over where they lie: 8..11 in a thread's registers, 0..5 across the
+// lanes of a wave, 6 and 7 through LDS, each in a fixed order, and what is left is written at its
+// outcomes' output indices. With several parts each writes its sums in state-bit order, contiguously,
+// and k_marg_pass_final adds them in order and puts them at the output indices.
+//
+// Bound: HBM. Reading 20 of 28 qubits (complex128) took 1248 us and 20 of 30 (complex64) 4713 us when the 4096
+// sums of every chunk passed through LDS and each outcome gathered its own by byte-wide bit lists; a
+// copy's rate would be 810 and 1620. Calls with their result on the host: 2.68 -> 1.43 ms and 5.99 -> 3.14
+// (8 MiB of results at scattered indices), 16 of 28 qubits 1.65 -> 0.77, 16 of 16 0.140 -> 0.064.
 constexpr int kMargChunkBits = 12;
 
 struct MargPassArgs {
@@ -1683,20 +1690,35 @@ struct MargPassArgs {
     uint64_t free_mask;          // unmeasured state bits above 11
     uint64_t m_total;            // 2^k outcomes
     uint32_t nparts;
-    int32_t k, klo, khi, nfree_lo;
-    uint8_t hi_meas[QIPGPU_MAX_QUBITS];   // measured state bits above 11, ascending (m_hi bit i)
-    uint8_t lo_meas[kMargChunkBits];      // measured state bits among 0..11, ascending (m_lo bit i)
-    uint8_t lo_free[kMargChunkBits];      // unmeasured state bits among 0..11, ascending
-    uint8_t opos[QIPGPU_MAX_QUBITS];      // state bit of output bit j
+    uint32_t lo_free;            // unmeasured state bits among 0..11
+    int32_t khi;
+    PosList hi_meas;             // measured state bits above 11, ascending (m_hi bit i)
+    PosList hi_out;              // the bit of each in the index written
+    PosList lo_out;              // the same for state bits 0..11 (0 where not measured)
 };
 
+// The output bit of each measured state bit, ascending.
+struct MargOrder {
+    int32_t k;
+    PosList out;
+};
+
+__device__ __forceinline__ uint64_t marg_out_index(uint64_t t, const MargOrder &o) {
+    uint64_t oi = 0;
+    for (int i = 0; i < o.k; ++i) oi |= (t >> i & 1ull) << o.out.at(i);
+    return oi;
+}
+
 template <typename R>
-__global__ __launch_bounds__(256) void k_marg_pass(const cx<R> *__restrict__ amps, MargPassArgs a, double *partial) {
-    __shared__ double sums[1 << kMargChunkBits];
-    __shared__ double red[256];
+__global__ __launch_bounds__(256) void k_marg_pass(const cx<R> *__restrict__ amps, MargPassArgs a, double *out) {
+    __shared__ double red[4][256];
     const uint32_t tid = threadIdx.x;
     const uint64_t m_hi = blockIdx.x / a.nparts, part = blockIdx.x % a.nparts;
-    const uint64_t hi_base = scatter_bits(m_hi, a.hi_meas, a.khi);
+    uint64_t hi_base = 0, oi = 0;
+    for (int i = 0; i < a.khi; ++i) {
+        hi_base |= (m_hi >> i & 1ull) << a.hi_meas.at(i);
+        oi |= (m_hi >> i & 1ull) << a.hi_out.at(i);
+    }
     // free bits of the first combination of this part; the next combination in ascending order is
     // (x - free_mask) & free_mask
     uint64_t x = 0;
@@ -1722,57 +1744,76 @@ __global__ __launch_bounds__(256) void k_marg_pass(const cx<R> *__restrict__ amp
         }
         x = (x - a.free_mask) & a.free_mask;
     }
+    // every branch below is uniform
+    const uint32_t lo_free = a.lo_free, reg_free = lo_free >> 8;
 #pragma unroll
-    for (int j = 0; j < 16; ++j) sums[tid + 256 * j] = acc[j];
-    __syncthreads();
-    // outcome m_lo sums the positions with its measured bits, the free ones ascending; with fewer
-    // than 256 outcomes, g = 256 / 2^klo threads share one (free combinations u = g', g' + g, ...)
-    const uint32_t nlo = 1u << a.klo;
-    const uint32_t g = nlo >= 256 ? 1u : 256u / nlo;
-    for (uint32_t idx = tid; idx < nlo * g; idx += 256) {
-        const uint32_t mlo = idx / g, gi = idx % g;
-        const uint32_t lb = (uint32_t)scatter_bits(mlo, a.lo_meas, a.klo);
-        double s = 0.0;
-        for (uint32_t u = gi; u < (uint32_t)a.nfree_lo; u += g) s += sums[lb | (uint32_t)scatter_bits(u, a.lo_free, kMargChunkBits - a.klo)];
-        if (g == 1) partial[(uint64_t)blockIdx.x * nlo + mlo] = s;
-        else red[idx] = s;
+    for (int b = 0; b < 4; ++b)
+        if (reg_free >> b & 1u) {
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (!(j >> b & 1)) acc[j] += acc[j | 1 << b];
+        }
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        if (j & reg_free) continue;
+#pragma unroll
+        for (int b = 0; b < 6; ++b)
+            if (lo_free >> b & 1u) acc[j] += __shfl_xor(acc[j], 1 << b, 64);
     }
-    if (g > 1) {
-        __syncthreads();
-        if (tid < nlo) {
-            double s = 0.0;
-            for (uint32_t gi = 0; gi < g; ++gi) s += red[tid * g + gi];
-            partial[(uint64_t)blockIdx.x * nlo + tid] = s;
+    if (lo_free & 0xc0u) {
+        // four registers a round; the threads whose free wave bits are 0 take the sums
+        const uint32_t s6 = lo_free & 0x40u, s7 = lo_free & 0x80u;
+#pragma unroll
+        for (int j0 = 0; j0 < 16; j0 += 4) {
+            if (j0 & reg_free) continue;
+            if (j0) __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 4; ++j) red[j][tid] = acc[j0 + j];
+            __syncthreads();
+            if (!(tid & lo_free & 0xc0u)) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    double s = acc[j0 + j];
+                    if (s6) s += red[j][tid | 0x40u];
+                    if (s7) s += red[j][tid | 0x80u];
+                    if (s6 && s7) s += red[j][tid | 0xc0u];
+                    acc[j0 + j] = s;
+                }
+            }
         }
     }
-}
-
-__device__ __forceinline__ uint64_t marg_out_index(uint64_t m_hi, uint64_t mlo, const MargPassArgs &a) {
-    const uint64_t sb = scatter_bits(m_hi, a.hi_meas, a.khi) | scatter_bits(mlo, a.lo_meas, a.klo);
-    uint64_t oi = 0;
-    for (int j = 0; j < a.k; ++j) oi |= ((sb >> a.opos[j]) & 1ull) << j;
-    return oi;
+    if (tid & lo_free) return;     // positions whose free bits are 0 write
+#pragma unroll
+    for (int b = 0; b < 8; ++b) oi |= (uint64_t)(tid >> b & 1u) << a.lo_out.at(b);
+    double *o = out + part * a.m_total + oi;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        if (j & reg_free) continue;
+        uint64_t oj = 0;
+#pragma unroll
+        for (int b = 0; b < 4; ++b) oj |= (uint64_t)(j >> b & 1) << a.lo_out.at(8 + b);
+        o[oj] = acc[j];
+    }
 }
 
 // one thread per outcome, the parts in order (few parts)
-__global__ __launch_bounds__(256) void k_marg_pass_final(const double *__restrict__ partial, MargPassArgs a, double *out) {
+__global__ __launch_bounds__(256) void k_marg_pass_final(const double *__restrict__ partial, uint64_t m_total,
+                                                         uint32_t nparts, MargOrder o, double *out) {
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.m_total) return;
-    const uint64_t m_hi = t >> a.klo, mlo = t & ((1ull << a.klo) - 1ull);
+    if (t >= m_total) return;
     double s = 0.0;
-    for (uint32_t p = 0; p < a.nparts; ++p) s += partial[((m_hi * a.nparts + p) << a.klo) + mlo];
-    out[marg_out_index(m_hi, mlo, a)] = s;
+    for (uint32_t p = 0; p < nparts; ++p) s += partial[p * m_total + t];
+    out[marg_out_index(t, o)] = s;
 }
 
 // one wavefront per outcome (many parts): lane l adds parts l, l + 64, ... in order, then a butterfly
-__global__ __launch_bounds__(64) void k_marg_pass_final_wave(const double *__restrict__ partial, MargPassArgs a,
-                                                             double *out) {
+__global__ __launch_bounds__(64) void k_marg_pass_final_wave(const double *__restrict__ partial, uint64_t m_total,
+                                                             uint32_t nparts, MargOrder o, double *out) {
     const uint64_t t = blockIdx.x;
-    const uint64_t m_hi = t >> a.klo, mlo = t & ((1ull << a.klo) - 1ull);
     double s = 0.0;
-    for (uint32_t p = threadIdx.x; p < a.nparts; p += 64) s += partial[((m_hi * a.nparts + p) << a.klo) + mlo];
+    for (uint32_t p = threadIdx.x; p < nparts; p += 64) s += partial[p * m_total + t];
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if (threadIdx.x == 0) out[marg_out_index(m_hi, mlo, a)] = s;
+    if (threadIdx.x == 0) out[marg_out_index(t, o)] = s;
 }
 
 namespace {
@@ -1807,25 +1848,24 @@ static int marginals_pass(qipgpu_state *s, const std::vector<int> &mpos, const u
     const int n = s->n, k = (int)mpos.size();
     MargPassArgs a;
     std::memset(&a, 0, sizeof(a));
-    a.k = k;
     a.m_total = 1ull << k;
-    std::vector<int> sorted(mpos);
-    std::sort(sorted.begin(), sorted.end());
     uint64_t meas_mask = 0;
-    for (int p : sorted) {
-        meas_mask |= 1ull << p;
-        if (p < kMargChunkBits) a.lo_meas[a.klo++] = (uint8_t)p;
-        else a.hi_meas[a.khi++] = (uint8_t)p;
+    for (int p : mpos) meas_mask |= 1ull << p;
+    MargOrder order;
+    std::memset(&order, 0, sizeof(order));
+    for (int p = 0; p < n; ++p) {
+        if (meas_mask >> p & 1) {
+            order.out.set(order.k++, (uint32_t)(std::find(opos, opos + k, (uint8_t)p) - opos));
+            if (p >= kMargChunkBits) a.hi_meas.set(a.khi++, (uint32_t)p);
+        } else if (p < kMargChunkBits) {
+            a.lo_free |= 1u << p;
+        } else {
+            a.free_mask |= 1ull << p;
+        }
     }
-    for (int b = 0; b < kMargChunkBits; ++b)
-        if (!(meas_mask >> b & 1)) a.lo_free[a.nfree_lo++] = (uint8_t)b;
-    a.nfree_lo = 1 << a.nfree_lo;   // combinations of the free low bits
-    for (int b = kMargChunkBits; b < n; ++b)
-        if (!(meas_mask >> b & 1)) a.free_mask |= 1ull << b;
-    for (int j = 0; j < k; ++j) a.opos[j] = opos[j];
     // about eight blocks per CU, each summing a power-of-two share of the free combinations. The
-    // partials (2^k per part, read back strided) stay within 8 MiB unless that leaves fewer than two
-    // blocks per CU, and within 256 MiB.
+    // partials (2^k per part) stay within 8 MiB unless that leaves fewer than two blocks per CU, and
+    // within 256 MiB. A single part is the result.
     const int nfree_hi = n - kMargChunkBits - a.khi;
     const size_t res_bytes = ((sizeof(double) * a.m_total + 255) / 256) * 256;
     const size_t part_cap = area ? (area->cap > res_bytes ? area->cap - res_bytes : 0) : (256ull << 20);
@@ -1835,16 +1875,24 @@ static int marginals_pass(qipgpu_state *s, const std::vector<int> &mpos, const u
            (sizeof(double) * a.m_total * nparts * 2 <= (8ull << 20) || blocks_of(nparts) < 512) &&
            sizeof(double) * a.m_total * nparts * 2 <= part_cap)
         nparts *= 2;
+    for (int p = 0, i = 0; p < n; ++p) {
+        if (!(meas_mask >> p & 1)) continue;
+        const uint32_t to = nparts > 1 ? (uint32_t)i : order.out.at(i);
+        if (p < kMargChunkBits) a.lo_out.set(p, to);
+        else a.hi_out.set(i - (order.k - a.khi), to);
+        ++i;
+    }
     a.nparts = (uint32_t)nparts;
     a.per = (1ull << nfree_hi) / nparts;
     const uint64_t nblk = (1ull << a.khi) * nparts;
     if (nblk > 0x7fffffffull) return set_error(QIPGPU_EUNSUP, "marginal grid too large");
     const size_t part_off = res_bytes;
     char *space = nullptr;
-    int rc = reduction_space(s, area, part_off + std::max(sizeof(double) * a.m_total * nparts, extra), &space);
+    const size_t part_bytes = nparts > 1 ? sizeof(double) * a.m_total * nparts : 0;
+    int rc = reduction_space(s, area, part_off + std::max(part_bytes, extra), &space);
     if (rc) return rc;
     double *d_out = reinterpret_cast<double *>(space);
-    double *d_part = reinterpret_cast<double *>(space + part_off);
+    double *d_part = nparts > 1 ? reinterpret_cast<double *>(space + part_off) : d_out;
     if (s->dtype == QIPGPU_C128)
         hipLaunchKernelGGL(k_marg_pass<double>, dim3((uint32_t)nblk), dim3(256), 0, s->stream, (const cx<double> *)s->amps,
                            a, d_part);
@@ -1852,10 +1900,13 @@ static int marginals_pass(qipgpu_state *s, const std::vector<int> &mpos, const u
         hipLaunchKernelGGL(k_marg_pass<float>, dim3((uint32_t)nblk), dim3(256), 0, s->stream, (const cx<float> *)s->amps,
                            a, d_part);
     QIP_LAUNCHED();
+    if (nparts == 1) return QIPGPU_OK;
     if (nparts >= 64)   // then 2^k_hi <= 32 and m_total <= 2^17 wavefronts
-        hipLaunchKernelGGL(k_marg_pass_final_wave, dim3((uint32_t)a.m_total), dim3(64), 0, s->stream, d_part, a, d_out);
+        hipLaunchKernelGGL(k_marg_pass_final_wave, dim3((uint32_t)a.m_total), dim3(64), 0, s->stream, d_part,
+                           a.m_total, a.nparts, order, d_out);
     else
-        hipLaunchKernelGGL(k_marg_pass_final, dim3(blocks_for(a.m_total, 256)), dim3(256), 0, s->stream, d_part, a, d_out);
+        hipLaunchKernelGGL(k_marg_pass_final, dim3(blocks_for(a.m_total, 256)), dim3(256), 0, s->stream, d_part,
+                           a.m_total, a.nparts, order, d_out);
     QIP_LAUNCHED();
     return QIPGPU_OK;
 }
