@@ -553,6 +553,74 @@ Shape shape_of(const qipgpu_state *s) {
     return s->n > kThinQubits ? kWide : kThin;
 }
 
+// Exchanges of state bits, all at once: amplitude i and amplitude P(i) change places, P the permutation of
+// the index bits that exchanges bit a.at(j) with b.at(j) for every j (all different). One pass over the amplitudes
+// that move, where tiles take the exchanges four to a pass. P acts on each index bit by itself, so a
+// workgroup's part of P(i) is formed once, in scalar registers, and a thread's part once per launch.
+// Bound: HBM, in runs of 2^(lowest exchanged bit) amplitudes.
+constexpr int kExchangesMax = 17;      // disjoint pairs of 34 state bits
+constexpr int kExchangeItems = 4;
+
+template <typename R>
+struct ExchangeArgs {
+    cx<R> *amps;
+    uint64_t nblocks;       // of 256 kExchangeItems amplitudes
+    uint64_t of_item[kExchangeItems];   // P(256 it)
+    PosList a, b;
+    PosList order;          // the state bit of each bit of the block number
+};
+
+template <typename R>
+__host__ __device__ __forceinline__ uint64_t exchanged(uint64_t i, const ExchangeArgs<R> &x) {
+    for (int j = 0; j < x.a.count; ++j) {
+        const uint32_t p = x.a.at(j), q = x.b.at(j);
+        const uint64_t d = (i >> p ^ i >> q) & 1ull;
+        i ^= d << p | d << q;
+    }
+    return i;
+}
+
+template <typename R>
+__global__ __launch_bounds__(256) void k_exchange(const ExchangeArgs<R> x) {
+    const uint64_t of_thread = exchanged<R>(threadIdx.x, x);
+    for (uint64_t blk = blockIdx.x; blk < x.nblocks; blk += gridDim.x) {
+        uint64_t base = 0;
+        for (int b = 0; b < x.order.count; ++b) base |= (blk >> b & 1ull) << x.order.at(b);
+        const uint64_t to = exchanged<R>(base, x);
+        uint64_t i[kExchangeItems], j[kExchangeItems];
+        bool any = false;
+#pragma unroll
+        for (int it = 0; it < kExchangeItems; ++it) {
+            i[it] = base + 256 * it + threadIdx.x;
+            j[it] = to | x.of_item[it] | of_thread;
+            any = any || i[it] < j[it];
+        }
+        if (__ballot(any) == 0) continue;      // the other side's waves move these
+        // a lane whose amplitude stays, or is another lane's to move, reads it and writes nothing: loads
+        // without a branch are all in flight at once
+        R vr[kExchangeItems], vi[kExchangeItems], wr[kExchangeItems], wi[kExchangeItems];
+#pragma unroll
+        for (int it = 0; it < kExchangeItems; ++it) {
+            const cx<R> v = x.amps[i[it]], w = x.amps[i[it] < j[it] ? j[it] : i[it]];
+            vr[it] = v.re;
+            vi[it] = v.im;
+            wr[it] = w.re;
+            wi[it] = w.im;
+        }
+#pragma unroll
+        for (int it = 0; it < kExchangeItems; ++it)
+            if (i[it] < j[it]) {
+                cx<R> v, w;
+                v.re = vr[it];
+                v.im = vi[it];
+                w.re = wr[it];
+                w.im = wi[it];
+                x.amps[i[it]] = w;
+                x.amps[j[it]] = v;
+            }
+    }
+}
+
 // ---- host side -------------------------------------------------------------------------------------
 
 uint64_t changed_bits(const HeldGate &g) {
@@ -619,10 +687,35 @@ void op_counts(const HeldGate &g, int *ops, int *coefs) {
     }
 }
 
+// A swap that k_exchange may take: no controls, and neither bit among those that every tile holds (its runs
+// would be shorter than a tile's).
+bool exchanges(const Shape &sh, int n, const HeldGate &g) {
+    return n > sh.tile_bits && g.kind == HeldGate::kSwap && !g.ctrl_mask && g.tpos[0] >= sh.low_bits &&
+           g.tpos[1] >= sh.low_bits;
+}
+
+// The swaps that the next k_exchange takes: the first held gate, and every later one on other bits that
+// may go before the gates left behind.
+void plan_exchange(const Shape &sh, int n, const std::vector<HeldGate> &held, std::vector<char> &taken) {
+    taken.assign(held.size(), 0);
+    uint64_t bits = 0;
+    Passed left;
+    for (size_t i = 0; i < held.size(); ++i) {
+        const HeldGate &g = held[i];
+        if (!exchanges(sh, n, g) || (changed_bits(g) & bits) || !left.lets(g)) {
+            left.add(g);
+            continue;
+        }
+        bits |= changed_bits(g);
+        taken[i] = 1;
+    }
+}
+
 // The held gates that the next pass takes, in order: the first, and every later one whose changed bits
 // fit the tile beside those taken and that may go before the gates left behind. On a layered circuit
-// the CNOTs and CZs of a layer so join the passes of its single-qubit gates.
-void plan_pass(const Shape &sh, const std::vector<HeldGate> &held, std::vector<char> &taken) {
+// the CNOTs and CZs of a layer so join the passes of its single-qubit gates. A swap that would bring two
+// bits of its own is left for k_exchange.
+void plan_pass(const Shape &sh, int n, const std::vector<HeldGate> &held, std::vector<char> &taken) {
     taken.assign(held.size(), 0);
     uint64_t high = 0;
     int ops = 0, coefs = 0;
@@ -632,7 +725,8 @@ void plan_pass(const Shape &sh, const std::vector<HeldGate> &held, std::vector<c
         const uint64_t h = (high | changed_bits(g)) & ~((1ull << sh.low_bits) - 1ull);
         int no, nc;
         op_counts(g, &no, &nc);
-        if (!left.lets(g) || __builtin_popcountll(h) > sh.high_bits() || ops + no > kOpsMax || coefs + nc > kCoefsMax) {
+        const bool apart = exchanges(sh, n, g) && __builtin_popcountll(h & ~high) > 1;
+        if (apart || !left.lets(g) || __builtin_popcountll(h) > sh.high_bits() || ops + no > kOpsMax || coefs + nc > kCoefsMax) {
             left.add(g);
             continue;
         }
@@ -818,16 +912,42 @@ int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
     return launch_gate(s, &k_tile_thin<R>, dim3(a.ntiles), dim3(256), a);
 }
 
+template <typename R>
+int launch_exchange(qipgpu_state *s, const std::vector<HeldGate> &swaps) {
+    ExchangeArgs<R> a;
+    std::memset(&a, 0, sizeof(a));
+    a.amps = (cx<R> *)s->amps;
+    a.nblocks = s->len / (256 * kExchangeItems);
+    if (swaps.size() > (size_t)kExchangesMax) return set_error(QIPGPU_EINVAL, "%zu disjoint swaps", swaps.size());
+    for (const HeldGate &g : swaps) {
+        a.a.set(a.a.count++, g.tpos[0]);
+        a.b.set(a.b.count++, g.tpos[1]);
+    }
+    // block numbers count the lowest and the highest bits in turn: the workgroups in flight then differ in
+    // both, so neither their amplitudes nor those these change places with lie all at one offset of the memory
+    // channels (a register's reversal sends neighbours to places that differ in the highest bits only)
+    for (int lo = 10, hi = s->n - 1; lo <= hi;) {
+        a.order.set(a.order.count++, (uint32_t)lo++);
+        if (lo <= hi) a.order.set(a.order.count++, (uint32_t)hi--);
+    }
+    for (int it = 0; it < kExchangeItems; ++it) a.of_item[it] = exchanged<R>(256u * it, a);
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(a.nblocks, 1u << 20);
+    return launch_gate(s, &k_exchange<R>, dim3(grid), dim3(256), a);
+}
+
 // Amplitude-sized cost of one launch (about 4 us of HBM time) when choosing between one pass for a run
 // and a launch per gate.
 constexpr uint64_t kLaunchCostAmps = 1ull << 19;
 
-// Take the next pass's gates out of the held ones and apply them: as one pass over the tiles, as one
-// sweep over the amplitudes that share the controls every gate has (diagonals only), or gate by gate
+// Take the next pass's gates out of the held ones and apply them: as one exchange of bits, as one pass over
+// the tiles, as one sweep over the amplitudes that share the controls every gate has (diagonals only), or gate by gate
 // where that moves fewer amplitudes.
 int apply_next(qipgpu_state *s) {
     std::vector<char> taken;
-    plan_pass(shape_of(s), s->held, taken);
+    const Shape shape = shape_of(s);
+    const bool exchange = exchanges(shape, s->n, s->held[0]);
+    if (exchange) plan_exchange(shape, s->n, s->held, taken);
+    else plan_pass(shape, s->n, s->held, taken);
     std::vector<HeldGate> gates;
     size_t w = 0;
     for (size_t i = 0; i < s->held.size(); ++i) {
@@ -835,6 +955,7 @@ int apply_next(qipgpu_state *s) {
         else s->held[w++] = s->held[i];
     }
     s->held.resize(w);
+    if (exchange) return s->dtype == QIPGPU_C128 ? launch_exchange<double>(s, gates) : launch_exchange<float>(s, gates);
     uint64_t common = ~0ull, separate = 0;
     bool diagonal = true;
     for (const HeldGate &g : gates) {

@@ -110,3 +110,18 @@ def test_every_target_and_control_of_small_states(n, dtype):
                 {(t, (t + n // 2) % n): SwapMat(1)}, {(below, t): numpy.diag(numpy.exp(1j * rng.uniform(0, 6, 4)))}]
     print("targets n", n, numpy.dtype(dtype).name, flush=True)
     check(n, dtype, seq, rng, dtype == numpy.complex128 and n <= 10)
+
+
+@pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
+@pytest.mark.parametrize("n", [11, 13, 16, 20, 22])
+def test_swaps_that_move_together(n, dtype):
+    """Swaps in one exchange: a register's reversal, its halves, swaps that share bits, swaps behind and
+    before gates on their bits, under a control and on the lowest bits."""
+    rng = numpy.random.default_rng(17 + n)
+    sw = lambda a, b: {(a, b): SwapMat(1)}    # noqa: E731
+    seq = [sw(i, n - 1 - i) for i in range(n // 2)]
+    seq += [{0: unitary(rng)}, {n - 1: HM}] + [sw(i, i + n // 2) for i in range(n // 2)]
+    seq += [sw(0, 1), sw(1, 2), sw(2, 0), {1: unitary(rng)}, sw(3, 1), {(0, 3, 5): CMat(SwapMat(1))}, sw(5, 6)]
+    seq += [{(2, 4): CMat(XM)}, sw(2, 3), sw(4, n - 1), {4: HM}, {(n - 2, n - 3): numpy.diag([1, 1j, -1, 1.0])}, sw(n - 2, 0)]
+    print("swaps n", n, numpy.dtype(dtype).name, flush=True)
+    check(n, dtype, seq, rng, dtype == numpy.complex128 and n <= 13)
