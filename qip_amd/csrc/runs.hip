@@ -260,18 +260,24 @@ __device__ __forceinline__ void pairs_on(Regs<R> &x, uint32_t regs, const RunOp 
 
 // The action is one bit of 32, tested bit by bit: to the compiler the branches are then independent,
 // each leaving the amplitudes where they are, while the branches of a switch meet in one place with a
-// copy of all 16 from each.
+// copy of all 16 from each. In two groups, so that an operation jumps over few others (order finding on 27 qubits,
+// 170 phases: 11.75 -> 11.3 ms).
 template <typename R>
 __device__ __forceinline__ void apply_op(Regs<R> &x, const RunOp &op, const Coefs &c, bool on) {
     const uint32_t act = op.action;
-    if (act & 0xfu << 4 * kGeneral) pairs_on<R, kGeneral, false>(x, act >> 4 * kGeneral, op, c, on);
-    if (act & 0xfu << 4 * kReal) pairs_on<R, kReal, false>(x, act >> 4 * kReal, op, c, on);
-    if (act & 0xfu << 4 * kFlip) pairs_on<R, kFlip, false>(x, act >> 4 * kFlip, op, c, on);
-    if (act & 1u << 4 * kPhase) factors<R, false>(x, c, op.live, on);
-    if (act & 1u << 4 * kNegate) negate<R>(x, op.live, on);
-    if (act & 0xfu << 4 * kSomeGeneral) pairs_on<R, kGeneral, true>(x, act >> 4 * kSomeGeneral, op, c, on);
-    if (act & 0xfu << 4 * kSomeFlip) pairs_on<R, kFlip, true>(x, act >> 4 * kSomeFlip, op, c, on);
-    if (act & 1u << 4 * kSomePhase) factors<R, true>(x, c, op.live, on);
+    constexpr uint32_t kFactors = 1u << 4 * kPhase | 1u << 4 * kNegate | 1u << 4 * kSomePhase;
+    if (act & kFactors) {
+        if (act & 1u << 4 * kPhase) factors<R, false>(x, c, op.live, on);
+        if (act & 1u << 4 * kNegate) negate<R>(x, op.live, on);
+        if (act & 1u << 4 * kSomePhase) factors<R, true>(x, c, op.live, on);
+    }
+    if (act & ~kFactors) {
+        if (act & 0xfu << 4 * kGeneral) pairs_on<R, kGeneral, false>(x, act >> 4 * kGeneral, op, c, on);
+        if (act & 0xfu << 4 * kReal) pairs_on<R, kReal, false>(x, act >> 4 * kReal, op, c, on);
+        if (act & 0xfu << 4 * kFlip) pairs_on<R, kFlip, false>(x, act >> 4 * kFlip, op, c, on);
+        if (act & 0xfu << 4 * kSomeGeneral) pairs_on<R, kGeneral, true>(x, act >> 4 * kSomeGeneral, op, c, on);
+        if (act & 0xfu << 4 * kSomeFlip) pairs_on<R, kFlip, true>(x, act >> 4 * kSomeFlip, op, c, on);
+    }
 }
 
 // Tile position u of register e in each layout: A: tid + 256 e;  B: (tid & 15) | e << 4 | (tid >> 4) << 8;
