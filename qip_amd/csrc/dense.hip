@@ -11,7 +11,9 @@
 //                        three real products on FP64 MFMA (v_mfma_f64_16x16x4f64), U's fragments in
 //                        LDS. It holds every amplitude of its bases before any is written, so in place
 //                        is safe. Small states take k_dense_split, a tile by four waves.
-//   k_dense_gemm<R>      K = 7..12, out of place: a 64 x 64 output tile per workgroup over 16-column
+//   k_dense_wide<R, K>   K = 7 and 8 on states of enough tiles, in place: a workgroup holds all rows of its bases
+//                        in 128 KB of LDS and forms Y on FP64 MFMA, U's fragments from the caches.
+//   k_dense_gemm<R>      other K = 7..12, out of place: a 64 x 64 output tile per workgroup over 16-column
 //                        steps of j through LDS, into a compact [D][nbase] buffer; k_dense_scatter
 //                        writes it back to the bases' positions.
 //   k_kron_general<R>    the reference's own formula, out of place: for every output row r, the sum
@@ -257,6 +259,132 @@ __global__ __launch_bounds__(kTileThreads) void k_dense_split(const DenseTileArg
     }
 }
 
+// ---- K = 7, 8: tiles in place in LDS --------------------------------------------------------------
+//
+// A tile is all D rows of 8192 / D bases, 128 KB of LDS as FP64 pairs, for one workgroup of 8 waves a CU. It
+// is read once: each wave forms D / 8 output rows for every base from it, with the rows numbered and the
+// fragments laid out as in k_dense_mfma, and writes them over the amplitudes read. The next tile is on
+// its way to registers meanwhile. A k-step takes 1 KB of U a row block from the L2 and CB KB of X from LDS
+// for 12 MFMAs of 64 cycles, so the matrix cores are the bound: 0.70 ms for 7 targets on 2^26 amplitudes at
+// the 73 TFLOP/s that a large FP64 product reaches. The GEMM below gathers its rows 16 B at a time when the
+// targets are low bits and writes its results back from a temporary as large as the state. A call on 2^26
+// amplitudes, targets low / high / scattered, by the GEMM and here:
+//   complex128 K = 7 4.19 / 1.51 / 2.05 -> 1.07 / 1.06 / 1.05 ms; K = 8 4.62 / 2.42 / 2.39 -> 1.81 / 1.80 / 1.78
+//   complex64 K = 7 4.07 / 1.33 / 1.45 -> 0.99 / 0.98 / 0.95 ms; K = 8 3.74 / 2.21 / 2.43 -> 1.73 / 1.74 / 1.71
+template <int K>
+struct WideShape {
+    static constexpr int D = 1 << K;
+    static constexpr int KS = D / 4;
+    static constexpr int RB = D / 16;
+    static constexpr int BASES = 8192 / D;
+    static constexpr int CB = BASES / 16;
+    static constexpr int WAVES = 8;
+    static constexpr int NR = RB / WAVES;        // row blocks of a wave
+    static_assert(K == 7 || K == 8, "tiles of 7 and 8 targets");
+};
+
+template <typename R, int K>
+struct DenseWideArgs {
+    cx<R> *amps;
+    uint64_t nbase, ntiles;
+    PosList pl;                             // target and control bits
+    uint64_t row_k[4];                      // offset of the two lowest targets' values, and the controls
+    uint64_t row_s[WideShape<K>::KS];       // offset of the other targets' values
+};
+
+template <typename R, int K>
+__global__ __launch_bounds__(512) void k_dense_wide(const DenseWideArgs<R, K> a, const f64x2 *__restrict__ frag) {
+    using M = WideShape<K>;
+    __shared__ f64x2 sX[M::D * M::BASES];   // [row][base]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kap = lane >> 4, rho = lane & 15;
+    const uint64_t row = kap & 2 ? (kap & 1 ? a.row_k[3] : a.row_k[2]) : (kap & 1 ? a.row_k[1] : a.row_k[0]);
+    // bases past the last (a state of one tile): their lanes work on an earlier one and store nothing
+    auto base_at = [&](int c) { return insert_zeros((uint64_t)(16 * c + rho) & (a.nbase - 1), a.pl) + row; };
+    // this wave loads 16 k-steps' rows of one column block
+    constexpr int kPerBlock = M::WAVES / M::CB;
+    const int lc = wave / kPerBlock, ls = wave % kPerBlock * 16;
+    const uint64_t load_at = base_at(lc);
+    auto tile_at = [&](uint64_t tile) { return a.amps + insert_zeros(tile * M::BASES, a.pl); };
+    cx<R> x[16];
+    uint64_t tile = blockIdx.x;
+    auto load = [&](uint64_t t) {
+        const cx<R> *p = tile_at(t) + load_at;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) x[e] = p[a.row_s[ls + e]];
+    };
+    const f64x2 *f = frag + (size_t)wave * M::NR * 64 + lane;
+    load(tile);
+    for (;;) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const cx<double> v = to_d(x[e]);
+            sX[(4 * (ls + e) + kap) * M::BASES + 16 * lc + rho] = f64x2{v.re, v.im};
+        }
+        const uint64_t next = tile + gridDim.x;
+        __syncthreads();
+        load(next < a.ntiles ? next : tile);
+        f64x4 acc[3][M::NR][M::CB];
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int r = 0; r < M::NR; ++r)
+#pragma unroll
+                for (int c = 0; c < M::CB; ++c) acc[m][r][c] = f64x4{0.0, 0.0, 0.0, 0.0};
+        // U's fragments four k-steps ahead (1.06 ms; two: 1.09). The loop is not unrolled further: 252 B of spills
+        // at K = 7.
+        constexpr int kAhead = 4;
+        f64x2 u[kAhead][M::NR];
+#pragma unroll
+        for (int s = 0; s < kAhead; ++s)
+#pragma unroll
+            for (int r = 0; r < M::NR; ++r) u[s][r] = f[(s * M::RB + r) * 64];
+#pragma unroll 1
+        for (int s0 = 0; s0 < M::KS; s0 += kAhead) {
+            const int sn = s0 + kAhead < M::KS ? s0 + kAhead : 0;
+#pragma unroll
+            for (int s = 0; s < kAhead; ++s) {
+                f64x2 now[M::NR];
+#pragma unroll
+                for (int r = 0; r < M::NR; ++r) {
+                    now[r] = u[s][r];
+                    u[s][r] = f[((sn + s) * M::RB + r) * 64];
+                }
+#pragma unroll
+                for (int c = 0; c < M::CB; ++c) {
+                    const f64x2 v = sX[(4 * (s0 + s) + kap) * M::BASES + 16 * c + rho];
+                    const double sum = v[0] + v[1];
+#pragma unroll
+                    for (int r = 0; r < M::NR; ++r) {
+                        acc[0][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(now[r][0], v[0], acc[0][r][c], 0, 0, 0);
+                        acc[1][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(now[r][1], v[1], acc[1][r][c], 0, 0, 0);
+                        acc[2][r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(now[r][0] + now[r][1], sum, acc[2][r][c], 0, 0, 0);
+                    }
+                }
+            }
+        }
+        cx<R> *p = tile_at(tile);
+#pragma unroll
+        for (int c = 0; c < M::CB; ++c) {
+            if ((uint64_t)(16 * c + rho) >= a.nbase) continue;
+            cx<R> *pc = p + base_at(c);
+#pragma unroll
+            for (int r = 0; r < M::NR; ++r)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const double t1 = acc[0][r][c][i], t2 = acc[1][r][c][i];
+                    cx<double> y;
+                    y.re = t1 - t2;
+                    y.im = acc[2][r][c][i] - t1 - t2;
+                    pc[a.row_s[4 * (wave * M::NR + r) + i]] = from_d<R>(y);
+                }
+        }
+        if (next >= a.ntiles) return;      // the same for every wave of the workgroup
+        tile = next;
+        __syncthreads();                   // every wave is done with this tile's rows
+    }
+}
+
 // ---- K = 7..12: tiled GEMM out of place ---------------------------------------------------------
 //
 // A workgroup computes a 64-row x 64-base block of Y = U X into a compact [D][nbase] buffer, over
@@ -483,15 +611,16 @@ PosList poslist(std::vector<int> pos) {
     return pl;
 }
 
-template <typename R, int K>
-int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<int> &allpos,
-                const std::complex<double> *U) {
-    using M = MfmaShape<K>;
+// The arguments (DenseTileArgs, DenseWideArgs) and U's fragments of a kernel that numbers the rows in
+// state-bit order: bit b of a row is the b-th lowest target bit.
+template <typename M, typename A>
+std::vector<std::complex<double>> tile_arguments(A &a, qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask,
+                                                 const std::vector<int> &allpos, const std::complex<double> *U) {
     constexpr int D = M::D;
-    // rows in state-bit order: bit b of a row is the b-th lowest target bit; its place in the caller's index
+    const int K = (int)tbits.size();
     std::vector<int> sorted(tbits);
     std::sort(sorted.begin(), sorted.end());
-    int caller[D];
+    int caller[D];      // a row's place in the caller's index
     for (int j = 0; j < D; ++j) {
         caller[j] = 0;
         for (int t = 0; t < K; ++t) {
@@ -499,9 +628,8 @@ int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
             caller[j] |= (j >> b & 1) << (K - 1 - t);
         }
     }
-    DenseTileArgs<R, K> a;
     std::memset(&a, 0, sizeof(a));
-    a.amps = (cx<R> *)s->amps;
+    a.amps = (decltype(a.amps))s->amps;
     a.nbase = s->len >> allpos.size();
     a.ntiles = (a.nbase + M::BASES - 1) / M::BASES;
     a.pl = poslist(allpos);
@@ -513,7 +641,15 @@ int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
     for (int st = 0; st < M::KS; ++st)
         for (int rb = 0; rb < M::RB; ++rb)
             for (int l = 0; l < 64; ++l)
-                frag[(st * M::RB + rb) * 64 + l] = U[caller[16 * rb + l % 16] * D + caller[4 * st + l / 16]];
+                frag[(size_t)(st * M::RB + rb) * 64 + l] = U[(size_t)caller[16 * rb + l % 16] * D + caller[4 * st + l / 16]];
+    return frag;
+}
+
+template <typename R, int K>
+int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<int> &allpos,
+                const std::complex<double> *U) {
+    DenseTileArgs<R, K> a;
+    const std::vector<std::complex<double>> frag = tile_arguments<MfmaShape<K>>(a, s, tbits, ctrl_mask, allpos, U);
     void *d = nullptr;
     int rc = ring_upload(s, frag.data(), frag.size() * sizeof(frag[0]), &d);
     if (rc) return rc;
@@ -562,6 +698,25 @@ int stage_gemm_operator(qipgpu_state *s, const std::vector<uint64_t> &off, const
     QIP_HIP(hipMemcpyAsync(s->d_gemm_op, s->h_gemm_op, need, hipMemcpyHostToDevice, s->stream));
     QIP_HIP(hipEventRecord(s->gemm_ev, s->stream));
     *dev = s->d_gemm_op;
+    return QIPGPU_OK;
+}
+
+// From this many tiles on k_dense_wide is used: a workgroup's waves have D / 4 k-steps of a whole tile before
+// them, where the GEMM spreads a small state's rows over workgroups. K = 7, us a call: 64 tiles (19 qubits)
+// 59 against the GEMM's 57, 128 tiles 61 / 63, 256 63 / 75; K = 8: 256 tiles (21 qubits) 134 / 119, 512 163 / 182.
+constexpr uint64_t kWideTiles7 = 128, kWideTiles8 = 512;
+
+template <typename R, int K>
+int launch_wide(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<int> &allpos,
+                const std::complex<double> *U) {
+    DenseWideArgs<R, K> a;
+    const std::vector<std::complex<double>> frag = tile_arguments<WideShape<K>>(a, s, tbits, ctrl_mask, allpos, U);
+    void *d = nullptr;
+    const int rc = stage_gemm_operator(s, {}, frag.data(), WideShape<K>::D, &d);
+    if (rc) return rc;
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(a.ntiles, (uint64_t)device_cus());
+    hipLaunchKernelGGL((k_dense_wide<R, K>), dim3(grid), dim3(512), 0, s->stream, a, (const f64x2 *)d);
+    QIP_LAUNCHED();
     return QIPGPU_OK;
 }
 
@@ -710,6 +865,12 @@ int dense_large(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
         case 4: return c128 ? launch_tile<double, 4>(s, tbits, ctrl_mask, allpos, U) : launch_tile<float, 4>(s, tbits, ctrl_mask, allpos, U);
         case 5: return c128 ? launch_tile<double, 5>(s, tbits, ctrl_mask, allpos, U) : launch_tile<float, 5>(s, tbits, ctrl_mask, allpos, U);
         case 6: return c128 ? launch_tile<double, 6>(s, tbits, ctrl_mask, allpos, U) : launch_tile<float, 6>(s, tbits, ctrl_mask, allpos, U);
+        case 7:
+            if ((s->len >> allpos.size()) / WideShape<7>::BASES < kWideTiles7) break;
+            return c128 ? launch_wide<double, 7>(s, tbits, ctrl_mask, allpos, U) : launch_wide<float, 7>(s, tbits, ctrl_mask, allpos, U);
+        case 8:
+            if ((s->len >> allpos.size()) / WideShape<8>::BASES < kWideTiles8) break;
+            return c128 ? launch_wide<double, 8>(s, tbits, ctrl_mask, allpos, U) : launch_wide<float, 8>(s, tbits, ctrl_mask, allpos, U);
         default: break;
     }
     if (K >= 7 && K <= QIPGPU_MAX_DENSE)
