@@ -102,8 +102,9 @@ int qipgpu_apply_kron(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
 /* Product of single-qubit operators, mats[4j..4j+3] (row-major 2x2 complex128) on targets[j], for
  * k <= QIPGPU_MAX_PRODUCT distinct qubits, in one sweep: the uncontrolled single-qubit factors of
  * one kronselect_dot descriptor (e.g. H on a register, qip/operators.py:97-99), which cdot_loop
- * also applies in one sweep. Computed in FP64 on a tile held in LDS, rounded once per amplitude;
- * needs n >= 12. */
+ * also applies in one sweep. Computed in FP64 on a tile in registers, rounded once per amplitude and
+ * pass; needs n >= 12. Held back on the state (qipgpu_fused_flush): a product that follows at once is
+ * multiplied into it, one that follows behind up to 4 diagonals shares a pass with it. */
 #define QIPGPU_MAX_PRODUCT 12
 int qipgpu_apply_product(qipgpu_state *s, int32_t k, const int32_t *targets, const double *mats);
 
@@ -266,8 +267,8 @@ int qipgpu_fused_record(qipgpu_state *s, int32_t n_gates, const int32_t *gate_k,
 /* Fusion width (1..6, default 6) and streaming (1, default) or deferred (0) launches; launches what
  * is recorded first. */
 int qipgpu_fused_set_recording(qipgpu_state *s, int32_t width, int32_t streaming);
-/* Compose and launch every recorded gate (the blocks back to back), after the held-back diagonal
- * gates (qipgpu_apply_diagonal); on any state, launches what the engine holds back. */
+/* Compose and launch every recorded gate (the blocks back to back), after the gates and products held
+ * back before them; on any state, launches what the engine holds back. */
 int qipgpu_fused_flush(qipgpu_state *s);
 /* Recorded gates not launched yet, and blocks launched since the first recording on this state. */
 int qipgpu_fused_recorded(const qipgpu_state *s, int64_t *pending_gates, int64_t *blocks_launched);

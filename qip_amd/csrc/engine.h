@@ -186,7 +186,7 @@ struct TempBuffer {
 
 // Make sure s->scratch holds at least `bytes`.
 int ensure_scratch(qipgpu_state *s, size_t bytes);
-// Copies between the caller's memory and the current device's through pinned staging memory (transfer.hip),
+// Copies between the caller's memory and that of `st`'s device through pinned staging memory (transfer.hip),
 // in `st`'s order: to the host, complete on return; to the device, enqueued, the host memory free on
 // return.
 int copy_to_host(hipStream_t st, void *host, const void *dev, size_t bytes);

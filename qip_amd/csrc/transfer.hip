@@ -114,6 +114,26 @@ void give(Staging *b) {
     destroy(b);
 }
 
+// The stream's device while a copy runs, the caller's afterwards: events are recorded on their own device's
+// streams only.
+struct OnDevice {
+    int before = 0;
+    bool changed = false;
+    hipError_t rc;
+    explicit OnDevice(int device) {
+        rc = hipGetDevice(&before);
+        if (rc == hipSuccess && before != device) {
+            rc = hipSetDevice(device);
+            changed = rc == hipSuccess;
+        }
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+    ~OnDevice() {
+        if (changed) (void)hipSetDevice(before);
+    }
+};
+
 struct Part {
     hipStream_t st;
     int device;
@@ -167,8 +187,10 @@ struct Part {
 // The copy, shared by threads that each take a stretch of it and enqueue on the same stream.
 int copy(hipStream_t st, char *host, char *dev, size_t bytes, bool out) {
     if (!bytes) return QIPGPU_OK;
-    int device = 0;
-    QIP_HIP(hipGetDevice(&device));
+    hipDevice_t device = 0;
+    QIP_HIP(hipStreamGetDevice(st, &device));
+    const OnDevice on(device);
+    QIP_HIP(on.rc);
     const int count = (int)std::max<size_t>(1, std::min<size_t>(kThreads, bytes / kThreadBytes));
     const size_t each = (bytes / count + kSlotBytes - 1) / kSlotBytes * kSlotBytes;   // whole pieces
     Part part[kThreads];
