@@ -267,7 +267,8 @@ int launch_product(qipgpu_state *s, const ProductArgs &a) {
 // on u bits 8..11 only.
 // Bound: HBM, as any product pass; it takes the place of two of them and of the diagonal's launch. 40
 // iterations of a search on 23 of 24 qubits with their start and reads, complex128: 96.3 ms with a pass
-// per 8 high bits of every layer (12 an iteration), 74.0 with 5; 80 iterations in complex64 84.2 -> 80.0.
+// per 8 high bits of every layer (12 an iteration), 74.0 with 5; 80 iterations in complex64 84.2 -> 80.0. A
+// pass without LDS 87 us in complex128 and 52 in complex64, one of k_product with LDS 96 and 68.
 struct PairArgs {
     ProductArgs p;                     // the first product (no X factor: xmask = 0)
     uint32_t fmask2, rmask2;           // the second, on the same u bits

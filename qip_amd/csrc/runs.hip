@@ -347,7 +347,7 @@ __device__ __forceinline__ Coefs coefs_at(const TileRunArgs<R> &a, uint32_t at) 
 // at 28 qubits, 8 Haar gates and 4 CNOTs: complex128 2220 us before, 1860 us now (4.6 TB/s; a copy of
 // that size takes 1627); complex64 1704 and 1397 (813). 12 Haar gates on the lowest bits: 2297 and 2093,
 // 1729 and 1790. A 28-qubit depth-20 layered circuit, 20 passes of CNOTs and CZs fewer as well: 200 ms
-// before, 122 ms now.
+// before, 117 ms now.
 //
 // 256 threads, 16 amplitudes each. The four tile bits that vary across a thread's registers are u bits
 // 8..11 as loaded (layout A), 4..7 (B) or 0..3 (C); an operation is applied in the layout that has its
