@@ -17,15 +17,14 @@
 #include <vector>
 
 #include "engine.h"
+#include "share.h"
 
 namespace qipgpu {
 
 namespace {
 
 constexpr int kSlots = 4;
-constexpr size_t kSlotBytes = size_t(1) << 20;
-constexpr size_t kThreadBytes = size_t(4) << 20;    // a thread for every 4 MiB
-constexpr int kThreads = 4;
+constexpr size_t kSlotBytes = kPieceBytes;
 constexpr size_t kKept = 8;                          // staging buffers kept for later copies (32 MiB)
 
 // Pinned memory that one thread has to itself from take() to give(). A slot may still be read by a copy to
@@ -191,18 +190,18 @@ int copy(hipStream_t st, char *host, char *dev, size_t bytes, bool out) {
     QIP_HIP(hipStreamGetDevice(st, &device));
     const OnDevice on(device);
     QIP_HIP(on.rc);
-    const int count = (int)std::max<size_t>(1, std::min<size_t>(kThreads, bytes / kThreadBytes));
-    const size_t each = (bytes / count + kSlotBytes - 1) / kSlotBytes * kSlotBytes;   // whole pieces
-    Part part[kThreads];
-    std::thread thread[kThreads];
-    int parts = 0;
-    for (size_t at = 0; at < bytes; at += each) {
-        Part &p = part[parts++];
+    const Shares shares = shares_of(bytes);
+    const int parts = shares.count;
+    Part part[kCopyThreads];
+    std::thread thread[kCopyThreads];
+    for (int i = 0; i < parts; ++i) {
+        const size_t at = i * shares.each;
+        Part &p = part[i];
         p.st = st;
         p.device = device;
         p.host = host + at;
         p.dev = dev + at;
-        p.bytes = std::min(each, bytes - at);
+        p.bytes = std::min(shares.each, bytes - at);
         p.out = out;
     }
     for (int i = 1; i < parts; ++i) {
