@@ -23,94 +23,104 @@ namespace qipgpu {
 
 namespace {
 
-constexpr int kSlots = 4;
-constexpr size_t kSlotBytes = kPieceBytes;
-constexpr size_t kKept = 8;                          // staging buffers kept for later copies (32 MiB)
+constexpr int kSlots = 4;           // pieces that a thread has on their way
+constexpr int kSlotsMade = 32;      // slots a device gets at most, 32 MiB, kept for later copies
 
-// Pinned memory that one thread has to itself from take() to give(). A slot may still be read by a copy to
-// the device then; whoever uses it next waits for its event.
-struct Staging {
+// Pinned memory for one piece, one thread's from take() to give(). `busy`: the copy that `done` marks may
+// still use it. A slot is given back while an upload reads it, so that the caller need not wait for the
+// queue, and is taken again only once that is over: a copy never waits for another queue's work.
+struct Slot {
     int device = 0;
     char *p = nullptr;
-    hipEvent_t ev[kSlots] = {};
-    bool busy[kSlots] = {};
+    hipEvent_t done = nullptr;
+    bool busy = false;
 
-    hipError_t wait(int slot) {
-        if (!busy[slot]) return hipSuccess;
-        const hipError_t e = hipEventSynchronize(ev[slot]);
-        if (e == hipSuccess) busy[slot] = false;
+    hipError_t wait() {
+        if (!busy) return hipSuccess;
+        const hipError_t e = hipEventSynchronize(done);
+        if (e == hipSuccess) busy = false;
         return e;
     }
-    hipError_t mark(int slot, hipStream_t st) {
-        const hipError_t e = hipEventRecord(ev[slot], st);
-        if (e == hipSuccess) busy[slot] = true;
+    hipError_t mark(hipStream_t st) {
+        const hipError_t e = hipEventRecord(done, st);
+        if (e == hipSuccess) busy = true;
         return e;
+    }
+    bool free() {
+        if (busy && hipEventQuery(done) == hipSuccess) busy = false;
+        if (busy) (void)hipGetLastError();      // "not ready" is no error of the next launch
+        return !busy;
     }
 };
 
-void destroy(Staging *b) {
-    for (int i = 0; i < kSlots; ++i) {
-        (void)b->wait(i);
-        if (b->ev[i]) (void)hipEventDestroy(b->ev[i]);
+struct Pool {
+    std::mutex mutex;
+    std::vector<Slot *> idle;       // the one given back longest ago first; room for every slot made
+    std::vector<int> made;          // per device
+};
+
+Pool &pool() {
+    static Pool *p = new Pool;      // alive as long as the process
+    return *p;
+}
+
+// kSlots more slots for `device`, one of them returned, the others in the pool; null where it has its share or there is
+// no memory.
+Slot *make(int device) {
+    Pool &pl = pool();
+    try {
+        std::lock_guard<std::mutex> lock(pl.mutex);
+        if ((size_t)device >= pl.made.size()) pl.made.resize(device + 1, 0);
+        if (pl.made[device] + kSlots > kSlotsMade) return nullptr;
+        size_t all = kSlots;
+        for (int m : pl.made) all += m;
+        pl.idle.reserve(all);
+        pl.made[device] += kSlots;
+    } catch (const std::bad_alloc &) {
+        return nullptr;
     }
-    if (b->p) (void)hipHostFree(b->p);
-    delete b;
-}
-
-std::mutex &pool_mutex() {
-    static std::mutex *m = new std::mutex;    // alive as long as the process
-    return *m;
-}
-
-std::vector<Staging *> &pool() {
-    static std::vector<Staging *> *v = new std::vector<Staging *>;
-    return *v;
-}
-
-hipError_t take(int device, Staging **out) {
-    {
-        std::lock_guard<std::mutex> lock(pool_mutex());
-        std::vector<Staging *> &v = pool();
-        for (size_t i = v.size(); i-- > 0;)
-            if (v[i]->device == device) {
-                *out = v[i];
-                v.erase(v.begin() + (long)i);
-                return hipSuccess;
-            }
-    }
-    Staging *b = new (std::nothrow) Staging;
-    if (!b) return hipErrorOutOfMemory;
-    b->device = device;
+    Slot *slot = new (std::nothrow) Slot[kSlots];       // never freed
     void *p = nullptr;
-    hipError_t e = hipHostMalloc(&p, kSlots * kSlotBytes, hipHostMallocDefault);
-    b->p = static_cast<char *>(p);
-    for (int i = 0; i < kSlots && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&b->ev[i], hipEventDisableTiming);
-    if (e != hipSuccess) {
-        destroy(b);
-        return e;
+    bool ok = slot && hipHostMalloc(&p, kSlots * kPieceBytes, hipHostMallocDefault) == hipSuccess;
+    for (int i = 0; i < kSlots && ok; ++i) {
+        slot[i].device = device;
+        slot[i].p = static_cast<char *>(p) + i * kPieceBytes;
+        ok = hipEventCreateWithFlags(&slot[i].done, hipEventDisableTiming) == hipSuccess;
     }
-    *out = b;
-    return hipSuccess;
+    std::unique_lock<std::mutex> lock(pl.mutex);
+    if (ok) {
+        for (int i = 1; i < kSlots; ++i) pl.idle.push_back(&slot[i]);
+        return slot;
+    }
+    pl.made[device] -= kSlots;
+    lock.unlock();
+    (void)hipGetLastError();
+    for (int i = 0; slot && i < kSlots; ++i)
+        if (slot[i].done) (void)hipEventDestroy(slot[i].done);
+    if (p) (void)hipHostFree(p);
+    delete[] slot;
+    return nullptr;
 }
 
-void give(Staging *b) {
+// A slot that nothing uses, or null.
+Slot *take(int device) {
     {
-        std::lock_guard<std::mutex> lock(pool_mutex());
-        std::vector<Staging *> &v = pool();
-        if (v.size() < kKept && v.capacity() >= kKept) {
-            v.push_back(b);
-            return;
-        }
-        if (v.capacity() < kKept) {
-            try {
-                v.reserve(kKept);
-                v.push_back(b);
-                return;
-            } catch (...) {
-            }
+        Pool &pl = pool();
+        std::lock_guard<std::mutex> lock(pl.mutex);
+        for (size_t i = 0; i < pl.idle.size(); ++i) {
+            Slot *slot = pl.idle[i];
+            if (slot->device != device || !slot->free()) continue;
+            pl.idle.erase(pl.idle.begin() + (long)i);
+            return slot;
         }
     }
-    destroy(b);
+    return make(device);
+}
+
+void give(Slot *slot) {
+    Pool &pl = pool();
+    std::lock_guard<std::mutex> lock(pl.mutex);
+    pl.idle.push_back(slot);
 }
 
 // The stream's device while a copy runs, the caller's afterwards: events are recorded on their own device's
@@ -140,44 +150,53 @@ struct Part {
     size_t bytes;
     bool out;           // device to host
     hipError_t rc = hipSuccess;
+    Slot *slot[kSlots] = {};
+    int slots = 0;      // piece i goes through slot i % slots
 
     void run() {
-        Staging *b = nullptr;
-        if ((rc = take(device, &b)) != hipSuccess) return;
-        rc = out ? copy_out(b) : copy_in(b);
-        // a copy that failed half way may have left slots in flight without an event
-        if (rc != hipSuccess) (void)hipStreamSynchronize(st);
-        give(b);
+        const size_t n = pieces();
+        while (slots < kSlots && (size_t)slots < n && (slot[slots] = take(device))) ++slots;
+        if (!slots) {
+            // every slot is under an upload that waits for its queue: the runtime's own copy, and this queue's end
+            rc = out ? hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st)
+                     : hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st);
+            if (rc == hipSuccess) rc = hipStreamSynchronize(st);
+            return;
+        }
+        rc = out ? copy_out(n) : copy_in(n);
+        if (rc != hipSuccess) {
+            // a copy that failed half way may have left slots in flight without an event
+            (void)hipStreamSynchronize(st);
+            for (int i = 0; i < slots; ++i) slot[i]->busy = false;
+        }
+        for (int i = 0; i < slots; ++i) give(slot[i]);
     }
-    size_t piece(size_t i) const { return std::min(kSlotBytes, bytes - i * kSlotBytes); }
-    hipError_t fetch(Staging *b, size_t i) {
-        const int slot = (int)(i % kSlots);
-        hipError_t e = b->wait(slot);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(b->p + slot * kSlotBytes, dev + i * kSlotBytes, piece(i), hipMemcpyDeviceToHost, st);
-        return e == hipSuccess ? b->mark(slot, st) : e;
+    size_t pieces() const { return (bytes + kPieceBytes - 1) / kPieceBytes; }
+    size_t piece(size_t i) const { return std::min(kPieceBytes, bytes - i * kPieceBytes); }
+    hipError_t fetch(size_t i) {
+        Slot *b = slot[i % slots];
+        const hipError_t e = hipMemcpyAsync(b->p, dev + i * kPieceBytes, piece(i), hipMemcpyDeviceToHost, st);
+        return e == hipSuccess ? b->mark(st) : e;
     }
-    hipError_t copy_out(Staging *b) {
-        const size_t n = (bytes + kSlotBytes - 1) / kSlotBytes;
+    hipError_t copy_out(size_t n) {
         hipError_t e = hipSuccess;
-        for (size_t i = 0; i < std::min<size_t>(n, kSlots) && e == hipSuccess; ++i) e = fetch(b, i);
+        for (size_t i = 0; i < std::min<size_t>(n, slots) && e == hipSuccess; ++i) e = fetch(i);
         for (size_t i = 0; i < n && e == hipSuccess; ++i) {
-            const int slot = (int)(i % kSlots);
-            if ((e = b->wait(slot)) != hipSuccess) break;
-            std::memcpy(host + i * kSlotBytes, b->p + slot * kSlotBytes, piece(i));
-            if (i + kSlots < n) e = fetch(b, i + kSlots);
+            Slot *b = slot[i % slots];
+            if ((e = b->wait()) != hipSuccess) break;
+            std::memcpy(host + i * kPieceBytes, b->p, piece(i));
+            if (i + slots < n) e = fetch(i + slots);
         }
         return e;
     }
-    hipError_t copy_in(Staging *b) {
-        const size_t n = (bytes + kSlotBytes - 1) / kSlotBytes;
+    hipError_t copy_in(size_t n) {
         hipError_t e = hipSuccess;
         for (size_t i = 0; i < n && e == hipSuccess; ++i) {
-            const int slot = (int)(i % kSlots);
-            if ((e = b->wait(slot)) != hipSuccess) break;
-            std::memcpy(b->p + slot * kSlotBytes, host + i * kSlotBytes, piece(i));
-            e = hipMemcpyAsync(dev + i * kSlotBytes, b->p + slot * kSlotBytes, piece(i), hipMemcpyHostToDevice, st);
-            if (e == hipSuccess) e = b->mark(slot, st);
+            Slot *b = slot[i % slots];
+            if ((e = b->wait()) != hipSuccess) break;
+            std::memcpy(b->p, host + i * kPieceBytes, piece(i));
+            e = hipMemcpyAsync(dev + i * kPieceBytes, b->p, piece(i), hipMemcpyHostToDevice, st);
+            if (e == hipSuccess) e = b->mark(st);
         }
         return e;
     }
