@@ -12,7 +12,6 @@
 #include <cstring>
 #include <mutex>
 #include <new>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -210,10 +209,8 @@ int copy(hipStream_t st, char *host, char *dev, size_t bytes, bool out) {
     const OnDevice on(device);
     QIP_HIP(on.rc);
     const Shares shares = shares_of(bytes);
-    const int parts = shares.count;
     Part part[kCopyThreads];
-    std::thread thread[kCopyThreads];
-    for (int i = 0; i < parts; ++i) {
+    for (int i = 0; i < shares.count; ++i) {
         const size_t at = i * shares.each;
         Part &p = part[i];
         p.st = st;
@@ -223,24 +220,13 @@ int copy(hipStream_t st, char *host, char *dev, size_t bytes, bool out) {
         p.bytes = std::min(shares.each, bytes - at);
         p.out = out;
     }
-    for (int i = 1; i < parts; ++i) {
-        Part *p = &part[i];
-        try {
-            thread[i] = std::thread([p] {
-                p->rc = hipSetDevice(p->device);
-                if (p->rc == hipSuccess) p->run();
-            });
-        } catch (const std::system_error &) {
-            // no thread to be had: this one takes the stretch too, below
-        }
-    }
-    part[0].run();
-    hipError_t e = part[0].rc;
-    for (int i = 1; i < parts; ++i) {
-        if (thread[i].joinable()) thread[i].join();
-        else part[i].run();
-        if (e == hipSuccess) e = part[i].rc;
-    }
+    auto work = [&part](int i) {
+        part[i].rc = hipSetDevice(part[i].device);
+        if (part[i].rc == hipSuccess) part[i].run();
+    };
+    run_shares<std::thread>(shares.count, work);
+    hipError_t e = hipSuccess;
+    for (int i = 0; i < shares.count && e == hipSuccess; ++i) e = part[i].rc;
     if (e != hipSuccess) {
         (void)hipGetLastError();
         return set_error(e == hipErrorOutOfMemory ? QIPGPU_ENOMEM : QIPGPU_EHIP, "a copy of %zu bytes %s failed: %s", bytes,
