@@ -642,12 +642,7 @@ int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
     const size_t b_glen = sizeof(int32_t) * n_groups, b_gpos = sizeof(int32_t) * total_idx;
     const size_t o_goff = ((b_glen + b_gpos + 15) / 16) * 16;
     const size_t o_feed = o_goff + ((sizeof(int64_t) * n_groups + 15) / 16) * 16;
-    // a real feed crosses the link as it is, behind the feeds, and is widened on the device
-    const size_t o_real = o_feed + sizeof(double) * 2 * total_feed;
-    size_t real_bytes = 0;
-    for (int g = 0; g < n_groups; ++g)
-        if (real && real[g]) real_bytes = std::max(real_bytes, sizeof(double) << group_len[g]);
-    int rc = ensure_scratch(s, o_real + real_bytes);
+    int rc = ensure_scratch(s, o_feed + sizeof(double) * 2 * total_feed);
     if (rc) return rc;
     char *d = static_cast<char *>(s->scratch);
     std::vector<char> h(o_feed);
@@ -658,13 +653,15 @@ int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
     for (int g = 0; g < n_groups; ++g) {
         const uint64_t count = 1ull << group_len[g];
         cx<double> *to = reinterpret_cast<cx<double> *>(d + o_feed) + goff[g];
+        // a real feed crosses the link as it is, to the amplitudes, which are written last and have room for
+        // it (2^n real numbers at most), and is widened from there
         const bool widen = real && real[g];
-        rc = copy_to_device(s->stream, widen ? (void *)(d + o_real) : (void *)to, feeds[g],
+        rc = copy_to_device(s->stream, widen ? s->amps : (void *)to, feeds[g],
                             (widen ? sizeof(double) : sizeof(cx<double>)) * count);
         if (rc) return rc;
         if (!widen) continue;
         hipLaunchKernelGGL(k_widen_feed, dim3(std::min<uint32_t>(blocks_for(count, 256), 1u << 16)), dim3(256), 0, s->stream,
-                           (const double *)(d + o_real), to, count);
+                           (const double *)s->amps, to, count);
         QIP_LAUNCHED();
     }
     InitArgs a;

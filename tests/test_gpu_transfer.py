@@ -1,6 +1,7 @@
 """Copies between host arrays and states through pinned staging memory (marked gpu): pieces of 1 MiB on four slots,
 threads from 8 MiB on. Every byte has to arrive, at sizes around those of a piece, the slots and a
 thread's share, and from several threads at once."""
+import ctypes
 import threading
 
 import numpy
@@ -64,6 +65,31 @@ def test_real_feeds_equal_complex_ones(lens, kinds, dtype):
     assert numpy.array_equal(a.get_state(), numpy.arange(2 ** n).astype(dtype))
     a.close()
     b.close()
+
+
+def test_a_real_feed_takes_no_more_device_memory_than_a_complex_one():
+    hip = ctypes.CDLL("libamdhip64.so")
+
+    def free_bytes():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    n, used, states = 25, [], []
+    for dtype in (numpy.float64, numpy.complex128, numpy.float64):      # the first use of a kernel takes memory too
+        feed = numpy.zeros(2 ** n, dtype=dtype)
+        feed[12345] = 1.0
+        free = free_bytes()
+        be = GpuBackend.make_state(n, [list(range(n))[::-1]], [feed])
+        be.synchronize()
+        used.append(free - free_bytes())
+        at = int(format(12345, '025b')[::-1], 2)
+        assert be.get_relative_range(at, at + 1)[0] == 1.0 and be.total_prob() == 1.0
+        states.append(be)
+    print("device memory of a state with a real, a complex and a real feed", used, flush=True)
+    for be in states:
+        be.close()
+    assert used[2] <= used[1] + (16 << 20)
 
 
 def test_threads_read_and_write_their_own_states():
