@@ -301,6 +301,10 @@ __global__ __launch_bounds__(256) void k_init_basis(uint4 *amps, uint64_t words,
         amps[i] = i ? make_uint4(0, 0, 0, 0) : first;
 }
 
+// Feeds of up to this many qubits (64 KiB) cross the link with the descriptor, in one copy: a copy each took longer than
+// their bytes (28 one-qubit feeds on 2^28 amplitudes 3.50 ms against 3.19 in one).
+constexpr int kPackedFeedBits = 12;
+
 // A feed given as real numbers.
 __global__ __launch_bounds__(256) void k_widen_feed(const double *__restrict__ in, cx<double> *__restrict__ out, uint64_t count) {
     const uint64_t stride = (uint64_t)gridDim.x * 256;
@@ -610,12 +614,12 @@ int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
     recorder_discard(s);
     if (n_groups < 0) return set_error(QIPGPU_EINVAL, "negative group count");
     uint64_t fed = 0;
-    int64_t total_idx = 0, total_feed = 0;
+    int64_t total_idx = 0, total_feed = 0, packed = 0;
     std::vector<int64_t> goff(std::max(n_groups, 1));
     for (int g = 0; g < n_groups; ++g) {
         if (group_len[g] < 1 || group_len[g] > s->n) return set_error(QIPGPU_EINVAL, "bad feed group length %d", group_len[g]);
-        goff[g] = total_feed;
         total_feed += 1ll << group_len[g];
+        if (group_len[g] <= kPackedFeedBits) packed += 1ll << group_len[g];
         for (int j = 0; j < group_len[g]; ++j) {
             int q = group_idx[total_idx + j];
             if (q < 0 || q >= s->n) return set_error(QIPGPU_EINVAL, "feed qubit index %d out of range", q);
@@ -636,7 +640,13 @@ int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
         QIP_LAUNCHED();
         return QIPGPU_OK;
     }
-    // device copies of the descriptor: [glen | gpos | pad | goff | feeds]
+    // device copies of the descriptor: [glen | gpos | pad | goff | short feeds | others]. What comes before the others is
+    // one copy
+    for (int64_t g = 0, at_short = 0, at_long = packed; g < n_groups; ++g) {
+        int64_t &at = group_len[g] <= kPackedFeedBits ? at_short : at_long;
+        goff[g] = at;
+        at += 1ll << group_len[g];
+    }
     std::vector<int32_t> gpos(total_idx);
     for (int64_t i = 0; i < total_idx; ++i) gpos[i] = s->n - 1 - group_idx[i];
     const size_t b_glen = sizeof(int32_t) * n_groups, b_gpos = sizeof(int32_t) * total_idx;
@@ -645,12 +655,26 @@ int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
     int rc = ensure_scratch(s, o_feed + sizeof(double) * 2 * total_feed);
     if (rc) return rc;
     char *d = static_cast<char *>(s->scratch);
-    std::vector<char> h(o_feed);
+    std::vector<char> h(o_feed + sizeof(cx<double>) * packed);
     std::memcpy(h.data(), group_len, b_glen);
     std::memcpy(h.data() + b_glen, gpos.data(), b_gpos);
     std::memcpy(h.data() + o_goff, goff.data(), sizeof(int64_t) * n_groups);
-    if ((rc = copy_to_device(s->stream, d, h.data(), o_feed))) return rc;
     for (int g = 0; g < n_groups; ++g) {
+        const size_t count = (size_t)1 << group_len[g];
+        if (group_len[g] > kPackedFeedBits) continue;
+        char *to = h.data() + o_feed + sizeof(cx<double>) * goff[g];
+        if (!real || !real[g]) {
+            std::memcpy(to, feeds[g], sizeof(cx<double>) * count);
+            continue;
+        }
+        for (size_t i = 0; i < count; ++i) {
+            const double v[2] = {feeds[g][i], 0.0};
+            std::memcpy(to + sizeof(v) * i, v, sizeof(v));
+        }
+    }
+    if ((rc = copy_to_device(s->stream, d, h.data(), h.size()))) return rc;
+    for (int g = 0; g < n_groups; ++g) {
+        if (group_len[g] <= kPackedFeedBits) continue;
         const uint64_t count = 1ull << group_len[g];
         cx<double> *to = reinterpret_cast<cx<double> *>(d + o_feed) + goff[g];
         // a real feed crosses the link as it is, to the amplitudes, which are written last and have room for

@@ -51,7 +51,7 @@ def test_basis_state(n, dtype):
 
 @pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
 @pytest.mark.parametrize("kinds", [("f8", "c16"), ("f4", "i8"), ("c8", "f8"), ("?", "f8")])
-@pytest.mark.parametrize("lens", [(1, 3), (18, 3), (2, 19)])
+@pytest.mark.parametrize("lens", [(1, 3), (18, 3), (2, 19), (12, 1), (13, 2), (11, 13)])
 def test_real_feeds_equal_complex_ones(lens, kinds, dtype):
     rng = numpy.random.default_rng(sum(lens))
     n = sum(lens)
@@ -65,6 +65,31 @@ def test_real_feeds_equal_complex_ones(lens, kinds, dtype):
     assert numpy.array_equal(a.get_state(), numpy.arange(2 ** n).astype(dtype))
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
+@pytest.mark.parametrize("lens", [(13, 1, 1), (1, 14, 2), (12, 1, 7), (2, 12, 4), (1,) * 15, (3, 2, 13)])
+def test_feeds_short_and_long_are_the_product_of_their_groups(lens, dtype):
+    rng = numpy.random.default_rng(len(lens) + sum(lens))
+    n = sum(lens)
+    perm = [int(q) for q in rng.permutation(n)]
+    groups, feeds, at = [], [], 0
+    for k in lens:
+        groups.append(perm[at:at + k])
+        feeds.append(rng.standard_normal(2 ** k) + (0 if at % 2 else 1j * rng.standard_normal(2 ** k)))
+        at += k
+    want = numpy.ones(2 ** n, dtype=numpy.complex128)
+    i = numpy.arange(2 ** n)
+    for g, f in zip(groups, feeds):
+        value = numpy.zeros(2 ** n, dtype=numpy.int64)
+        for q in g:
+            value = value << 1 | (i >> (n - 1 - q) & 1)
+        want *= f[value]
+    be = GpuBackend.make_state(n, groups, feeds, statetype=dtype)
+    eps = numpy.finfo(dtype).eps
+    # a rounding per product, and one on the way to the state's precision
+    assert numpy.max(numpy.abs(be.get_state() - want) / numpy.abs(want)) < 4 * len(lens) * 2.3e-16 + 2 * eps
+    be.close()
 
 
 def test_a_real_feed_takes_no_more_device_memory_than_a_complex_one():

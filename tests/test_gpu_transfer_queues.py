@@ -83,6 +83,27 @@ def test_a_copy_does_not_wait_for_another_states_queue(what):
         b.close()
 
 
+def test_fed_initialisations_do_not_wait_for_their_own_queue():
+    """Ten of them behind queued work: each is one copy, and all of them return before the work is done."""
+    a, work = busy_state()
+    rng = numpy.random.default_rng(4)
+    feeds = [rng.standard_normal(2) + (0 if q % 2 else 1j * rng.standard_normal(2)) for q in range(28)]
+    feeds = [f / numpy.linalg.norm(f) for f in feeds]
+    groups = [[q] for q in range(28)]
+    work()
+    for _ in range(10):
+        a.reinit(groups, feeds)
+    t = time.perf_counter()
+    a.synchronize()
+    assert time.perf_counter() - t > 0.1
+    want = numpy.ones(1, dtype=numpy.complex128)
+    for f in feeds[14:]:
+        want = numpy.kron(want, f)
+    lead = numpy.prod([f[0] for f in feeds[:14]])
+    assert numpy.max(numpy.abs(a.get_relative_range(0, 2 ** 14) - lead * want)) < 1e-15
+    a.close()
+
+
 def test_more_uploads_behind_one_queue_than_there_is_staging_memory():
     a, work = busy_state(0.3)
     work()
