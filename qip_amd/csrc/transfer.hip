@@ -1,13 +1,15 @@
 // transfer.hip -- copies between the caller's arrays and device memory, through pinned staging memory.
 //
 // The runtime's own copies of pageable memory pass through its staging buffers a piece at a time, each
-// piece waiting for the one before: 17 GB/s out of a 16 MiB state, and 113 us for 256 KiB. Here a copy is
-// cut into pieces of 1 MiB on four slots of pinned memory, so that the copy engine works on some while the
+// piece waiting for the one before: 17 GB/s out of a 16 MiB state. Here a copy is
+// cut into pieces of 1 MiB on four slots of pinned memory, so that the link works on some while the
 // processor copies others, and a copy of 8 MiB and more is shared by up to four threads: what bounds
 // a large result is the processor's first touch of the caller's fresh pages (64 MiB: 4.9 ms by one
 // thread, 2.3 by four; the link takes 1.2; shares of 1 or 2 MiB and 8 threads measured the same).
 // With real feeds crossing as real numbers: a search on a fed 24-qubit register 74.0 -> 23.3 ms, a
 // 16-qubit Fourier transform with its 1 MiB input, state and probabilities 369 -> 333 us.
+// A call, us, by the runtime's copies and here: reads of 64 KiB 13 / 13, 1 MiB 62 / 61, 16 MiB 920 / 595; uploads of
+// 64 KiB 14 / 7 (18 until they are there), 1 MiB 56 / 33 (60), 16 MiB 464 / 227 (455).
 #include <algorithm>
 #include <cstring>
 #include <mutex>
@@ -20,7 +22,31 @@
 
 namespace qipgpu {
 
+// A slot's words to device memory, read with system-scope loads, so that no cache holds an older copy of a slot
+// that is used again. In the state's own queue: a transfer by the copy engines waits for the queue's kernels
+// and they for it, some 10 us a piece (uploads waited for, us, copy engine -> here: 64 KiB 20 -> 17, 1 MiB 64 -> 60,
+// 4 MiB 170 -> 139, 16 MiB 600 -> 455). 16, 32 and 64 workgroups take 1 MiB in 80, 62 and 60 us.
+constexpr uint32_t kMoveBlocks = 64;
+
+__global__ __launch_bounds__(256) void k_move(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst, uint32_t words) {
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256)
+        dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The words of a short upload as kernel arguments: no slot, and no event that holds up the kernel behind it
+// (a small addition 22 -> 17 us with its wait).
+constexpr uint32_t kPayloadWords = 480;
+struct Payload {
+    uint64_t w[kPayloadWords];
+};
+
+__global__ __launch_bounds__(256) void k_payload(uint64_t *dst, uint32_t words, const Payload p) {
+    for (uint32_t i = threadIdx.x; i < words; i += 256) dst[i] = p.w[i];
+}
+
 namespace {
+
+bool in_words(const void *p, size_t bytes) { return !((reinterpret_cast<uintptr_t>(p) | bytes) & 7u); }
 
 constexpr int kSlots = 4;           // pieces that a thread has on their way
 constexpr int kSlotsMade = 32;      // slots a device gets at most, 32 MiB, kept for later copies
@@ -177,7 +203,22 @@ struct Part {
         const hipError_t e = hipMemcpyAsync(b->p, dev + i * kPieceBytes, piece(i), hipMemcpyDeviceToHost, st);
         return e == hipSuccess ? b->mark(st) : e;
     }
+    hipError_t put(char *to, const char *from, size_t size) {
+        if (!in_words(to, size)) return hipMemcpyAsync(to, from, size, hipMemcpyHostToDevice, st);
+        const uint32_t words = (uint32_t)(size / 8);
+        hipLaunchKernelGGL(k_move, dim3(std::min((words + 255) / 256, kMoveBlocks)), dim3(256), 0, st, (const uint64_t *)from,
+                           (uint64_t *)to, words);
+        return hipGetLastError();
+    }
     hipError_t copy_out(size_t n) {
+        if (n == 1) {
+            // an event would wait in the hardware queue, which other streams share; the stream's end is the copy's own
+            // (128 KiB 22 us with an event, 16 so; a state whose queue is empty is read past a busy one)
+            hipError_t e = hipMemcpyAsync(slot[0]->p, dev, bytes, hipMemcpyDeviceToHost, st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);
+            if (e == hipSuccess) std::memcpy(host, slot[0]->p, bytes);
+            return e;
+        }
         hipError_t e = hipSuccess;
         for (size_t i = 0; i < std::min<size_t>(n, slots) && e == hipSuccess; ++i) e = fetch(i);
         for (size_t i = 0; i < n && e == hipSuccess; ++i) {
@@ -194,7 +235,7 @@ struct Part {
             Slot *b = slot[i % slots];
             if ((e = b->wait()) != hipSuccess) break;
             std::memcpy(b->p, host + i * kPieceBytes, piece(i));
-            e = hipMemcpyAsync(dev + i * kPieceBytes, b->p, piece(i), hipMemcpyHostToDevice, st);
+            e = put(dev + i * kPieceBytes, b->p, piece(i));
             if (e == hipSuccess) e = b->mark(st);
         }
         return e;
@@ -208,6 +249,13 @@ int copy(hipStream_t st, char *host, char *dev, size_t bytes, bool out) {
     QIP_HIP(hipStreamGetDevice(st, &device));
     const OnDevice on(device);
     QIP_HIP(on.rc);
+    if (!out && bytes <= sizeof(Payload) && in_words(dev, bytes)) {
+        Payload p;
+        std::memcpy(p.w, host, bytes);
+        hipLaunchKernelGGL(k_payload, dim3(1), dim3(256), 0, st, (uint64_t *)dev, (uint32_t)(bytes / 8), p);
+        QIP_LAUNCHED();
+        return QIPGPU_OK;
+    }
     const Shares shares = shares_of(bytes);
     Part part[kCopyThreads];
     for (int i = 0; i < shares.count; ++i) {

@@ -19,7 +19,7 @@ def vector(count, seed, dtype=numpy.complex64):
     return (rng.standard_normal(count) + 1j * rng.standard_normal(count)).astype(dtype)
 
 
-@pytest.mark.parametrize("start,count", [(0, 1), (5, 3), (1, MIB - 1), (0, MIB), (7, MIB + 1), (0, 4 * MIB), (3, 4 * MIB + 5),
+@pytest.mark.parametrize("start,count", [(0, 1), (5, 3), (0, 479), (1, 480), (2, 481), (3, 482), (1, 16384), (1, 16385), (1, MIB - 1), (0, MIB), (7, MIB + 1), (0, 4 * MIB), (3, 4 * MIB + 5),
                                          (0, 5 * MIB), (1, 8 * MIB - 1), (0, 8 * MIB), (9, 12 * MIB + 3), (0, 16 * MIB),
                                          (11, 19 * MIB + 77), (0, 32 * MIB)])
 def test_ranges_arrive_whole(start, count):
