@@ -217,6 +217,7 @@ def func_table(func, n_reg1: int, cache: bool = False) -> _FuncTable:
 
 PRODUCT_MAX = 12            # single-qubit factors per product sweep (QIPGPU_MAX_PRODUCT)
 PRODUCT_LOW_BITS = 4        # lowest state bits every product sweep keeps in its tile
+SHORT_FEED = 12             # qubits of the feeds that the engine takes in one copy
 PRODUCT_MIN_QUBITS = 12     # the product sweep tiles 12 state bits
 
 
@@ -339,11 +340,13 @@ class GpuBackend(StateType):
             _capi.check(self._lib.qipgpu_init_product(self._h, 0, None, None, None), "init")
             return
         groups = [list(g) for g in index_groups][:len(feed_list)]
+        # short feeds go as one array of complex numbers: their number counts, not their bytes
+        short = bool(groups) and all(len(g) <= SHORT_FEED for g in groups)
         feeds = []
         for g, f in zip(groups, feed_list):
-            # real feeds cross the link as real numbers (half the bytes) and are widened on the device
+            # longer real ones cross the link as real numbers (half the bytes) and are widened on the device
             v = numpy.asarray(f)
-            real = v.dtype.kind in "fiub"
+            real = not short and v.dtype.kind in "fiub"
             v = numpy.ascontiguousarray(v, dtype=numpy.float64 if real else numpy.complex128).ravel()
             if v.shape[0] < 2 ** len(g):
                 raise IndexError("feed of length {} for {} qubits".format(v.shape[0], len(g)))
@@ -354,6 +357,11 @@ class GpuBackend(StateType):
             return
         glen = _capi.i32([len(g) for g in groups])
         gidx = _capi.i32([q for g in groups for q in g])
+        if short:
+            flat = numpy.concatenate(feeds).view(numpy.float64)
+            _capi.check(self._lib.qipgpu_init_product(self._h, len(groups), _capi.ptr(glen), _capi.ptr(gidx),
+                                                      _capi.ptr(flat)), "init")
+            return
         at = (ctypes.c_void_p * len(feeds))(*[v.ctypes.data for v in feeds])
         kinds = _capi.i32([v.dtype == numpy.float64 for v in feeds])
         _capi.check(self._lib.qipgpu_init_feeds(self._h, len(groups), _capi.ptr(glen), _capi.ptr(gidx), at,

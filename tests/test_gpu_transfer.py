@@ -92,6 +92,14 @@ def test_feeds_short_and_long_are_the_product_of_their_groups(lens, dtype):
     be.close()
 
 
+def test_feeds_beyond_the_groups_are_left_out():
+    one, zero = numpy.array([0.0, 1.0]), numpy.array([1.0, 0.0])
+    for groups, feeds, at in (([], [one], 0), ([[0]], [one, zero], 4), ([[2], [0]], [one, one, numpy.ones(2 ** 14)], 5)):
+        be = GpuBackend.make_state(3, groups, feeds)
+        assert numpy.array_equal(be.get_state(), numpy.arange(8) == at)
+        be.close()
+
+
 def test_a_real_feed_takes_no_more_device_memory_than_a_complex_one():
     hip = ctypes.CDLL("libamdhip64.so")
 
