@@ -533,14 +533,19 @@ int pair_pass(qipgpu_state *s, const HeldProduct &b, const std::vector<HeldGate>
     return s->dtype == QIPGPU_C128 ? launch_pair<double>(s, a) : launch_pair<float>(s, a);
 }
 
-bool finite(const HeldProduct &h) {
+// Whether factors may be multiplied together: every part of an entry is 0 or so far from the limits of FP64 that a
+// product of two neither overflows nor loses bits to underflow (and none is an infinity or a NaN, which
+// would spread). Applied in turn, factors outside this range may still leave amplitudes of ordinary size.
+bool composable(const HeldProduct &h) {
+    const auto fits = [](double x) { return x == 0.0 || (std::fabs(x) >= 0x1p-500 && std::fabs(x) <= 0x1p500); };
     for (int p : bits_of(h.bits))
         for (const cx<double> &e : h.m[p])
-            if (!std::isfinite(e.re) || !std::isfinite(e.im)) return false;
+            if (!fits(e.re) || !fits(e.im)) return false;
     return true;
 }
 
-// h := f on state bit p after what h has there, in FP64 (exact where either is a permutation). Two X cancel.
+// h := f on state bit p after what h has there, in FP64 (exact where either is a permutation), both composable. Two X
+// cancel.
 void compose(HeldProduct &h, int p, const Factor &f) {
     if (!(h.bits >> p & 1)) {
         h.bits |= 1ull << p;
@@ -597,8 +602,7 @@ extern "C" int qipgpu_apply_product(qipgpu_state *s, int32_t k, const int32_t *t
     // The product is held back: one that follows it at once is multiplied into it (its factors, 2x2 in
     // FP64), one that follows after diagonals may share a pass with it (shared_bits). On 23 of 24
     // qubits an H layer, an X layer, a controlled Z, an X layer and an H layer are 5 passes, 12 when
-    // each layer had its own. An infinity or a NaN in a factor would spread through such products, so
-    // factors that hold one meet the state by themselves.
+    // each layer had its own. Factors that are not composable meet the state by themselves.
     HeldProduct f;
     f.m.resize(s->n);
     for (int j = 0; j < k; ++j) {
@@ -609,11 +613,10 @@ extern "C" int qipgpu_apply_product(qipgpu_state *s, int32_t k, const int32_t *t
             f.m[p][e].im = mats[8 * j + 2 * e + 1];
         }
     }
-    const bool plain = finite(f);
-    if (s->after.bits ? !plain || !finite(s->after) : !s->held.empty() && (!s->before.bits || !plain)) {
+    const HeldProduct &last = s->after.bits ? s->after : s->before;
+    if ((s->before.bits || !s->held.empty()) && (!last.bits || !composable(f) || !composable(last))) {
         if ((rc = flush_held(s))) return rc;
     }
-    if (s->before.bits && s->held.empty() && (!plain || !finite(s->before)) && (rc = flush_held(s))) return rc;
     HeldProduct &h = s->before.bits && !s->held.empty() ? s->after : s->before;
     if (!h.bits) h.m.assign(s->n, Factor());
     for (int p : bits_of(f.bits)) compose(h, p, f.m[p]);

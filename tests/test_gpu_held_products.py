@@ -113,3 +113,37 @@ def test_products_of_unlike_bits_and_kinds(dtype, tol):
            layer(range(2, 9), n, u), z, layer(range(9), n, mixed), layer(range(12), n, mixed), z]
     for stop in range(1, len(seq) + 1):
         check(GpuBackend.make_state, n, seq[:stop], rng, dtype, tol)
+
+
+@pytest.mark.parametrize("between", [False, True])
+@pytest.mark.parametrize("entries,scale", [((1e200, 1e-200), 1e-300), ((1e-200, 1e200), 1e300), ((3e-160, 2.0), 1e200), ((1e300, 0.5), 1e-308),
+                                           ((numpy.inf, 1.0), 1.0)])
+def test_factors_near_the_limits_are_not_multiplied_together(entries, scale, between):
+    """What two such products leave does not depend on whether the first was held: applied in turn they keep
+    these amplitudes in range, their product would overflow or lose its bits."""
+    n = 12
+    rng = numpy.random.default_rng(3)
+    v = rng.standard_normal(2 ** n) + 1j * rng.standard_normal(2 ** n)
+    # the first qubit's halves at the scales that two applications bring back
+    v.reshape(2, -1)[0] *= scale
+    v.reshape(2, -1)[1] *= 1.0 / scale if entries[1] in (1e200, 1e-200) else 1.0
+    step = {0: numpy.diag(entries), 7: HM}
+    turn = {(0, 3): CMat(numpy.diag([1.0, 1j]))}
+    out = []
+    for flush in (True, False):
+        be = GpuBackend.make_state(n, [], [])
+        be.overwrite_relative_range(0, 2 ** n, v)
+        for d in [step] + ([turn] if between else []) + [step]:
+            be.kronselect_dot(d)
+            if flush:
+                be.flush()
+        out.append(be.get_state())
+        be.close()
+    a, b = (x.view(numpy.float64) for x in out)
+    assert numpy.array_equal(numpy.isnan(a), numpy.isnan(b)) and numpy.array_equal(numpy.isinf(a), numpy.isinf(b))
+    if numpy.isfinite(entries[0]):
+        assert numpy.isfinite(a).all() and a.any()
+    # a rounding per factor and pass, against the largest amplitude of the half (H mixes amplitudes within one)
+    for x, y in zip(a.reshape(2, -1), b.reshape(2, -1)):
+        if numpy.isfinite(x).all():
+            assert numpy.abs(x - y).max() <= 1e-14 * numpy.abs(x).max()
