@@ -11,6 +11,7 @@
 //                        three real products on FP64 MFMA (v_mfma_f64_16x16x4f64), U's fragments in
 //                        LDS. It holds every amplitude of its bases before any is written, so in place
 //                        is safe. Small states take k_dense_split, a tile by four waves.
+//   k_dense_low<R>       the same on the four lowest state bits, a tile loaded and stored in address order.
 //   k_dense_wide<R, K>   K = 7 and 8 on states of enough tiles, in place: a workgroup holds all rows of its bases
 //                        in 128 KB of LDS and forms Y on FP64 MFMA, U's fragments from the caches.
 //   k_dense_gemm<R>      other K = 7..12, out of place: a 64 x 64 output tile per workgroup over 16-column
@@ -84,10 +85,11 @@ __device__ __forceinline__ uint64_t base_of(uint64_t g, const PosList &pl, uint6
 // that a large FP64 product reaches). Per call on 2^28 amplitudes, targets low / high / scattered,
 // with the tile in LDS (four barriers a tile) before, and now; a copy takes 1.63 (complex128) and
 // 0.81 ms (complex64):
-//   complex128 K = 4 1.77 / 1.89 / 1.84 -> 1.90 / 1.66 / 1.72 ms; K = 5 1.95 / 1.77 / 1.96 -> 1.87 / 1.67 /
-//   1.78; K = 6 2.93 / 2.45 / 2.39 -> 1.75 / 1.79 / 1.76
-//   complex64 K = 4 1.40 / 1.05 / 1.05 -> 1.11 / 0.85 / 0.93; K = 5 1.95 / 1.51 / 1.51 -> 1.10 / 0.96 / 0.92;
-//   K = 6 2.93 / 2.38 / 2.38 -> 1.62 / 1.61 / 1.60
+//   complex128 K = 4 1.76 / 1.87 / 1.69 -> 1.90 / 1.66 / 1.61 ms; K = 5 1.94 / 1.76 / 1.66 -> 1.88 / 1.67 /
+//   1.72; K = 6 2.94 / 2.46 / 2.40 -> 1.74 / 1.79 / 1.82
+//   complex64 K = 4 1.39 / 1.04 / 1.04 -> 1.11 / 0.84 / 0.86; K = 5 1.95 / 1.51 / 1.51 -> 1.10 / 0.95 / 0.90;
+//   K = 6 2.95 / 2.39 / 2.39 -> 1.62 / 1.61 / 1.60
+// (K = 4 on the four lowest bits is k_dense_low's.)
 // Workgroups take tiles a grid apart: 1.66 against 1.74 ms (K = 4, high targets) with contiguous ranges.
 template <int K>
 struct MfmaShape {
@@ -198,6 +200,91 @@ __global__ __launch_bounds__(kTileThreads, 2) void k_dense_mfma(const DenseTileA
     };
     // two register buffers alternate (the last prefetch re-reads an in-range tile and is not used)
     cx<R> xa[16], xb[16];
+    load(xa, t);
+    for (;;) {
+        const uint64_t t1 = t + step, t2 = t1 + step;
+        load(xb, min(t1, end - 1));
+        process(xa, t);
+        if (t1 >= end) return;
+        load(xa, min(t2, end - 1));
+        process(xb, t1);
+        if (t2 >= end) return;
+        t = t2;
+    }
+}
+
+// Four targets on the four lowest state bits: a base is 16 amplitudes in a row, and k_dense_mfma's lanes, 16 along the
+// bases, would touch 16 B of a line each. Here a wave loads and stores its tile in address order and turns it
+// through LDS of its own (slots of 16 amplitudes padded by one), so there is still no barrier in the loop.
+// Bound: HBM. A call, by k_dense_mfma and here: 2^28 amplitudes complex128 1908 -> 1690 us, complex64 1110 -> 863; 2^26 481
+// -> 430 and 286 -> 218; 2^24 77 -> 78 and 66 -> 52; 2^22 30 -> 31 and 27 -> 24. One bit higher k_dense_mfma takes 1690
+// and 836 at 2^28; on 5 of the lowest bits its runs are 128 B and more in complex128 (1877).
+template <typename R>
+__global__ __launch_bounds__(kTileThreads, 2) void k_dense_low(const DenseTileArgs<R, 4> a, const f64x2 *__restrict__ frag) {
+    using M = MfmaShape<4>;
+    // an amplitude as a vector: structs copied from memory to LDS went through scratch memory
+    typedef R Amp __attribute__((ext_vector_type(2)));
+    __shared__ f64x2 sU[M::KS * 64];
+    __shared__ Amp turn[kTileWaves][1024 + 64];
+    for (int e = threadIdx.x; e < M::KS * 64; e += kTileThreads) sU[e] = frag[e];
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // amplitude 64 j + lane of the tile is row lane % 16 of base 4 j + lane / 16
+    Amp *const line = &turn[wave][17 * (lane >> 4) + (lane & 15)];             // + 68 j
+    Amp *const cell = &turn[wave][17 * (lane & 15) + (lane >> 4)];             // base 16 c + lane % 16, row 4 s + lane / 16: + 272 c + 4 s
+    const uint64_t at = insert_zeros((uint64_t)(lane >> 4), a.pl) + a.row_k[0] + (lane & 15);
+    uint64_t base[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) base[j] = insert_zeros(4ull * j, a.pl);
+    f64x2 u[M::KS];
+#pragma unroll
+    for (int s = 0; s < M::KS; ++s) u[s] = sU[s * 64 + lane];
+    const uint64_t step = (uint64_t)gridDim.x * kTileWaves, end = a.ntiles;
+    uint64_t t = (uint64_t)blockIdx.x * kTileWaves + wave;
+    if (t >= end) return;
+    // the wave's LDS accesses are carried out in order: only the compiler has to keep theirs
+    auto in_order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    Amp *const amps = reinterpret_cast<Amp *>(a.amps) + at;
+    auto tile_at = [&](uint64_t tile) { return amps + insert_zeros(tile * M::BASES, a.pl); };
+    auto load = [&](Amp (&x)[16], uint64_t tile) {
+        const Amp *p = tile_at(tile);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) x[j] = p[base[j]];
+    };
+    auto process = [&](const Amp (&x)[16], uint64_t tile) {
+        Amp *p = tile_at(tile);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) line[68 * j] = x[j];
+        in_order();
+#pragma unroll
+        for (int c = 0; c < M::CB; ++c) {
+            f64x4 acc[3];
+#pragma unroll
+            for (int m = 0; m < 3; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int s = 0; s < M::KS; ++s) {
+                const Amp v = cell[272 * c + 4 * s];
+                const double re = v.x, im = v.y;
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s][0], re, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s][1], im, acc[1], 0, 0, 0);
+                acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(u[s][0] + u[s][1], re + im, acc[2], 0, 0, 0);
+            }
+            // row 4 i + lane / 16: the cells this lane read
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                cell[272 * c + 4 * i] = Amp{(R)(acc[0][i] - acc[1][i]), (R)(acc[2][i] - acc[0][i] - acc[1][i])};
+            }
+        }
+        in_order();
+#pragma unroll
+        for (int j = 0; j < 16; ++j) p[base[j]] = line[68 * j];
+        in_order();
+    };
+    Amp xa[16], xb[16];
     load(xa, t);
     for (;;) {
         const uint64_t t1 = t + step, t2 = t1 + step;
@@ -660,6 +747,13 @@ int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
         return QIPGPU_OK;
     }
     const uint64_t grid = std::min<uint64_t>((a.ntiles + kTileWaves - 1) / kTileWaves, (uint64_t)device_cus() * 2);
+    if constexpr (K == 4) {
+        if (*std::max_element(tbits.begin(), tbits.end()) == 3) {      // the lowest four: figures at the kernel
+            hipLaunchKernelGGL(k_dense_low<R>, dim3((uint32_t)grid), dim3(kTileThreads), 0, s->stream, a, (const f64x2 *)d);
+            QIP_LAUNCHED();
+            return QIPGPU_OK;
+        }
+    }
     hipLaunchKernelGGL((k_dense_mfma<R, K>), dim3((uint32_t)grid), dim3(kTileThreads), 0, s->stream, a,
                        (const f64x2 *)d);
     QIP_LAUNCHED();
