@@ -8,7 +8,7 @@
 // thread, 2.3 by four; the link takes 1.2; shares of 1 or 2 MiB and 8 threads measured the same).
 // With real feeds crossing as real numbers: a search on a fed 24-qubit register 74.0 -> 23.3 ms, a
 // 16-qubit Fourier transform with its 1 MiB input, state and probabilities 369 -> 333 us.
-// A call, us, by the runtime's copies and here: reads of 64 KiB 13 / 13, 1 MiB 62 / 61, 16 MiB 920 / 595; uploads of
+// A call, us, by the runtime's copies and here: reads of 64 KiB 13 / 13, 1 MiB 62 / 61, 16 MiB 920 / 475; uploads of
 // 64 KiB 14 / 7 (18 until they are there), 1 MiB 56 / 33 (60), 16 MiB 464 / 227 (455).
 #include <algorithm>
 #include <cstring>
@@ -22,15 +22,20 @@
 
 namespace qipgpu {
 
-// A slot's words to device memory, read with system-scope loads, so that no cache holds an older copy of a slot
-// that is used again. In the state's own queue: a transfer by the copy engines waits for the queue's kernels
-// and they for it, some 10 us a piece (uploads waited for, us, copy engine -> here: 64 KiB 20 -> 17, 1 MiB 64 -> 60,
-// 4 MiB 170 -> 139, 16 MiB 600 -> 455). 16, 32 and 64 workgroups take 1 MiB in 80, 62 and 60 us.
+// Words between a slot and device memory, the host's with system scope: no cache holds an older copy of a slot that
+// is used again, and what is written there does not stay in one. In the state's own queue: a transfer by the copy
+// engines waits for the queue's kernels and they for it, some 10 us a piece (uploads waited for, us, copy engine ->
+// here: 64 KiB 20 -> 17, 1 MiB 64 -> 60, 4 MiB 170 -> 139, 16 MiB 600 -> 455), and of several pieces of a read from
+// two threads each took 150 us in some processes (8 MiB 1330 us, 450 to 510 so; 16 MiB 600 -> 475). 16, 32
+// and 64 workgroups upload 1 MiB in 80, 62 and 60 us.
 constexpr uint32_t kMoveBlocks = 64;
 
+template <bool OUT>
 __global__ __launch_bounds__(256) void k_move(const uint64_t *__restrict__ src, uint64_t *__restrict__ dst, uint32_t words) {
-    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256)
-        dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    for (uint32_t i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) {
+        if constexpr (OUT) __hip_atomic_store(dst + i, src[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        else dst[i] = __hip_atomic_load(src + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
 // The words of a short upload as kernel arguments: no slot, and no event that holds up the kernel behind it
@@ -198,17 +203,19 @@ struct Part {
     }
     size_t pieces() const { return (bytes + kPieceBytes - 1) / kPieceBytes; }
     size_t piece(size_t i) const { return std::min(kPieceBytes, bytes - i * kPieceBytes); }
+    hipError_t move(char *to, const char *from, size_t size) const {
+        if (!in_words(to, size) || !in_words(from, 0))
+            return hipMemcpyAsync(to, from, size, out ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, st);
+        const uint32_t words = (uint32_t)(size / 8);
+        const dim3 grid(std::min((words + 255) / 256, kMoveBlocks));
+        if (out) hipLaunchKernelGGL(k_move<true>, grid, dim3(256), 0, st, (const uint64_t *)from, (uint64_t *)to, words);
+        else hipLaunchKernelGGL(k_move<false>, grid, dim3(256), 0, st, (const uint64_t *)from, (uint64_t *)to, words);
+        return hipGetLastError();
+    }
     hipError_t fetch(size_t i) {
         Slot *b = slot[i % slots];
-        const hipError_t e = hipMemcpyAsync(b->p, dev + i * kPieceBytes, piece(i), hipMemcpyDeviceToHost, st);
+        const hipError_t e = move(b->p, dev + i * kPieceBytes, piece(i));
         return e == hipSuccess ? b->mark(st) : e;
-    }
-    hipError_t put(char *to, const char *from, size_t size) {
-        if (!in_words(to, size)) return hipMemcpyAsync(to, from, size, hipMemcpyHostToDevice, st);
-        const uint32_t words = (uint32_t)(size / 8);
-        hipLaunchKernelGGL(k_move, dim3(std::min((words + 255) / 256, kMoveBlocks)), dim3(256), 0, st, (const uint64_t *)from,
-                           (uint64_t *)to, words);
-        return hipGetLastError();
     }
     hipError_t copy_out(size_t n) {
         if (n == 1) {
@@ -235,7 +242,7 @@ struct Part {
             Slot *b = slot[i % slots];
             if ((e = b->wait()) != hipSuccess) break;
             std::memcpy(b->p, host + i * kPieceBytes, piece(i));
-            e = put(dev + i * kPieceBytes, b->p, piece(i));
+            e = move(dev + i * kPieceBytes, b->p, piece(i));
             if (e == hipSuccess) e = b->mark(st);
         }
         return e;
