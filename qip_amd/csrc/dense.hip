@@ -698,17 +698,15 @@ PosList poslist(std::vector<int> pos) {
     return pl;
 }
 
-// The arguments (DenseTileArgs, DenseWideArgs) and U's fragments of a kernel that numbers the rows in
-// state-bit order: bit b of a row is the b-th lowest target bit.
+// The arguments (DenseTileArgs, DenseWideArgs) of a kernel that numbers the rows in state-bit order: bit b of a
+// row is the b-th lowest target bit. caller[j]: row j's place in the caller's index.
 template <typename M, typename A>
-std::vector<std::complex<double>> tile_arguments(A &a, qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask,
-                                                 const std::vector<int> &allpos, const std::complex<double> *U) {
-    constexpr int D = M::D;
+void tile_arguments(A &a, int (&caller)[M::D], qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask,
+                    const std::vector<int> &allpos) {
     const int K = (int)tbits.size();
     std::vector<int> sorted(tbits);
     std::sort(sorted.begin(), sorted.end());
-    int caller[D];      // a row's place in the caller's index
-    for (int j = 0; j < D; ++j) {
+    for (int j = 0; j < M::D; ++j) {
         caller[j] = 0;
         for (int t = 0; t < K; ++t) {
             const int b = (int)(std::find(sorted.begin(), sorted.end(), tbits[t]) - sorted.begin());
@@ -724,19 +722,25 @@ std::vector<std::complex<double>> tile_arguments(A &a, qipgpu_state *s, const st
         a.row_k[j] = ctrl_mask + ((uint64_t)(j & 1) << sorted[0]) + ((uint64_t)(j >> 1) << sorted[1]);
     for (int j = 0; j < M::KS; ++j)
         for (int b = 2; b < K; ++b) a.row_s[j] += (uint64_t)(j >> (b - 2) & 1) << sorted[b];
-    std::vector<std::complex<double>> frag((size_t)D * D);
+}
+
+// U's fragments for such a kernel, D x D entries: [k-step][row block][lane].
+template <typename M>
+void fragments(std::complex<double> *out, const int (&caller)[M::D], const std::complex<double> *U) {
     for (int st = 0; st < M::KS; ++st)
         for (int rb = 0; rb < M::RB; ++rb)
             for (int l = 0; l < 64; ++l)
-                frag[(size_t)(st * M::RB + rb) * 64 + l] = U[(size_t)caller[16 * rb + l % 16] * D + caller[4 * st + l / 16]];
-    return frag;
+                out[(size_t)(st * M::RB + rb) * 64 + l] = U[(size_t)caller[16 * rb + l % 16] * M::D + caller[4 * st + l / 16]];
 }
 
 template <typename R, int K>
 int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<int> &allpos,
                 const std::complex<double> *U) {
     DenseTileArgs<R, K> a;
-    const std::vector<std::complex<double>> frag = tile_arguments<MfmaShape<K>>(a, s, tbits, ctrl_mask, allpos, U);
+    int caller[1 << K];
+    tile_arguments<MfmaShape<K>>(a, caller, s, tbits, ctrl_mask, allpos);
+    std::vector<std::complex<double>> frag((size_t)1 << 2 * K);
+    fragments<MfmaShape<K>>(frag.data(), caller, U);
     void *d = nullptr;
     int rc = ring_upload(s, frag.data(), frag.size() * sizeof(frag[0]), &d);
     if (rc) return rc;
@@ -763,13 +767,13 @@ int launch_tile(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
 // Temporaries of wide dense operators up to this size stay with the state for the next call.
 constexpr size_t kKeepGemmTmpBytes = size_t(1) << 30;
 
-// The offsets and U of a wide dense operator into the state's operator buffer, on its queue: through
+// `need` bytes of a wide dense operator into the state's operator buffer, on its queue: `fill` writes them to
 // pinned memory, so the copy is asynchronous and the queue is not drained first. The pinned buffer is
 // rewritten only once the previous copy out of it has run; the device buffer is rewritten in queue
-// order, after the kernels that read it.
-int stage_gemm_operator(qipgpu_state *s, const std::vector<uint64_t> &off, const std::complex<double> *U, size_t D,
-                        void **dev) {
-    const size_t ob = off.size() * sizeof(uint64_t), ub = D * D * sizeof(cx<double>), need = ob + ub;
+// order, after the kernels that read it. (Fragments go straight to the pinned buffer: by an array of their own, 1 MiB
+// of fresh pages, a waited-for call of K = 8 on 22 qubits took 290 us, 244 so; the GEMM 239.)
+template <typename F>
+int stage_gemm_operator(qipgpu_state *s, size_t need, F fill, void **dev) {
     if (!s->gemm_ev) QIP_HIP(hipEventCreateWithFlags(&s->gemm_ev, hipEventDisableTiming));
     else QIP_HIP(hipEventSynchronize(s->gemm_ev));
     if (s->h_gemm_op_bytes < need) {
@@ -787,8 +791,7 @@ int stage_gemm_operator(qipgpu_state *s, const std::vector<uint64_t> &off, const
         QIP_HIP(hipMalloc(&s->d_gemm_op, need));
         s->d_gemm_op_bytes = need;
     }
-    std::memcpy(s->h_gemm_op, off.data(), ob);
-    std::memcpy((char *)s->h_gemm_op + ob, U, ub);
+    fill(static_cast<char *>(s->h_gemm_op));
     QIP_HIP(hipMemcpyAsync(s->d_gemm_op, s->h_gemm_op, need, hipMemcpyHostToDevice, s->stream));
     QIP_HIP(hipEventRecord(s->gemm_ev, s->stream));
     *dev = s->d_gemm_op;
@@ -796,17 +799,22 @@ int stage_gemm_operator(qipgpu_state *s, const std::vector<uint64_t> &off, const
 }
 
 // From this many tiles on k_dense_wide is used: a workgroup's waves have D / 4 k-steps of a whole tile before
-// them, where the GEMM spreads a small state's rows over workgroups. K = 7, us a call: 64 tiles (19 qubits)
-// 59 against the GEMM's 57, 128 tiles 61 / 63, 256 63 / 75; K = 8: 256 tiles (21 qubits) 134 / 119, 512 163 / 182.
-constexpr uint64_t kWideTiles7 = 128, kWideTiles8 = 512;
+// them, where the GEMM spreads a small state's rows over workgroups, and its fragments cost the host more than
+// a copy of U. GEMM / k_dense_wide, complex128, targets low, us a call among others and a call waited for: K = 7
+// 128 tiles (20 qubits) 63 / 62 and 77 / 82, 256 77 / 65 and 91 / 84; K = 8 256 tiles (21 qubits) 119 / 134,
+// 512 187 / 160 and 239 / 244. complex64: 62 / 61 and 76 / 80, 77 / 61 and 90 / 80; 512 tiles 196 / 154 and 248 / 241.
+constexpr uint64_t kWideTiles7 = 256, kWideTiles8 = 512;
 
 template <typename R, int K>
 int launch_wide(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_mask, const std::vector<int> &allpos,
                 const std::complex<double> *U) {
     DenseWideArgs<R, K> a;
-    const std::vector<std::complex<double>> frag = tile_arguments<WideShape<K>>(a, s, tbits, ctrl_mask, allpos, U);
+    int caller[1 << K];
+    tile_arguments<WideShape<K>>(a, caller, s, tbits, ctrl_mask, allpos);
     void *d = nullptr;
-    const int rc = stage_gemm_operator(s, {}, frag.data(), WideShape<K>::D, &d);
+    const int rc = stage_gemm_operator(s, sizeof(std::complex<double>) << 2 * K, [&](char *to) {
+        fragments<WideShape<K>>(reinterpret_cast<std::complex<double> *>(to), caller, U);
+    }, &d);
     if (rc) return rc;
     const uint32_t grid = (uint32_t)std::min<uint64_t>(a.ntiles, (uint64_t)device_cus());
     hipLaunchKernelGGL((k_dense_wide<R, K>), dim3(grid), dim3(512), 0, s->stream, a, (const f64x2 *)d);
@@ -821,7 +829,11 @@ int launch_gemm(qipgpu_state *s, const std::vector<int> &tbits, uint64_t ctrl_ma
     const int D = 1 << K;
     const std::vector<uint64_t> off = offsets(tbits);
     void *op = nullptr;
-    int rc = stage_gemm_operator(s, off, U, (size_t)D, &op);
+    const size_t ob = off.size() * sizeof(uint64_t), ub = (size_t)D * D * sizeof(cx<double>);
+    int rc = stage_gemm_operator(s, ob + ub, [&](char *to) {
+        std::memcpy(to, off.data(), ob);
+        std::memcpy(to + ob, U, ub);
+    }, &op);
     if (rc) return rc;
     const uint64_t nbase = s->len >> allpos.size();
     // the compact temporary: the state's kept one when small, else one for this call
