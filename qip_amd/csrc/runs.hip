@@ -945,6 +945,11 @@ int launch_exchange(qipgpu_state *s, const std::vector<HeldGate> &swaps) {
 // and a launch per gate.
 constexpr uint64_t kLaunchCostAmps = 1ull << 19;
 
+// A swap alone moves half of the amplitudes by either kernel: on states that the caches (256 MiB) hold in good part
+// k_exchange is the faster, beyond them the sweep of its own. High bits, us, sweep / k_exchange: complex128 256 MiB
+// 87 / 68, 512 MiB 196 / 121, 1 GiB 422 / 441, 4 GiB 1540 / 1642; complex64 512 MiB 195 / 135, 1 GiB 373 / 438, 2 GiB 774 / 832.
+constexpr uint64_t kLoneSwapBytes = 512ull << 20;
+
 // Take the next pass's gates out of the held ones and apply them: as one exchange of bits, as one pass over
 // the tiles, as one sweep over the amplitudes that share the controls every gate has (diagonals only), or gate by gate
 // where that moves fewer amplitudes.
@@ -961,7 +966,8 @@ int apply_next(qipgpu_state *s) {
         else s->held[w++] = s->held[i];
     }
     s->held.resize(w);
-    if (exchange) return s->dtype == QIPGPU_C128 ? launch_exchange<double>(s, gates) : launch_exchange<float>(s, gates);
+    if (exchange && (gates.size() > 1 || s->len * s->amp_bytes <= kLoneSwapBytes))
+        return s->dtype == QIPGPU_C128 ? launch_exchange<double>(s, gates) : launch_exchange<float>(s, gates);
     uint64_t common = ~0ull, separate = 0;
     bool diagonal = true;
     for (const HeldGate &g : gates) {

@@ -7,6 +7,7 @@ import pytest
 
 from oracle.oracle_backend import OracleBackend
 from qip_amd import CMat, GpuBackend, SwapMat
+from qip_amd.backend import max_abs_diff
 
 pytestmark = pytest.mark.gpu
 HM = numpy.array([[1.0, 1.0], [1.0, -1.0]]) / numpy.sqrt(2.0)
@@ -125,3 +126,25 @@ def test_swaps_that_move_together(n, dtype):
     seq += [{(2, 4): CMat(XM)}, sw(2, 3), sw(4, n - 1), {4: HM}, {(n - 2, n - 3): numpy.diag([1, 1j, -1, 1.0])}, sw(n - 2, 0)]
     print("swaps n", n, numpy.dtype(dtype).name, flush=True)
     check(n, dtype, seq, rng, dtype == numpy.complex128 and n <= 13)
+
+
+@pytest.mark.parametrize("n,dtype", [(25, numpy.complex128), (26, numpy.complex128), (26, numpy.complex64), (27, numpy.complex64)])
+def test_a_swap_alone_on_either_side_of_the_caches(n, dtype):
+    """512 MiB and 1 GiB: swaps each by itself against the same ones together."""
+    rng = numpy.random.default_rng(n)
+    groups = [list(range(0, n, 2)), list(range(1, n, 2))]
+    feeds = [rng.standard_normal(2 ** len(g)) + 1j * rng.standard_normal(2 ** len(g)) for g in groups]
+    states = [GpuBackend.make_state(n, groups, feeds, statetype=dtype) for _ in range(2)]
+    swaps = [(0, 1), (2, n - 5), (n // 2, 5)]
+    for a, b in swaps:
+        states[0].kronselect_dot({(a, b): SwapMat(1)})
+        states[1].kronselect_dot({(a, b): SwapMat(1)})
+        states[1].synchronize()
+    assert max_abs_diff(*states) == 0.0
+    for a, b in swaps[::-1]:
+        states[0].kronselect_dot({(b, a): SwapMat(1)})
+        states[0].flush()
+    states[1].reinit(groups, feeds)
+    assert max_abs_diff(*states) == 0.0
+    for s in states:
+        s.close()
