@@ -549,14 +549,21 @@ __global__ __launch_bounds__(256) void k_tile_thin(const TileRunArgs<R> a) {
     }
 }
 
-// States of up to 19 qubits take the thin kernel. Graphs of a Fourier transform / of 8 layers of a random
-// circuit in complex128, us a launch, wide -> thin: 13 qubits 86 / 153 -> 54 / 96, 16 124 / 190 -> 74 / 122,
-// 18 146 / 232 -> 97 / 176, 19 170 / 280 -> 136 / 263; 20 196 / 316 -> 215 / 342 (its 1024 tiles fill the
-// GPU, and a pass's instructions for four amplitudes count again).
+// States of up to 19 qubits take the thin kernel, but for one kind of pass on 19. Graphs of a Fourier transform / of 8 layers of a random circuit, us a
+// launch, wide -> thin: complex128 10 qubits 56 / 107 -> 37 / 64, 13 80 / 149 -> 53 / 95, 16 110 / 184 -> 71 / 122, 18 127 / 226
+// -> 86 / 176, 19 154 / 275 -> 127 / 265, 20 177 / 311 -> 203 / 356 (its 1024 tiles fill the GPU, and a pass's instructions
+// for four amplitudes count again); complex64 10 52 / 108 -> 36 / 61, 13 75 / 154 -> 48 / 99, 16 104 / 191 -> 63 / 124, 18 121 /
+// 222 -> 75 / 163, 19 142 / 251 -> 110 / 232, 20 157 / 289 -> 176 / 367. On 19 qubits passes of nothing but single-qubit
+// operators, a move through LDS for every other one, are the wide kernel's: a layer of them 47 / 43 us thin and 38 to 41 /
+// 35 to 38 wide (complex128 / complex64), while swaps, phases and controlled gates are the thin one's (19 phases 20 / 19 and
+// 25 / 25).
 constexpr int kThinQubits = 19;
 
 Shape shape_of(const qipgpu_state *s) {
-    return s->n > kThinQubits ? kWide : kThin;
+    if (s->n != kThinQubits) return s->n > kThinQubits ? kWide : kThin;
+    for (const HeldGate &g : s->held)
+        if (g.kind != HeldGate::kSingle || g.ctrl_mask) return kThin;
+    return kWide;
 }
 
 // Exchanges of state bits, all at once: amplitude i and amplitude P(i) change places, P the permutation of
@@ -744,9 +751,8 @@ void plan_pass(const Shape &sh, int n, const std::vector<HeldGate> &held, std::v
 }
 
 template <typename R>
-int launch_pass(qipgpu_state *s, const std::vector<HeldGate> &gates) {
+int launch_pass(qipgpu_state *s, const Shape &shape, const std::vector<HeldGate> &gates) {
     const int n = s->n;
-    const Shape shape = shape_of(s);
     TileRunArgs<R> a;
     std::memset(&a, 0, sizeof(a));
     a.amps = (cx<R> *)s->amps;
@@ -992,7 +998,7 @@ int apply_next(qipgpu_state *s) {
         }
         return QIPGPU_OK;
     }
-    return s->dtype == QIPGPU_C128 ? launch_pass<double>(s, gates) : launch_pass<float>(s, gates);
+    return s->dtype == QIPGPU_C128 ? launch_pass<double>(s, shape, gates) : launch_pass<float>(s, shape, gates);
 }
 
 }  // namespace

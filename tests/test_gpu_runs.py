@@ -148,3 +148,15 @@ def test_a_swap_alone_on_either_side_of_the_caches(n, dtype):
     assert max_abs_diff(*states) == 0.0
     for s in states:
         s.close()
+
+
+@pytest.mark.parametrize("dtype", [numpy.complex128, numpy.complex64])
+@pytest.mark.parametrize("n", [18, 19, 20])
+def test_layers_of_single_qubit_operators_around_the_size_where_tiles_change(n, dtype):
+    """Layers of nothing else (on 19 qubits tiles of 4096), with a phase at the end of one (tiles of 1024), and between
+    gates under controls."""
+    rng = numpy.random.default_rng(1900 + n)
+    layer = lambda m: [{int(q): m()} for q in rng.permutation(n)]    # noqa: E731
+    seq = layer(lambda: unitary(rng)) + layer(lambda: HM) + layer(lambda: XM)
+    seq += [{3: numpy.diag([1.0, 1j])}] + layer(lambda: unitary(rng)) + [{(n - 1, 4): CMat(XM)}] + layer(lambda: XM) * 5
+    check(n, dtype, seq, rng, False)
