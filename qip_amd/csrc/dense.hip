@@ -128,18 +128,12 @@ __global__ __launch_bounds__(kTileThreads, 2) void k_dense_mfma(const DenseTileA
     for (int e = threadIdx.x; e < NF; e += kTileThreads) sU[e] = frag[e];
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // this lane's part of its bases' positions; lanes past the last base work on an earlier one and
-    // store nothing (there is one tile then)
+    // this lane's part of its bases' positions (every tile is full: there are more than kSplitTiles)
     uint64_t at[M::CB];
-    bool stored[M::CB];
+    const int kap = lane >> 4;
+    const uint64_t row = kap & 2 ? (kap & 1 ? a.row_k[3] : a.row_k[2]) : (kap & 1 ? a.row_k[1] : a.row_k[0]);
 #pragma unroll
-    for (int c = 0; c < M::CB; ++c) {
-        const uint64_t g = 16 * c + (lane & 15);
-        stored[c] = g < a.nbase;
-        const int kap = lane >> 4;
-        const uint64_t row = kap & 2 ? (kap & 1 ? a.row_k[3] : a.row_k[2]) : (kap & 1 ? a.row_k[1] : a.row_k[0]);
-        at[c] = insert_zeros(g & (a.nbase - 1), a.pl) + row;
-    }
+    for (int c = 0; c < M::CB; ++c) at[c] = insert_zeros((uint64_t)(16 * c + (lane & 15)), a.pl) + row;
     const uint64_t step = (uint64_t)gridDim.x * kTileWaves, end = a.ntiles;
     uint64_t t = (uint64_t)blockIdx.x * kTileWaves + wave;
     if (t >= end) return;
@@ -194,7 +188,8 @@ __global__ __launch_bounds__(kTileThreads, 2) void k_dense_mfma(const DenseTileA
                             cx<double> y;
                             y.re = t1 - t2;
                             y.im = acc[2][r][c][i] - t1 - t2;
-                            if (stored[c0 + c]) p[at[c0 + c] + a.row_s[4 * (r0 + r) + i]] = from_d<R>(y);
+                            __builtin_amdgcn_sched_barrier(0);   // kept apart: K = 6, complex64, 1.620 ms scheduled freely, 1.602 so
+                            p[at[c0 + c] + a.row_s[4 * (r0 + r) + i]] = from_d<R>(y);
                         }
             }
     };
@@ -386,8 +381,7 @@ __global__ __launch_bounds__(512) void k_dense_wide(const DenseWideArgs<R, K> a,
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kap = lane >> 4, rho = lane & 15;
     const uint64_t row = kap & 2 ? (kap & 1 ? a.row_k[3] : a.row_k[2]) : (kap & 1 ? a.row_k[1] : a.row_k[0]);
-    // bases past the last (a state of one tile): their lanes work on an earlier one and store nothing
-    auto base_at = [&](int c) { return insert_zeros((uint64_t)(16 * c + rho) & (a.nbase - 1), a.pl) + row; };
+    auto base_at = [&](int c) { return insert_zeros((uint64_t)(16 * c + rho), a.pl) + row; };
     // this wave loads 16 k-steps' rows of one column block
     constexpr int kPerBlock = M::WAVES / M::CB;
     const int lc = wave / kPerBlock, ls = wave % kPerBlock * 16;
@@ -453,7 +447,6 @@ __global__ __launch_bounds__(512) void k_dense_wide(const DenseWideArgs<R, K> a,
         cx<R> *p = tile_at(tile);
 #pragma unroll
         for (int c = 0; c < M::CB; ++c) {
-            if ((uint64_t)(16 * c + rho) >= a.nbase) continue;
             cx<R> *pc = p + base_at(c);
 #pragma unroll
             for (int r = 0; r < M::NR; ++r)
