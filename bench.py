@@ -24,9 +24,9 @@ Beside it, in the same run:
     the reference's -O3 -ffast-math -fopenmp flags, all visible cores) on a time-bounded sample of
     the circuit's own gates at full size, extrapolated to the circuit's gate mix.
 
-The default run then measures every other configuration in the same process and nests each under
-"configs" in the same JSON line, with its own rate, the roofline of its dominant kernel, a bounded
-CPU baseline (--config-cpu-seconds of work) and its error figures: qft16 (16-qubit QFT graph),
+The default run then measures every other configuration in the same process and puts the rate, the roofline of
+the dominant kernel and the CPU baseline (--config-cpu-seconds of work) of each under "configs" in the same
+JSON line; its whole entry, with its cases and error figures, goes to stderr as a line of its own: qft16 (16-qubit QFT graph),
 circuit28 (28-qubit depth-20 circuit, plain complex128 vs unfused complex64), grover24 (24-qubit
 Grover search in both forms), batch512 (512 uneven circuits in the batching form), measure28
 (marginal probabilities, norm and measurement on a 28-qubit complex128 state), func28 (func_apply
@@ -1101,6 +1101,26 @@ def bench_circuit30(args):
 SECONDARY = (("qft16", "bench_qft16"), ("circuit28", "bench_circuit28"), ("grover24", "bench_grover24"),
              ("batch512", "bench_batch512"), ("measure28", "bench_measure28"), ("func28", "bench_func28"),
              ("dense28", "bench_dense28"))
+# What the result line keeps of a configuration besides its headline run: the whole entry goes to stderr, so that the
+# line stays a few kilobytes.
+_SUMMARY = {"metric": None, "value": None, "unit": None, "ms_per_step": None, "steps": None, "dtype": None, "wall_s": None,
+            "roofline": ("bound", "achieved", "peak", "unit", "frac"), "cpu_baseline": ("value", "unit", "cores", "kind")}
+
+
+def summary(entry):
+    def short(v):
+        return float("{:.6g}".format(v)) if isinstance(v, float) else v
+
+    out = {}
+    for key, inner in _SUMMARY.items():
+        v = entry.get(key)
+        if inner and isinstance(v, dict):
+            out[key] = {k: short(v[k]) for k in inner if k in v}
+        elif v is not None:
+            out[key] = short(v)
+    return out
+
+
 _LINE_ONLY = ("n_gpus", "higher_is_better", "scaling", "vs_baseline", "data")
 
 
@@ -1123,8 +1143,8 @@ def main():
     ap.add_argument("--workload", default="all",
                     choices=["all", "circuit30", "circuit28", "grover24", "qft16", "batch512", "measure28", "func28",
                              "dense28", "product24"],
-                    help="all (default): the headline, then every other configuration nested under 'configs' in the "
-                         "same JSON line; or one workload alone, as its own JSON line")
+                    help="all (default): the headline, then every other configuration, its figures under 'configs' in the "
+                         "same JSON line and its whole entry on stderr; or one workload alone, as its own JSON line")
     ap.add_argument("--case", choices=sorted(PRODUCT_CASES), default=None,
                     help="product24 only: one case, complex64 at 24 qubits (for counter runs)")
     args = ap.parse_args()
@@ -1149,8 +1169,9 @@ def main():
             line = globals()[fn](sub)
             entry = {k: v for k, v in line.items() if k not in _LINE_ONLY}
             entry["wall_s"] = time.perf_counter() - t
-            configs[name] = entry
+            configs[name] = summary(entry)
             log("config {}: {:.4g} {} in {:.1f} s".format(name, line["value"], line["unit"], entry["wall_s"]))
+            log("config {}: {}".format(name, json.dumps(entry)))
         result["configs"] = configs
     if args.copy_calibration_gib > 0:
         copy_calibration(HipEvents(), int(args.copy_calibration_gib * 2 ** 30))
