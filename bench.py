@@ -65,20 +65,20 @@ FUSED6_PMC_30Q = {"fetch_kib": 4196076.3, "fetch_scale": 1048576.0 / 524314.6,
 
 # HBM traffic of one k_marg_pass launch on a 28-qubit complex128 state (4 GiB), measured the same way
 # by two rocprofv3 --pmc runs of `bench.py --workload measure28 --no-cpu-baseline
-# --copy-calibration-gib 1` (mean over the 42 launches of the run; FETCH_SIZE reads 524313.75 KiB for
+# --copy-calibration-gib 1` (mean over the 42 launches of the run; FETCH_SIZE reads 524314.2 KiB for
 # the 1 GiB copy, WRITE_SIZE 1048576 KiB). Commands and figures: profiles/k_marg_pass_measure28.txt.
-MARG_PMC_28Q = {"fetch_kib": 2097182.76, "fetch_scale": 1048576.0 / 524313.75,
-                "write_kib": 3026.64, "write_scale": 1.0}
+MARG_PMC_28Q = {"fetch_kib": 2097230.9, "fetch_scale": 1048576.0 / 524314.2,
+                "write_kib": 718.0, "write_scale": 1.0}
 
 
 # HBM traffic of one k_tile_run pass (a held run of single-qubit gates) on a 28-qubit complex128 state
 # (4 GiB), measured by two rocprofv3 --pmc runs of `bench.py --workload circuit28 --no-cpu-baseline
-# --copy-calibration-gib 1` (mean over the run's 102 complex128 passes; FETCH_SIZE reads 524315.2 KiB
-# for the 1 GiB copy, WRITE_SIZE 1048576 KiB): 1.0031x the pass's algorithmic bytes, the excess being the
+# --copy-calibration-gib 1` (mean over the run's 66 complex128 passes; FETCH_SIZE reads 524316.4 KiB
+# for the 1 GiB copy, WRITE_SIZE 1048576 KiB): 1.0034x the pass's algorithmic bytes, the excess being the
 # last prefetch of each workgroup, which re-reads a tile. Commands and figures:
 # profiles/k_tile_run_circuit28_depth20.txt.
-TILE_RUN_PMC_28Q = {"fetch_kib": 2110371.9, "fetch_scale": 1048576.0 / 524315.2,
-                    "write_kib": 4194310.4, "write_scale": 1.0}
+TILE_RUN_PMC_28Q = {"fetch_kib": 2111689.4, "fetch_scale": 1048576.0 / 524316.4,
+                    "write_kib": 4194309.6, "write_scale": 1.0}
 
 
 def pmc_bytes(p) -> int:
@@ -518,7 +518,7 @@ def bench_qft16(args):
     out = _line("16-qubit QFT circuits/s (graph run incl. state upload and read-back)", 1.0 / dt, "circuits/s", reps,
                 warm, dt * 1e3, "c128", cfg, max_abs_err_vs_ifft=err, max_abs_err_probabilities=perr,
                 ms_first_run_walking_graph=walk_ms, fused_c128=fused128,
-                roofline={"bound": "launch", "kernel": "k_diag_chain<double> (controlled phases, 120 of the 144 gates, per gate)",
+                roofline={"bound": "launch", "kernel": "k_tile_thin<double> (controlled phases, 120 of the 144 gates, held and flushed; per gate)",
                           "achieved": diag_gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": diag_gbs / HBM_PEAK_GBS,
                           "traffic": None, "bytes_per_launch": diag_bytes, "avg_launch_ms": diag_ms,
                           "note": "a 1 MiB state stays in cache: each launch is bound by launch latency, not HBM"})
@@ -745,7 +745,7 @@ def bench_dense28(args):
     be.close()
     be = GpuBackend.make_state(26, [], [])
     be.kronselect_dot({q: numpy.array([[1, 1], [1, -1]]) / numpy.sqrt(2) for q in range(26)})
-    run_case(be, 26, "k8_gemm_scattered", [0, 3, 6, 9, 12, 15, 18, 25], 0, 8)
+    run_case(be, 26, "k8_scattered", [0, 3, 6, 9, 12, 15, 18, 25], 0, 8)
     be.close()
     tiles = [c for k, c in cases.items() if k.startswith(("k4", "k5", "k6")) and c["controls"] == 0]
     value = sum(c["algorithmic_gbs"] for c in tiles) / len(tiles)
