@@ -71,7 +71,8 @@ int qipgpu_init_feeds(qipgpu_state *s, int32_t n_groups, const int32_t *group_le
 /* Copies of amplitude windows [start, end) in the state's own dtype:
  *   get:  get_state / get_relative_range   (qip/backend.py:106-107,168-169)
  *   set:  overwrite_relative_range          (qip/backend.py:171-172)
- *   add:  addto_relative_range              (qip/backend.py:174-175) */
+ *   add:  addto_relative_range              (qip/backend.py:174-175)
+ * set and add read `host` before they return; the state is written in the order of its queue. */
 int qipgpu_get_range(qipgpu_state *s, int64_t start, int64_t end, void *host);
 int qipgpu_set_range(qipgpu_state *s, int64_t start, int64_t end, const void *host);
 int qipgpu_add_range(qipgpu_state *s, int64_t start, int64_t end, const void *host);
@@ -81,8 +82,8 @@ int qipgpu_add_range(qipgpu_state *s, int64_t start, int64_t end, const void *ho
  * `controls` qubit being 1 (the C_MAT structure diag(I, M), kronprod.pyx:215-225). The engine
  * finds further control qubits and diagonal structure inside `mat` itself, so a caller may pass
  * a whole controlled operator as one dense matrix. k <= QIPGPU_MAX_DENSE. Up to 3 targets are
- * applied from registers, 4..6 through LDS tiles on FP64 MFMA, 7..12 as an FP64 GEMM out of place
- * (a temporary of 2^(n - controls) amplitudes). */
+ * applied from registers, 4..6 on FP64 MFMA in place, 7 and 8 the same with tiles in LDS on states of
+ * enough tiles, other 7..12 as an FP64 GEMM out of place (a temporary of 2^(n - controls) amplitudes). */
 int qipgpu_apply_matrix(qipgpu_state *s, int32_t k, const int32_t *targets, const double *mat,
                         int32_t n_ctrl, const int32_t *controls);
 
@@ -119,8 +120,10 @@ int qipgpu_apply_product(qipgpu_state *s, int32_t k, const int32_t *targets, con
  * A gate that rounds nothing (X, a swap, a factor -1, under any controls) may join a run before gates
  * on other bits, which changes no value. What is held is applied, in order, by any other call on the
  * state (qipgpu_synchronize, qipgpu_fused_flush, any read). A run goes gate by gate where separate
- * sweeps would move fewer bytes. The state is bit for bit what one launch per gate gives, but for the
- * sign of zeros. */
+ * sweeps would move fewer bytes. As long as every amplitude is finite, the state is bit for bit what one
+ * launch per gate gives, but for the sign of zeros. (In a run X and swaps move amplitudes, a factor -1 turns
+ * signs, a factor 1 is left out and a real matrix forms no products with its zero imaginary parts; a gate's own
+ * sweep forms the products with zeros, which an infinity or a NaN turns into NaN.) */
 int qipgpu_apply_diagonal(qipgpu_state *s, int32_t k, const int32_t *targets, const double *diag,
                           int32_t n_ctrl, const int32_t *controls);
 

@@ -1959,7 +1959,7 @@ static int marginals_dev(qipgpu_state *s, int32_t k, const int32_t *indices, Ord
         for (int j = 0; j < k; ++j) a.opos[j] = (uint8_t)sorted[j];
     }
     fill_poslist(a.mpl, mpos);
-    // every outcome of up to 2^26: one pass over the state (its partials stay within 1 GiB)
+    // every outcome of up to 2^26: one pass over the state (its partials stay within 256 MiB)
     if (n >= kMargChunkBits && k >= 1 && k <= 26 && m_lo == 0 && m_count == (1ull << k))
         return marginals_pass(s, mpos, a.opos, extra, area);
     const bool serial = a.terms <= 64;

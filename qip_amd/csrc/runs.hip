@@ -11,7 +11,9 @@
 // Results. Each gate is applied by itself, with the expression its own sweep uses: a pair by k_dense's
 // FP64 sums from zero, a factor by k_diag's product, each rounded to the state's precision. Gates
 // change places only where that changes no amplitude's value (plan_pass). So the state is what one
-// launch per gate gives, bit for bit but for the sign of a zero.
+// launch per gate gives, bit for bit but for the sign of a zero, as long as every amplitude is finite: X, swaps
+// and factors of 1 and -1 form no products here, and a real matrix none with its zero imaginary parts, where a
+// gate's own sweep multiplies by those zeros (an infinity or a NaN would make a NaN of them).
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
